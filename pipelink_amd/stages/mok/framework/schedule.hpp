@@ -13,6 +13,10 @@
 #define MOK_SCHED_FN __device__ __forceinline__
 // wave-uniform by construction; say so, so that the value lives in a scalar register
 #define MOK_SCHED_UNIFORM(x) __builtin_amdgcn_readfirstlane(x)
+#define MOK_SCHED_COUNT(n, holds) mok_framework::count_by_wave(n, holds)
+#endif
+#ifndef MOK_SCHED_COUNT
+#define MOK_SCHED_COUNT(n, holds) mok_framework::count(n, holds)
 #endif
 
 namespace mok_framework {
@@ -21,14 +25,33 @@ constexpr int NUM_XCD = 8;       // lists
 constexpr int TILE_X = 256;      // routed rows of a tile   (the GEMM owner's published facts; the stage source
 constexpr int TILE_W = 256;      // weight rows of a tile    checks them against the owner's header)
 
+// how many of the first n numbers a condition holds for: one after the other; by a wave (all of its lanes take part and get
+// the answer), where the reads behind the condition are 64 at a time instead of a chain of LDS latencies
+template <class Holds>
+MOK_SCHED_FN int count(int n, Holds holds) {
+  int c = 0;
+  for (int i = 0; i < n; ++i) c += holds(i) ? 1 : 0;
+  return c;
+}
+#ifdef __HIP_DEVICE_COMPILE__
+template <class Holds>
+MOK_SCHED_FN int count_by_wave(int n, Holds holds) {
+  int c = 0;
+  for (int i = threadIdx.x & 63; i - (int)(threadIdx.x & 63) < n; i += 64)
+    c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i < n && holds(i)));
+  return c;
+}
+#endif
+
 // the schedule's tables in LDS: exclusive prefix sums per expert, and one word of the last workgroup
 struct Tables {
   int row_begin[MAX_EXPERTS + 1];
   int tile_begin[MAX_EXPERTS + 1];
-  uint32_t last;   // 1 in the workgroup that leaves the launch last
+  uint32_t last;   // 1 + the list `claim` is of, or 0 if every list has been handed out; in the end: 1 in the workgroup
+                   // that leaves the launch last
   uint32_t claim;  // what the list's queue answered this workgroup's last request
 
-  // exclusive prefix sums of rows and row tiles per expert (one thread; every workgroup computes its own copy)
+  // exclusive prefix sums of rows and row tiles per expert, one expert after the other
   MOK_SCHED_FN void fill(const int32_t* tokens_per_expert, int ne) {
     int rows = 0, tiles = 0;
     for (int e = 0; e < ne; ++e) {
@@ -40,6 +63,29 @@ struct Tables {
     }
     row_begin[ne] = rows;
     tile_begin[ne] = tiles;
+  }
+  // The same by the 64 lanes of one wave, an expert per lane (every workgroup computes its own copy).  `scan` is the
+  // inclusive sum over the lanes up to this one, `last_lane` lane 63's value.  fill() by one thread is a chain of `ne`
+  // memory reads, one after the other, in front of everything else a launch does: a launch of one token and 32 experts
+  // took 54.4 us with it and takes 53.2 us.
+  template <class Scan, class Last>
+  MOK_SCHED_FN void fill_by_wave(const int32_t* tokens_per_expert, int ne, int lane, Scan scan, Last last_lane) {
+    int rows = 0, tiles = 0;
+    for (int e0 = 0; e0 < ne; e0 += 64) {
+      const int e = e0 + lane;
+      const int c = e < ne ? tokens_per_expert[e] : 0, t = (c + TILE_X - 1) / TILE_X;
+      const int c_sum = scan(c), t_sum = scan(t);
+      if (e < ne) {
+        row_begin[e] = rows + c_sum - c;
+        tile_begin[e] = tiles + t_sum - t;
+      }
+      rows += last_lane(c_sum);
+      tiles += last_lane(t_sum);
+    }
+    if (lane == 0) {
+      row_begin[ne] = rows;
+      tile_begin[ne] = tiles;
+    }
   }
 };
 
@@ -66,9 +112,10 @@ struct Schedule {
     const int idx = gate_up ? share(q, gu) + i : share(q, d) + i - gate_up_items;  // in the sequence of its GEMM's tiles
     const int cols = gate_up ? gate_up_cols : down_cols;
     // last e with tile_begin[e] * cols <= idx: it has row tiles, since tile_begin[e + 1] * cols > idx
+    // (a workgroup's next item is usually the same expert's)
     int lo = cursor;
-    if (tab.tile_begin[lo] * cols > idx) lo = 0;  // the other GEMM: from the start
-    while (lo + 1 < g.num_experts && tab.tile_begin[lo + 1] * cols <= idx) ++lo;
+    if (tab.tile_begin[lo] * cols > idx || (lo + 1 < g.num_experts && tab.tile_begin[lo + 1] * cols <= idx))
+      lo = MOK_SCHED_COUNT(g.num_experts, [&](int e) { return tab.tile_begin[e] * cols <= idx; }) - 1;
     cursor = lo;
     const int e = MOK_SCHED_UNIFORM(lo);
     const int t0 = tab.tile_begin[e], t1 = tab.tile_begin[e + 1];
