@@ -117,6 +117,9 @@ int plk_mok_forward_static(plk_mok_session* s, const plk_mok_problem* p, void* s
  * (padding bytes zeroed). */
 int plk_mxfp8_quantize(uint64_t src, int src_is_bf16, int64_t rows, int32_t k, uint64_t dst_q, int32_t ld_q,
                        uint64_t dst_sc, int32_t ld_sc, void* stream);
+/* The same, and the code rows' pad bytes zeroed. */
+int plk_mxfp8_quantize_zero_pad(uint64_t src, int src_is_bf16, int64_t rows, int32_t k, uint64_t dst_q, int32_t ld_q,
+                                uint64_t dst_sc, int32_t ld_sc, void* stream);
 
 /* Row-major e8m0 scales src [rows, ld_sc] -> slot-major dst [ceil(k/128), rows, 4] (pad bytes 0).
  * For a weight tensor [E, N, K] call it once per expert (or once with rows = E*N when the

@@ -178,10 +178,9 @@ def mxfp8_quantize_device(src: torch.Tensor, pitch: int | None = None) -> tuple[
     rows, k = src.shape
     ld = scale_pitch(k)
     pitch = k if pitch is None else pitch
-    q = torch.empty((rows, pitch), dtype=torch.uint8, device=src.device) if pitch == k else \
-        torch.zeros((rows, pitch), dtype=torch.uint8, device=src.device)
+    q = torch.empty((rows, pitch), dtype=torch.uint8, device=src.device)
     sc = torch.empty((rows, ld), dtype=torch.uint8, device=src.device)
     lib = load_library()
-    check(lib, lib.plk_mxfp8_quantize(src.data_ptr(), int(src.dtype == torch.bfloat16), rows, k, q.data_ptr(), pitch,
-                                      sc.data_ptr(), ld, c_void_p(torch.cuda.current_stream().cuda_stream)))
+    check(lib, lib.plk_mxfp8_quantize_zero_pad(src.data_ptr(), int(src.dtype == torch.bfloat16), rows, k, q.data_ptr(), pitch,
+                                               sc.data_ptr(), ld, c_void_p(torch.cuda.current_stream().cuda_stream)))
     return q, sc

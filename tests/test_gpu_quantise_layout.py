@@ -1,0 +1,48 @@
+"""The device quantiser and the weight layout conversions at the edges of their kernels' pieces, against the oracle (bit
+for bit) and numpy's transpositions."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import mxfp8
+
+pytestmark = pytest.mark.gpu
+
+
+# a row of 4 pieces and up; rows that end inside a workgroup's 1024 pieces, at its end and one behind; a piece's row more
+# than one row on; pitches that are no multiple of 8, and pads longer than a row has pieces
+@pytest.mark.parametrize("rows,k,pad", [(1, 32, 0), (3, 32, 4), (256, 32, 96), (257, 32, 60), (1025, 64, 0), (7, 2848, 20),
+                                        (64, 128, 0), (65, 128, 128), (129, 2880, 64), (2, 32768, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_quantiser_at_the_edges_of_its_pieces(rows, k, pad, dtype):
+    from pipelink_amd.host.mok import mxfp8_quantize_device, scale_pitch
+
+    g = torch.Generator().manual_seed(rows + k)
+    x = torch.randn(rows, k, generator=g) * torch.exp2(torch.randint(-130, 120, (rows, 1), generator=g).float())
+    x[0, 0], x[-1, -1], x[-1, 0] = float("nan"), -float("inf"), -0.0
+    x[rows // 2, k - 32:] = 0
+    # the values start 8 bytes (bf16) or 16 bytes (fp32) into their allocation
+    room = torch.empty(rows * k + 4, dtype=dtype, device="cuda")
+    src = room[4:].view(rows, k)
+    src.copy_(x.to(dtype))
+    q, sc = mxfp8_quantize_device(src, pitch=k + pad)
+    oq, osc = mxfp8.mx_quantize(x.to(dtype).float().numpy())
+    assert q.shape == (rows, k + pad) and sc.shape == (rows, scale_pitch(k))
+    assert np.array_equal(q[:, :k].cpu().numpy(), oq) and not q[:, k:].any()
+    assert np.array_equal(sc[:, :k // 32].cpu().numpy(), osc[:, :k // 32]) and not sc[:, k // 32:].any()
+
+
+def test_quantiser_of_the_plain_entry_leaves_the_pad_alone():
+    from pipelink_amd.host.backend import check, load_library
+
+    lib = load_library()
+    x = torch.randn(9, 96, device="cuda")
+    q = torch.full((9, 128), 0xA5, dtype=torch.uint8, device="cuda")
+    sc = torch.empty((9, 3), dtype=torch.uint8, device="cuda")   # a scale pitch without padding
+    check(lib, lib.plk_mxfp8_quantize(x.data_ptr(), 0, 9, 96, q.data_ptr(), 128, sc.data_ptr(), 3,
+                                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    oq, osc = mxfp8.mx_quantize(x.cpu().numpy())
+    assert np.array_equal(q[:, :96].cpu().numpy(), oq) and bool((q[:, 96:] == 0xA5).all())
+    assert np.array_equal(sc.cpu().numpy(), osc[:, :3])
