@@ -130,6 +130,12 @@ int plk_mxfp8_scales_to_slot_major(uint64_t src, int64_t rows, int32_t k, int32_
  * 16-byte aligned addresses).  For a weight tensor [E, N, K] call it once per expert with rows = N. */
 int plk_mxfp8_codes_to_k64_tiled(uint64_t src, int64_t rows, int32_t k, int64_t ld_q, uint64_t dst, void* stream);
 
+/* Both conversions for a whole weight tensor [experts, rows, ld] in one launch each. */
+int plk_mxfp8_scales_to_slot_major_experts(uint64_t src, int32_t experts, int64_t rows, int32_t k, int32_t ld_sc, uint64_t dst,
+                                           void* stream);
+int plk_mxfp8_codes_to_k64_tiled_experts(uint64_t src, int32_t experts, int64_t rows, int32_t k, int64_t ld_q, uint64_t dst,
+                                         void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -81,6 +81,8 @@ SIGNATURES = {
     "plk_mok_session_launches": (c_int, [c_void_p, c_int]),
     "plk_mxfp8_scales_to_slot_major": (c_int, [c_uint64, c_int64, c_int32, c_int32, c_uint64, c_void_p]),
     "plk_mxfp8_codes_to_k64_tiled": (c_int, [c_uint64, c_int64, c_int32, c_int64, c_uint64, c_void_p]),
+    "plk_mxfp8_scales_to_slot_major_experts": (c_int, [c_uint64, c_int32, c_int64, c_int32, c_int32, c_uint64, c_void_p]),
+    "plk_mxfp8_codes_to_k64_tiled_experts": (c_int, [c_uint64, c_int32, c_int64, c_int32, c_int64, c_uint64, c_void_p]),
     "plk_mxfp8_quantize": (c_int, [c_uint64, c_int, c_int64, c_int32, c_uint64, c_int32, c_uint64, c_int32, c_void_p]),
     "plk_mxfp8_quantize_zero_pad": (c_int, [c_uint64, c_int, c_int64, c_int32, c_uint64, c_int32, c_uint64, c_int32, c_void_p]),
 }

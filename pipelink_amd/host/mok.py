@@ -36,8 +36,8 @@ def weight_scales_to_slot_major(sc: torch.Tensor, k: int) -> torch.Tensor:
     out = torch.empty((e, scale_slots(k), n, 4), dtype=torch.uint8, device=sc.device)
     lib = load_library()
     stream = c_void_p(torch.cuda.current_stream().cuda_stream)
-    for i in range(e):
-        check(lib, lib.plk_mxfp8_scales_to_slot_major(sc[i].data_ptr(), n, k, ld, out[i].data_ptr(), stream))
+    if e:
+        check(lib, lib.plk_mxfp8_scales_to_slot_major_experts(sc.data_ptr(), e, n, k, ld, out.data_ptr(), stream))
     return out
 
 
@@ -51,8 +51,8 @@ def weight_codes_to_k64_tiled(q: torch.Tensor, k: int) -> torch.Tensor:
     out = torch.empty((e, k // 64, n, 64), dtype=torch.uint8, device=q.device)
     lib = load_library()
     stream = c_void_p(torch.cuda.current_stream().cuda_stream)
-    for i in range(e):
-        check(lib, lib.plk_mxfp8_codes_to_k64_tiled(q[i].data_ptr(), n, k, ld, out[i].data_ptr(), stream))
+    if e:
+        check(lib, lib.plk_mxfp8_codes_to_k64_tiled_experts(q.data_ptr(), e, n, k, ld, out.data_ptr(), stream))
     return out
 
 

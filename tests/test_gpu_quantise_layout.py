@@ -34,6 +34,29 @@ def test_quantiser_at_the_edges_of_its_pieces(rows, k, pad, dtype):
     assert np.array_equal(sc[:, :k // 32].cpu().numpy(), osc[:, :k // 32]) and not sc[:, k // 32:].any()
 
 
+# one row to one behind a workgroup's; one column, an odd number, a pair of them and one more; a scale row that is no
+# multiple of four bytes, one that holds one dword more than it needs, more slots than a workgroup's
+@pytest.mark.parametrize("e,n,k,ld,ld_sc", [(1, 1, 64, 64, 2), (3, 127, 192, 208, 6), (2, 129, 128, 128, 4), (5, 64, 320, 336, 11),
+                                            (2, 65, 2880, 2880, 96), (33, 31, 4224, 4224, 136)])
+def test_weight_layouts_at_the_edges_of_their_tiles(e, n, k, ld, ld_sc):
+    from pipelink_amd.host.mok import weight_codes_to_k64_tiled, weight_scales_to_slot_major
+
+    g = torch.Generator().manual_seed(n)
+    q = torch.randint(0, 256, (e, n, ld), dtype=torch.uint8, generator=g)
+    sc = torch.randint(0, 256, (e, n, ld_sc), dtype=torch.uint8, generator=g)
+    tiled = weight_codes_to_k64_tiled(q.cuda(), k).cpu().numpy()
+    assert np.array_equal(tiled, q.numpy()[:, :, :k].reshape(e, n, k // 64, 64).transpose(0, 2, 1, 3))
+    slots = (k + 127) // 128
+    want = np.zeros((e, n, 4 * slots), np.uint8)
+    want[:, :, :k // 32] = sc.numpy()[:, :, :k // 32]
+    want = want.reshape(e, n, slots, 4).transpose(0, 2, 1, 3)
+    assert np.array_equal(weight_scales_to_slot_major(sc.cuda(), k).cpu().numpy(), want)
+    # scale bytes that do not start on a dword
+    room = torch.empty(e * n * ld_sc + 1, dtype=torch.uint8, device="cuda")
+    room[1:].copy_(sc.flatten())
+    assert np.array_equal(weight_scales_to_slot_major(room[1:].view(e, n, ld_sc), k).cpu().numpy(), want)
+
+
 def test_quantiser_of_the_plain_entry_leaves_the_pad_alone():
     from pipelink_amd.host.backend import check, load_library
 
