@@ -10,6 +10,10 @@ from ..stages.attention.params import params_blobs
 
 HEAD_DIM = 128
 Q_TILE = 128
+# A grid of at most this many tiles of 128 queries is launched as twice as many of 64, each with a wave per half of the
+# keys: us whole / half at 256 compute units: 256 tiles 25.7 / 22.3, 384 tiles 41.4 / 35.4, 480 tiles 54.3 / 54.2, 512 tiles
+# 57.6 / 61.4 and 24.8 / 28.8
+HALF_TILES_UP_TO = 384
 
 
 def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, v_bits: np.ndarray, *, scale: float | None = None,
@@ -31,6 +35,7 @@ def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, 
         raise ValueError("operands are uint16 bf16 bit patterns")
     if s * d * 2 >= 1 << 31:
         raise ValueError("one head of K or V must stay below 2 GiB")
+    tiles = b * hq * (s // Q_TILE)
     buffers = {"q": q_bits, "k": k_bits, "v": v_bits, "o": ((b, s, hq * d), np.uint16)}
     return open_hostless(link_json, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
-                         grid=(b * hq * (s // Q_TILE),), backend=backend, image=image)
+                         grid=(tiles if tiles > HALF_TILES_UP_TO else 2 * tiles,), backend=backend, image=image)

@@ -1,4 +1,5 @@
-// Package fa.core: flash-attention forward for one tile of 128 queries of one head.
+// Package fa.core: flash-attention forward for one tile of 128 queries of one head, or, in a launch of twice as many
+// workgroups, of 64 (half tiles).
 //
 // Orientation.  Scores are computed transposed, S^T = K . Q^T (keys are the MFMA rows, queries the
 // columns), so that a lane holds ONE query (column lane % 32) and 16 of the block's 32 keys: row maxima
@@ -14,6 +15,13 @@
 // (8 bytes) and lane j receives element j % 4 of the data of lanes j / 4, j / 4 + 4, j / 4 + 8, j / 4 + 12
 // (measured with a probe); so lane i points at key kbase + i / 4, d = dbase + 4 (i % 4), and lane j gets keys
 // kbase .. kbase + 3 at d = dbase + j.
+//
+// A tile is a chain of key blocks; a grid that leaves most SIMDs with one wave or none takes as long as the longest chain,
+// with nothing beside it.  With half tiles waves 0 and 1 have 32 queries each and the first 32 keys of every block, waves 2
+// and 3 the same queries and the other 32 keys: twice the workgroups, each block half as long for a wave.  The two halves
+// of a query's sum meet through LDS at the end.  us, whole / half tiles: B 1, 32 heads, S 1152, window 700 (288 tiles) 26.3 /
+// 21.2; S 512 causal (128 tiles) 14.6 / 11.8; 8 heads, S 4096 (256 tiles) 81.8 / 62.4; 32 heads, S 2048 (512 tiles) 57.6 /
+// 61.4; the stated B 4, S 4096 (4096 tiles) 583 / 695: with two waves on every SIMD a key block costs its loads twice.
 //
 // Two LDS buffers per operand: block i + 1 is in flight while block i is multiplied; one barrier per block.
 #include <pipelink/stage.hpp>
@@ -88,13 +96,17 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
   const pipelink_host_view view{params, nullptr};
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
-  const int q_tiles = p.seq / FA_Q_TILE;
+  // the host launches a workgroup per tile of 128 queries, or two: which one, the grid says
+  const int heads = p.batch * p.q_heads;
+  const bool split = (int64_t)gridDim.x > (int64_t)heads * (p.seq / FA_Q_TILE);
+  const int tile_queries = split ? FA_Q_TILE / 2 : FA_Q_TILE;
+  const int q_tiles = p.seq / tile_queries;
   // Causal tiles cost in proportion to their position: the latest (longest) tiles of every head are
   // dispatched first, so that the grid does not end on a few long ones.  bh = batch * q_heads + head.
-  const int heads = p.batch * p.q_heads;
   const int tile = q_tiles - 1 - (int)(blockIdx.x / heads), bh = blockIdx.x % heads;
   const int b = bh / p.q_heads, h = bh % p.q_heads, kvh = h / (p.q_heads / p.kv_heads);
-  const int q0 = tile * FA_Q_TILE, qw = q0 + 32 * wave;               // the wave's first query
+  const int q0 = tile * tile_queries, qw = q0 + 32 * (split ? wave & 1 : wave);  // the wave's first query
+  const int key0 = split ? 32 * (wave >> 1) : 0;                                 // its first key of every block
   const uint32_t head_bytes = (uint32_t)p.seq * FA_D * 2;
   const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(p.k) + ((int64_t)b * p.kv_heads + kvh) * p.seq * FA_D, 0, (int)head_bytes, 0x00020000);
@@ -118,8 +130,8 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
   bool seen = false;  // this lane's query has met a key it may see (decided on unscaled scores: the scale is the caller's)
 
   // the mask package says which stretch of keys the tile's queries may see at all: blocks [first_block, blocks)
-  const int keys = pipelink_call_mask_key_count(&view, q0, q0 + FA_Q_TILE - 1);
-  const int first_block = pipelink_call_mask_key_begin(&view, q0, q0 + FA_Q_TILE - 1) / FA_K_BLOCK;
+  const int keys = pipelink_call_mask_key_count(&view, q0, q0 + tile_queries - 1);
+  const int first_block = pipelink_call_mask_key_begin(&view, q0, q0 + tile_queries - 1) / FA_K_BLOCK;
   const int blocks = (keys + FA_K_BLOCK - 1) / FA_K_BLOCK;
   const int wave_keys = pipelink_call_mask_key_count(&view, qw, qw + 31), wave_begin = pipelink_call_mask_key_begin(&view, qw, qw + 31);
   // Schedule.  Two LDS buffers per operand: block i + 1 is in flight while block i is multiplied; one barrier per
@@ -134,7 +146,7 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
 #pragma unroll
   for (int pb = 0; pb < 2; ++pb)
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) k_at[pb][kk] = buf + pb * BUF_BYTES + l32 * (FA_D * 2) + 16 * k_place(l32, 2 * kk + half);
+    for (int kk = 0; kk < 8; ++kk) k_at[pb][kk] = buf + pb * BUF_BYTES + (key0 + l32) * (FA_D * 2) + 16 * k_place(l32, 2 * kk + half);
   const int v_key = 4 * half + (li >> 2);  // the key (within a group of 16) this lane points at for the transposing read
   const unsigned char* v_at[2][4];
 #pragma unroll
@@ -142,7 +154,7 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
       const int d = 32 * db + dgroup + 4 * (li & 3);
-      v_at[pb][db] = buf + pb * BUF_BYTES + K_BYTES + v_key * (FA_D * 2) + 16 * v_place(v_key, d >> 3) + 2 * (d & 4);
+      v_at[pb][db] = buf + pb * BUF_BYTES + K_BYTES + (key0 + v_key) * (FA_D * 2) + 16 * v_place(v_key, d >> 3) + 2 * (d & 4);
     }
   // the 8 pieces (4 blocks of d x two halves of 8 keys) of the group of 16 keys that starts at key `first`
   auto read_v_group = [&](int pb, int first, v4s (&piece)[8]) {
@@ -155,29 +167,30 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
   };
   issue_block<false>(kres, (uint32_t)first_block * FA_K_BLOCK * FA_D * 2, buf, wave, lane);
   issue_block<true>(vres, (uint32_t)first_block * FA_K_BLOCK * FA_D * 2, buf + K_BYTES, wave, lane);
-  // one block of 64 keys; PB = (i - first_block) % 2 (the buffer pair) is a compile-time constant so that the address tables are registers
-  auto block = [&](int i, auto pair) {
-    constexpr int PB = decltype(pair)::value;
+  // one block of 64 keys, NT tiles of 32 of them this wave's; PB = (i - first_block) % 2 (the buffer pair) is a compile-time
+  // constant so that the address tables are registers
+  auto block = [&](int i, auto pair, auto tiles) {
+    constexpr int PB = decltype(pair)::value, NT = decltype(tiles)::value;
     __syncthreads();  // blocks i of K and V have landed (the barrier drains every wave's loads); buffers of block i - 1 are free
     if (i + 1 < blocks) {
       issue_block<false>(kres, (uint32_t)(i + 1) * FA_K_BLOCK * FA_D * 2, buf + (1 - PB) * BUF_BYTES, wave, lane);
       issue_block<true>(vres, (uint32_t)(i + 1) * FA_K_BLOCK * FA_D * 2, buf + (1 - PB) * BUF_BYTES + K_BYTES, wave, lane);
     }
-    const int k0 = i * FA_K_BLOCK;
-    if (k0 >= wave_keys || k0 + FA_K_BLOCK <= wave_begin) return;  // no query of this wave sees a key of this block: only the loads and the barrier
-    // ---- S^T = K . Q^T : two 32-key tiles -----------------------------------------------------------
-    v16f s[2];
+    const int k0 = i * FA_K_BLOCK + key0;
+    if (k0 >= wave_keys || k0 + 32 * NT <= wave_begin) return;  // no query of this wave sees a key of this block: only the loads and the barrier
+    // ---- S^T = K . Q^T : NT 32-key tiles -----------------------------------------------------------
+    v16f s[NT];
     v4s piece[2][8];
     {
-      v4i kf[2][8];
+      v4i kf[NT][8];
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk) kf[t][kk] = *reinterpret_cast<const v4i*>(k_at[PB][kk] + t * 32 * (FA_D * 2));
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_setprio(2);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int t = 0; t < NT; ++t) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
 #pragma unroll
@@ -189,10 +202,10 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
     }
     // ---- mask, online softmax (in units of log2: exp2(x * scale_log2e - max)) -------------------------------
     const int query = qw + l32;
-    const bool all = pipelink_call_mask_all_visible(&view, qw, qw + 31, k0, k0 + FA_K_BLOCK - 1);
+    const bool all = pipelink_call_mask_all_visible(&view, qw, qw + 31, k0, k0 + 32 * NT - 1);
     if (!all) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = k0 + 32 * t + 8 * (r / 4) + 4 * half + r % 4;
@@ -201,7 +214,7 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
     }
     float block_max = MASKED;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) block_max = fmaxf(block_max, s[t][r]);
     block_max = max_with_other_half(block_max);
@@ -221,7 +234,7 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
     const float reference = seen ? new_max : -MASKED;
     float block_sum = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], p.scale_log2e, -reference));
@@ -236,12 +249,12 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
     }
-    // ---- O^T += V^T . P^T : four groups of 16 keys, four 32-row blocks of d ----------------------------
+    // ---- O^T += V^T . P^T : 2 NT groups of 16 keys, four 32-row blocks of d ----------------------------
     __builtin_amdgcn_s_setprio(2);
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi) {
+    for (int gi = 0; gi < 2 * NT; ++gi) {
       const int t = gi >> 1, g = gi & 1;
-      if (gi + 1 < 4) read_v_group(PB, 16 * (gi + 1), piece[(gi + 1) & 1]);
+      if (gi + 1 < 2 * NT) read_v_group(PB, 16 * (gi + 1), piece[(gi + 1) & 1]);
       __builtin_amdgcn_sched_barrier(0);
       v8f pf;
 #pragma unroll
@@ -257,9 +270,47 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
     }
     __builtin_amdgcn_s_setprio(0);
   };
-  for (int i = first_block; i < blocks; i += 2) {
-    block(i, std::integral_constant<int, 0>{});
-    if (i + 1 < blocks) block(i + 1, std::integral_constant<int, 1>{});
+  auto stream = [&](auto tiles) {
+    for (int i = first_block; i < blocks; i += 2) {
+      block(i, std::integral_constant<int, 0>{}, tiles);
+      if (i + 1 < blocks) block(i + 1, std::integral_constant<int, 1>{}, tiles);
+    }
+  };
+  if (split) {
+    stream(std::integral_constant<int, 1>{});
+    // the other half of the keys: waves 2 and 3 hand what they have to waves 0 and 1.  A half that has seen no key for a
+    // query has no maximum, and nothing to add.
+    if (!seen) row_max = MASKED;
+    unsigned char* const part = buf + (wave & 1) * (17 * 1024);  // 16 x 1 KB of O^T, then the maxima and the sums
+    __syncthreads();  // nobody reads keys or values any more
+    if (wave >= 2) {
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const v4f f = {o[db][4 * q4], o[db][4 * q4 + 1], o[db][4 * q4 + 2], o[db][4 * q4 + 3]};
+          *reinterpret_cast<v4f*>(part + (4 * db + q4) * 1024 + lane * 16) = f;
+        }
+      *reinterpret_cast<float*>(part + 16 * 1024 + lane * 8) = row_max;
+      *reinterpret_cast<float*>(part + 16 * 1024 + lane * 8 + 4) = row_sum;
+    }
+    __syncthreads();
+    if (wave >= 2) return;
+    const float other_max = *reinterpret_cast<const float*>(part + 16 * 1024 + lane * 8);
+    const float other_sum = *reinterpret_cast<const float*>(part + 16 * 1024 + lane * 8 + 4);
+    const float top = fmaxf(row_max, other_max);
+    const float mine = __builtin_amdgcn_exp2f(row_max - top), others = __builtin_amdgcn_exp2f(other_max - top);
+    row_sum = row_sum * mine + other_sum * others;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        const v4f f = *reinterpret_cast<const v4f*>(part + (4 * db + q4) * 1024 + lane * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[db][4 * q4 + e] = o[db][4 * q4 + e] * mine + f[e] * others;
+      }
+  } else {
+    stream(std::integral_constant<int, 2>{});
   }
   // ---- O[b][query][h][d] = O^T / row_sum, bf16 ------------------------------------------------------------
   const float inv = row_sum > 0.0f ? __builtin_amdgcn_rcpf(row_sum) : 0.0f;
