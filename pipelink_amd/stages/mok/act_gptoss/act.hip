@@ -105,7 +105,39 @@ __device__ __forceinline__ void forward(const MokActResidue& p, const MokActTask
     if (half == 0) stage[STAGE_SCALE_OFF + trow * 4 + (tcol >> 5)] = (uint8_t)e;
   };
   // ---- activation + requant into an LDS tile [256 rows][128 codes] + [256 rows][4 scales] ----
-  const int placement = tile_placement(t.row_end - t.row_begin, p.cols - t.col_begin);
+  const int placement = tile_placement(t.row_end - t.row_begin, p.cols - t.col_begin, t.flags);
+  // The tile is counted when all of it is in memory: every wave waits until its own stores have been written through (a
+  // store leaves the wave's vector-memory count when it is acknowledged; the barrier's workgroup-scope fence does not wait
+  // for that), then the workgroup meets, then one thread counts the tile.  The row tile's counter reaches the number of
+  // gate/up column tiles when all of its `hidden` can be read by any workgroup
+  // (campaigns/mok/port/framework/interp_fwd.cu:174-213: the reference's act -> down dependency).
+  auto count_tile = [&]() {
+    if (t.counter_idx >= 0 && counters.base) __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+    __syncthreads();  // also: the staging tile shares LDS with the GEMM ring of the next tile
+    if (t.counter_idx >= 0 && counters.base && tid == 0)
+      __hip_atomic_fetch_add(counters.base + t.counter_idx, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  const __amdgpu_buffer_rsrc_t out_q =
+      __builtin_amdgcn_make_buffer_rsrc(p.hidden_q, 0, (int)((uint32_t)p.rows * (uint32_t)p.ld_q), 0x00020000);
+  if constexpr (SMALL) {
+    if (__builtin_expect(placement == TILE_NARROW, 0)) {  // one block of 32 columns of at most 32 rows, in wave 0
+      const int col = t.col_begin;
+      if (wave == 0) {
+        requantise(from_acc(acc.v[0][0]), from_acc(acc.v[2][0]), lane & 31, 0);
+        const int trow = lane >> 1, row = t.row_begin + trow, chunk = lane & 1;
+        if (row < t.row_end && col < p.cols) {
+          const v4i v = *reinterpret_cast<const v4i*>(stage + trow * STAGE_PITCH + chunk * 16);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), out_q,
+                                                 (int)((uint32_t)row * (uint32_t)p.ld_q + (uint32_t)(col + chunk * 16)), 0, 16);
+          if (chunk == 0)
+            __hip_atomic_store(p.hidden_sc + (int64_t)row * p.ld_sc + (col >> 5), stage[STAGE_SCALE_OFF + trow * 4],
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      count_tile();
+      return;
+    }
+  }
   if constexpr (!SMALL) {
     (void)placement;
     // (a wave whose rows or columns all lie past the end computes on an accumulator the GEMM owner
@@ -132,8 +164,6 @@ __device__ __forceinline__ void forward(const MokActResidue& p, const MokActTask
   // another XCD -- a down tile of the same launch, once the row tile's counter says so -- reads them.
   const int chunk = lane & 7;
   const bool col_ok = t.col_begin + chunk * 16 < p.cols;  // column extents are multiples of 32
-  const __amdgpu_buffer_rsrc_t out_q =
-      __builtin_amdgcn_make_buffer_rsrc(p.hidden_q, 0, (int)((uint32_t)p.rows * (uint32_t)p.ld_q), 0x00020000);
 #pragma unroll
   for (int it = 0; it < TILE_X / (THREADS / 64) / 8; ++it) {
     const int trow = wave * (TILE_X / (THREADS / 64)) + it * 8 + (lane >> 3);
@@ -159,15 +189,7 @@ __device__ __forceinline__ void forward(const MokActResidue& p, const MokActTask
       }
     }
   }
-  // The tile is counted when all of it is in memory: every wave waits until its own stores above have been written
-  // through (a store leaves the wave's vector-memory count when it is acknowledged; the barrier's workgroup-scope
-  // fence does not wait for that), then the workgroup meets, then one thread counts the tile.  The row tile's counter
-  // reaches the number of gate/up column tiles when all of its `hidden` can be read by any workgroup
-  // (campaigns/mok/port/framework/interp_fwd.cu:174-213: the reference's act -> down dependency).
-  if (t.counter_idx >= 0 && counters.base) __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
-  __syncthreads();  // also: the staging tile shares LDS with the GEMM ring of the next tile
-  if (t.counter_idx >= 0 && counters.base && tid == 0)
-    __hip_atomic_fetch_add(counters.base + t.counter_idx, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  count_tile();
 }
 
 }  // namespace mok_act_owner

@@ -12,7 +12,7 @@
 // of the same rows; within each, expert by expert, column tile by column tile, row tiles innermost, so that
 // workgroups that run at the same time share a weight tile and one XCD's L2 sees a contiguous run of experts.  A
 // workgroup's first two tiles are fixed by its id; after that the list's queue (a word of the workspace) hands the
-// tiles out in list order, one atomic per tile, and a workgroup whose list is handed out asks the next list's queue
+// tiles out in list order, one atomic per tile, and a workgroup whose list is handed out asks another list that has tiles left
 // (the reference asks the cluster launch control for its next tile, interp_fwd.cu:137-160).  Tiles differ in cost
 // (full ones, and those of few rows or few columns, which have a placement of their own), and turns of equal length
 // leave the workgroups that drew the full ones tiles behind the others.  A down tile reads rows of `hidden` that up
@@ -105,7 +105,7 @@ __device__ __attribute__((noinline)) SmallTileResult small_tile(const void* para
   const bool early = next.op != 0 && pipelink_call_gemm_ready(&view, &next, &counters);
   if (early) pipelink_call_gemm_prefetch(&view, &next, &carry);
   if (task.op == MOK_GEMM_FWD_ROUTED_GATE_UP) {
-    const MokActTask act{MOK_ACT_FWD_ROUTED, task.row_begin, task.row_end, task.col_begin, task.task_idx, task.counter_idx, 0u};
+    const MokActTask act{MOK_ACT_FWD_ROUTED, task.row_begin, task.row_end, task.col_begin, task.task_idx, task.counter_idx, task.flags};
     pipelink_call_act_fwd_small(&view, &act, &counters, &phase, &acc);
   } else {
     pipelink_call_gemm_store_small(&view, &task, &acc);
@@ -129,11 +129,12 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
   // exclusive prefix sums of rows and row tiles per expert (every workgroup computes its own copy)
   if (threadIdx.x < 64)
     tab.fill_by_wave(g.tokens_per_expert, ne, threadIdx.x, [](int v) { return wave_scan(v); },
-                     [](int v) { return __builtin_amdgcn_readlane(v, 63); });
+                     [](int v) { return __builtin_amdgcn_readlane(v, 63); }, [](bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; });
   __syncthreads();
 
-  const Schedule sched{g, tab, tab.tile_begin[ne], g.op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : g.num_col_tiles_gate_up,
-                       g.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : g.num_col_tiles_down};
+  Schedule sched{g, tab, tab.tile_begin[ne], g.op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : g.num_col_tiles_gate_up,
+                 g.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : g.num_col_tiles_down};
+  if (__builtin_amdgcn_readfirstlane((int)tab.last)) sched.cut();
   const MokCounters counters{g.op == MOK_FWD_BOTH ? reinterpret_cast<int32_t*>(g.workspace + MOK_WS_COUNTERS) : nullptr,
                              g.workspace + MOK_WS_STATUS};
   uint32_t phase = 0;
@@ -147,25 +148,30 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
     // the first tile has no mainloop in front of it to look ahead from
     pipelink_call_gemm_stage(&view, &task, &counters);
     __syncthreads();  // waits for the staged loads, then the barrier
-    if (!pipelink_call_gemm_ready(&view, &task, &counters)) pipelink_call_gemm_wait(&view, &task, &counters);
+    bool early = false;  // the prefetch of the tile at the loop's head has been issued
     mok::GemmCarry carry;
-    pipelink_call_gemm_prefetch(&view, &task, &carry);
     // The tile after this one: the workgroup's second turn.  From there on tiles are handed out by the list's queue (a
     // counter in the workspace), one request per tile, made while the tile before the one before is multiplied: tiles
     // differ in cost (full ones, and those with few rows or few columns), and turns of equal length would leave the
     // workgroups that drew the full ones behind the others by several tiles' time.
-    // A workgroup whose list has been handed out goes on with the next list's queue (and so on, once round): the
+    // A workgroup whose list has been handed out goes on with another list that has tiles left (the next one first): the
     // lists are cut by number of tiles, not by cost, and whole XCDs would otherwise end a tile or two before others.
     int list = q;       // the list this workgroup asks
     bool asking = true;  // (a workgroup that has found every list handed out asks no more)
     MokGemmTask next = task;
-    if (i + turn < items) next = sched.decode(q, i + turn, cursor);
-    else next.op = 0;  // no task: mok_gemm_fwd looks ahead to nothing
     for (;;) {
+      if (!early) {
+        if (!pipelink_call_gemm_ready(&view, &task, &counters)) pipelink_call_gemm_wait(&view, &task, &counters);
+        pipelink_call_gemm_prefetch(&view, &task, &carry);
+      }
+      if (i >= 0) {  // the first tile's loads are on their way: the second turn
+        if (i + turn < items) next = sched.decode(q, i + turn, cursor);
+        else next.op = 0;  // no task: mok_gemm_fwd looks ahead to nothing
+        i = -1;
+      }
       const bool has_next = next.op != 0;
       const bool asks = has_next && asking;
       uint32_t answer = 0;
-      bool early;
       if (pipelink_call_gemm_placement(&view, &task) != mok::TILE_FULL) {
         const SmallTileResult res = small_tile(params, task, next, counters.base, counters.status, asks ? g.workspace + MOK_WS_QUEUE + list : nullptr, carry);
         carry = res.carry;
@@ -181,9 +187,13 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
         // The next tile's first loads fly while this tile's epilogue computes -- unless its rows are not complete yet:
         // then this tile is finished (and counted) first, so that nobody waits for a workgroup that waits.
         early = has_next && pipelink_call_gemm_ready(&view, &next, &counters);
-        if (early) pipelink_call_gemm_prefetch(&view, &next, &carry);
+        if (early) {
+          MokGemmTask whole = next;
+          whole.flags = 0u;  // (a launch with full tiles cuts none: the code for parts is not needed here)
+          pipelink_call_gemm_prefetch(&view, &whole, &carry);
+        }
         if (task.op == MOK_GEMM_FWD_ROUTED_GATE_UP) {
-          const MokActTask act{MOK_ACT_FWD_ROUTED, task.row_begin, task.row_end, task.col_begin, task.task_idx, task.counter_idx, 0u};
+          const MokActTask act{MOK_ACT_FWD_ROUTED, task.row_begin, task.row_end, task.col_begin, task.task_idx, task.counter_idx, task.flags};
           pipelink_call_act_fwd(&view, &act, &counters, &phase, &acc);
         } else {
           pipelink_call_gemm_store(&view, &task, &acc);
@@ -231,10 +241,6 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
         if (asking) after = sched.decode(list, k, cursor);
       }
       if (!has_next) break;
-      if (!early) {
-        pipelink_call_gemm_wait(&view, &next, &counters);
-        pipelink_call_gemm_prefetch(&view, &next, &carry);
-      }
       task = next;
       next = after;
     }

@@ -24,6 +24,8 @@ constexpr int MAX_EXPERTS = 256;
 constexpr int NUM_XCD = 8;       // lists
 constexpr int TILE_X = 256;      // routed rows of a tile   (the GEMM owner's published facts; the stage source
 constexpr int TILE_W = 256;      // weight rows of a tile    checks them against the owner's header)
+constexpr int NARROW_ROWS = 32;  // routed rows a quarter of a column tile (MOK_TASK_QUARTER) holds at most
+constexpr int CHIP = 256;        // workgroups that run at once (one per compute unit)
 
 // how many of the first n numbers a condition holds for: one after the other; by a wave (all of its lanes take part and get
 // the answer), where the reads behind the condition are 64 at a time instead of a chain of LDS latencies
@@ -47,7 +49,7 @@ MOK_SCHED_FN int count_by_wave(int n, Holds holds) {
 struct Tables {
   int row_begin[MAX_EXPERTS + 1];
   int tile_begin[MAX_EXPERTS + 1];
-  uint32_t last;   // 1 + the list `claim` is of, or 0 if every list has been handed out; in the end: 1 in the workgroup
+  uint32_t last;   // at first: no expert has more than NARROW_ROWS rows; then: 1 + the list `claim` is of, or 0 if every list has been handed out; in the end: 1 in the workgroup
                    // that leaves the launch last
   uint32_t claim;  // what the list's queue answered this workgroup's last request
 
@@ -68,9 +70,11 @@ struct Tables {
   // inclusive sum over the lanes up to this one, `last_lane` lane 63's value.  fill() by one thread is a chain of `ne`
   // memory reads, one after the other, in front of everything else a launch does: a launch of one token and 32 experts
   // took 54.4 us with it and takes 53.2 us.
-  template <class Scan, class Last>
-  MOK_SCHED_FN void fill_by_wave(const int32_t* tokens_per_expert, int ne, int lane, Scan scan, Last last_lane) {
+  // `any` is true if its argument is in any lane.  Leaves in `last` whether every expert has at most NARROW_ROWS rows.
+  template <class Scan, class Last, class Any>
+  MOK_SCHED_FN void fill_by_wave(const int32_t* tokens_per_expert, int ne, int lane, Scan scan, Last last_lane, Any any) {
     int rows = 0, tiles = 0;
+    bool more = false;
     for (int e0 = 0; e0 < ne; e0 += 64) {
       const int e = e0 + lane;
       const int c = e < ne ? tokens_per_expert[e] : 0, t = (c + TILE_X - 1) / TILE_X;
@@ -81,8 +85,10 @@ struct Tables {
       }
       rows += last_lane(c_sum);
       tiles += last_lane(t_sum);
+      more = more || any(c > NARROW_ROWS);
     }
     if (lane == 0) {
+      last = more ? 0u : 1u;
       row_begin[ne] = rows;
       tile_begin[ne] = tiles;
     }
@@ -94,22 +100,41 @@ struct Schedule {
   const Tables& tab;
   int row_tiles;  // of all experts
   int gate_up_cols, down_cols;  // column tiles of the GEMMs this launch runs (0: not run)
+  int gate_up_cut = 0, down_cut = 0;  // a column tile is 2^cut tasks (one or four)
+
+  // Narrow tiles (for launches all of whose experts have at most NARROW_ROWS rows): a GEMM's column tiles are cut in four
+  // if the quarters still run at once.  More of them than that would take a second turn, whose start costs more than the
+  // finer cut gives, us per forward: one token of 2880 x 2880, top 4 of 32, is 92 gate/up and 48 down tiles: 53.2 whole,
+  // 44.2 with the down tiles cut, 49.4 with both (368 and 192 quarters); two tokens (184 and 96): 53.4 whole, 63.2 cut;
+  // 1024 x 1536, top 2 of 16, one token: 31.1 whole, 21.6 cut.  (Halves as well, where quarters do not fit, are 39.7 for
+  // the one token, but their code beside this costs every launch of whole small tiles 1 to 2 %.)
+  // (From the numbers of both GEMMs whatever this launch runs: one launch and two give the same sums.)
+  MOK_SCHED_FN void cut() {
+    down_cut = cut_of(row_tiles * g.num_col_tiles_down);
+    // (the parts of a gate/up tile share cache lines of `hidden`, which only narrow down tiles read at device scope)
+    gate_up_cut = down_cut ? cut_of(row_tiles * g.num_col_tiles_gate_up) : 0;
+  }
+  MOK_SCHED_FN static int cut_of(int tiles) { return 4 * tiles <= CHIP ? 2 : 0; }
+  MOK_SCHED_FN int gate_up_items() const { return row_tiles * gate_up_cols << gate_up_cut; }
+  MOK_SCHED_FN int down_items() const { return row_tiles * down_cols << down_cut; }
 
   // List q: the q-th eighth of the gate/up tiles (all experts' tiles in one sequence: expert by expert, column tile by
   // column tile, row tiles innermost), then the q-th eighth of the down tiles.
   MOK_SCHED_FN int share(int q, int total) const { return (int)((long long)q * total / NUM_XCD); }
   MOK_SCHED_FN int length(int q) const {
-    const int gu = row_tiles * gate_up_cols, d = row_tiles * down_cols;
+    const int gu = gate_up_items(), d = down_items();
     return share(q + 1, gu) - share(q, gu) + share(q + 1, d) - share(q, d);
   }
 
   // item i of list q -> task.  `cursor` is the expert of the item this workgroup decoded last: a workgroup's items
   // come in growing order as long as it stays in one GEMM, so the search usually ends where it starts.
   MOK_SCHED_FN MokGemmTask decode(int q, int i, int& cursor) const {
-    const int gu = row_tiles * gate_up_cols, d = row_tiles * down_cols;
-    const int gate_up_items = share(q + 1, gu) - share(q, gu);
-    const bool gate_up = i < gate_up_items;
-    const int idx = gate_up ? share(q, gu) + i : share(q, d) + i - gate_up_items;  // in the sequence of its GEMM's tiles
+    const int gu = gate_up_items(), d = down_items();
+    const int mine = share(q + 1, gu) - share(q, gu);
+    const bool gate_up = i < mine;
+    const int item = gate_up ? share(q, gu) + i : share(q, d) + i - mine;  // in the sequence of its GEMM's items
+    const int cut = gate_up ? gate_up_cut : down_cut;                      // a column tile's parts are neighbours
+    const int idx = item >> cut, part = item - (idx << cut);
     const int cols = gate_up ? gate_up_cols : down_cols;
     // last e with tile_begin[e] * cols <= idx: it has row tiles, since tile_begin[e + 1] * cols > idx
     // (a workgroup's next item is usually the same expert's)
@@ -130,11 +155,11 @@ struct Schedule {
     t.expert = e;
     t.row_begin = MOK_SCHED_UNIFORM(first);
     t.row_end = MOK_SCHED_UNIFORM(tab.row_begin[e + 1]);
-    t.col_begin = MOK_SCHED_UNIFORM(col * (gate_up ? TILE_W / 2 : TILE_W));
+    t.col_begin = MOK_SCHED_UNIFORM(((col << cut) + part) * ((gate_up ? TILE_W / 2 : TILE_W) >> cut));
     t.task_idx = MOK_SCHED_UNIFORM(q << 24 | i);
     t.counter_idx = MOK_SCHED_UNIFORM(both ? tile : -1);
-    t.wait_target = gate_up ? 0 : gate_up_cols;
-    t.flags = 0u;
+    t.wait_target = gate_up ? 0 : gate_up_cols << gate_up_cut;
+    t.flags = (uint32_t)MOK_SCHED_UNIFORM(cut != 0 ? MOK_TASK_QUARTER : 0);
     return t;
   }
 };

@@ -59,6 +59,7 @@ constexpr int W_LOADS = W_GROUPS;              // loads of one weight slot issue
 // extent returns zeros instead of faulting.  One operand of one expert is 16 MiB below 4 GiB
 // (the host checks).
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 // Lane offset of the rows and columns a tile has past the end of its expert's rows or of the
 // weight matrix: beyond every extent (the host keeps operands 16 MiB below 4 GiB), so the
@@ -218,19 +219,32 @@ __device__ __forceinline__ v8i read_frag(const unsigned char* slot, int off) {
   return r;
 }
 
-// A zeroed accumulator fragment.  Written by one instruction of the matrix pipe (an integer MFMA of zeros, eight
+// Zeroed accumulator fragments.  Each is written by one instruction of the matrix pipe (an integer MFMA of zeros, eight
 // passes) instead of sixteen register writes: a wave issues in order, one instruction every four or five clocks, and 256
 // writes per tile are half a microsecond in which it issues nothing else.  (The zero is opaque to the compiler, which
 // would otherwise fold the product back into the writes.)
-// The instruction is written out so that its result is born in the accumulator registers (left to the compiler it
-// may be born in vector registers and copied, which the mainloop has none to spare for); nothing reads the fragment
-// for hundreds of instructions, so the matrix pipe's result latency needs no attention here.
-__device__ __forceinline__ v16f zero_fragment() {
+// The instructions are written out so that their results are born in the accumulator registers (left to the compiler
+// they may be born in vector registers and copied, which the mainloop has none to spare for).  The compiler does not know
+// that they take eight passes and may copy a result at once, so all fragments of a tile are cleared in one block that ends
+// behind the last result.
+#define PL_ZERO(N, Z) "v_mfma_i32_32x32x16_i8 %" #N ", %" #Z ", %" #Z ", 0\n"
+#define PL_ZEROED "s_nop 15\ns_nop 3"
+__device__ __forceinline__ void zero_fragments(v16f& a, v16f& b, v16f& c, v16f& d) {
   long z = 0;
-  v16f f;
-  asm volatile("v_mfma_i32_32x32x16_i8 %0, %1, %1, 0" : "=a"(f) : "v"(z));
-  return f;
+  asm volatile(PL_ZERO(0, 4) PL_ZERO(1, 4) PL_ZERO(2, 4) PL_ZERO(3, 4) PL_ZEROED : "=a"(a), "=a"(b), "=a"(c), "=a"(d) : "v"(z));
 }
+__device__ __forceinline__ void zero_fragments(AccFrag& acc) {
+  long z = 0;
+  asm volatile(PL_ZERO(0, 16) PL_ZERO(1, 16) PL_ZERO(2, 16) PL_ZERO(3, 16) PL_ZERO(4, 16) PL_ZERO(5, 16) PL_ZERO(6, 16) PL_ZERO(7, 16)
+               PL_ZERO(8, 16) PL_ZERO(9, 16) PL_ZERO(10, 16) PL_ZERO(11, 16) PL_ZERO(12, 16) PL_ZERO(13, 16) PL_ZERO(14, 16) PL_ZERO(15, 16)
+               PL_ZEROED
+               : "=a"(acc.v[0][0]), "=a"(acc.v[0][1]), "=a"(acc.v[0][2]), "=a"(acc.v[0][3]), "=a"(acc.v[1][0]), "=a"(acc.v[1][1]),
+                 "=a"(acc.v[1][2]), "=a"(acc.v[1][3]), "=a"(acc.v[2][0]), "=a"(acc.v[2][1]), "=a"(acc.v[2][2]), "=a"(acc.v[2][3]),
+                 "=a"(acc.v[3][0]), "=a"(acc.v[3][1]), "=a"(acc.v[3][2]), "=a"(acc.v[3][3])
+               : "v"(z));
+}
+#undef PL_ZEROED
+#undef PL_ZERO
 
 // Workgroup barrier without the release/acquire fence of __syncthreads(): a fence would
 // drain every outstanding global->LDS load (vmcnt(0)) and serialise the ring.  Ordering of
@@ -533,11 +547,150 @@ __device__ __forceinline__ void wait_few(int loads) {  // a multiple of FEW_LOAD
 // which placement the task's tile has: its routed rows that exist, its output columns that exist
 __device__ __forceinline__ int placement_of(const MokGemmResidue& g, const MokGemmTask& t) {
   const int cols = (t.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? g.w_gate.rows : g.w_down.rows) - t.col_begin;
-  return tile_placement(t.row_end - t.row_begin, cols);
+  return tile_placement(t.row_end - t.row_begin, cols, t.flags);
+}
+
+// ---- narrow tiles: a quarter of a column tile for at most 32 routed rows -----------------------------------------------
+// A launch of a few tokens has fewer column tiles than the chip has compute units, and one compute unit streams weights
+// at about 40 GB/s whatever the others do: the launch takes as long as one tile's stream.  The schedule then cuts each
+// column tile in four (schedule.hpp says when, and what it measured).
+// 64 weight rows would leave waves without a fragment, so the waves split the contraction instead: wave w multiplies every
+// fourth pair of slots, all 64 weight rows x 32 routed rows, from a ring of its own that no other wave touches -- no barrier
+// in the loop -- and the four partial sums meet in wave 0 through LDS.
+//   a wave's LDS: 16 KB of the head, 20 KB of the arena and 3 KB of scale buffers (four pairs of 256 B each for the two
+//   halves of the weight rows and the routed rows); a slot is 4 KB of weight rows and 2 KB of routed rows.
+constexpr int NARROW_ROWS = 32;
+template <int DEPTH>
+struct NarrowRing {
+  static constexpr int HALF_BYTES = NARROW_ROWS * K_SLOT;                     // a half of the weight rows
+  static constexpr int SLOT_BYTES = 2 * HALF_BYTES + NARROW_ROWS * K_SLOT;    // 6 KB
+  static constexpr int ARENA = (2 * DEPTH - 3) * BUF_BYTES / WAVES;           // bytes per wave
+  static constexpr int HEAD_SLOTS = BUF_BYTES / SLOT_BYTES;                   // 2
+  static constexpr int SLOTS = HEAD_SLOTS + ARENA / SLOT_BYTES;               // 5 (2 with the arena of depth 2)
+  static_assert(SLOTS <= 6, "a slot's scales outlive the ring's turn: four pairs of scale buffers");
+  unsigned char *head, *arena, *scales;
+  __device__ __forceinline__ explicit NarrowRing(int wave) {
+    const Rings<DEPTH> r;
+    head = r.head + wave * BUF_BYTES;
+    arena = r.arena + wave * ARENA;
+    scales = r.wscale() + wave * ((WSCALE_BYTES + XSCALE_BYTES) / WAVES);
+  }
+  __device__ __forceinline__ unsigned char* slot(int pos) const {  // pos = the wave's slot mod SLOTS
+    return pos < HEAD_SLOTS ? head + pos * SLOT_BYTES : arena + (pos - HEAD_SLOTS) * SLOT_BYTES;
+  }
+  __device__ __forceinline__ unsigned char* pair(int p) const { return scales + (p & 3) * 768; }  // the wave's p-th pair
+};
+struct NarrowLoader {
+  rsrc_t x, xsc, w[2], wsc[2];     // w: gate and up matrix, or the down matrix twice
+  uint32_t wsrc[2][2];             // [half of the weight rows][16-row group]
+  uint32_t wscsrc[2];              // this lane's weight row of each half
+  uint32_t w_slot_pitch, wsc_pair_pitch;
+  bool written;                    // the routed rows are this launch's `hidden`: read at device scope
+};
+__device__ __forceinline__ void gather_narrow(const MokGemmResidue& g, const MokGemmTask& t, GemmCarry& c) {
+  const int lane = fresh_tid() & 63;
+  const bool gate_up = t.op == MOK_GEMM_FWD_ROUTED_GATE_UP;
+  const MokMxView& act = gate_up ? g.x : g.hidden;
+  const bool gathered = gate_up && g.row_token;
+  const int32_t* staged_token = reinterpret_cast<const int32_t*>(Rings<2>().tokens());
+  const int lrow = lane >> 2, chunk = 16 * ((lane & 3) ^ swizzle(lrow));
+  auto source = [&](int trow) { return gathered ? staged_token[trow] : t.row_begin + trow; };
+#pragma unroll
+  for (int i = 0; i < X_GROUPS; ++i) {  // (two groups of 16 rows; the carry has room for four)
+    const int trow = (i & 1) * 16 + lrow;
+    c.xsrc[i] = t.row_begin + trow < t.row_end ? (uint32_t)source(trow) * (uint32_t)act.ld_q + chunk : PAST_THE_END;
+  }
+  const int srow = lane & 31;
+  c.xscsrc = t.row_begin + srow < t.row_end ? (uint32_t)source(srow) * (uint32_t)act.ld_sc : PAST_THE_END;
+}
+__device__ __forceinline__ NarrowLoader make_narrow_loader(const MokGemmResidue& g, const MokGemmTask& t) {
+  const int lane = fresh_tid() & 63;
+  const bool gate_up = t.op == MOK_GEMM_FWD_ROUTED_GATE_UP;
+  const int expert = __builtin_amdgcn_readfirstlane(t.expert);
+  const MokMxView& act = gate_up ? g.x : g.hidden;
+  NarrowLoader ld;
+  ld.x = make_rsrc(act.q, (uint32_t)act.rows * (uint32_t)act.ld_q);
+  ld.xsc = make_rsrc(act.sc, (uint32_t)act.rows * (uint32_t)act.ld_sc);
+  ld.written = !gate_up;
+  const int lrow = lane >> 2, chunk = 16 * ((lane & 3) ^ swizzle(lrow));
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const MokMxView& wv = !gate_up ? g.w_down : h ? g.w_up : g.w_gate;
+    const int col0 = t.col_begin + (gate_up ? 0 : NARROW_ROWS * h);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int col = col0 + i * 16 + lrow;
+      ld.wsrc[h][i] = col < wv.rows ? (uint32_t)col * (uint32_t)K_SLOT + chunk : PAST_THE_END;
+    }
+    const int scol = col0 + (lane & (NARROW_ROWS - 1));
+    ld.wscsrc[h] = scol < wv.rows ? (uint32_t)scol * 4u : PAST_THE_END;
+    ld.w[h] = make_rsrc(wv.q + (int64_t)expert * wv.expert_pitch_q, (uint32_t)wv.rows * (uint32_t)wv.k);
+    ld.wsc[h] = make_rsrc(wv.sc + (int64_t)expert * wv.expert_pitch_sc, (uint32_t)((wv.k + K_PAIR - 1) / K_PAIR) * (uint32_t)wv.rows * 4u);
+  }
+  const int rows = gate_up ? g.w_gate.rows : g.w_down.rows;
+  ld.w_slot_pitch = (uint32_t)rows * (uint32_t)K_SLOT;
+  ld.wsc_pair_pitch = (uint32_t)rows * 4u;
+  return ld;
+}
+// all loads of the wave's i-th slot, into ring position pos: [a pair's block scales] [routed rows] [weight rows]
+template <int DEPTH>
+__device__ __forceinline__ void issue_narrow(const NarrowLoader& ld, const GemmCarry& c, const NarrowRing<DEPTH>& ring, int wave,
+                                             int i, int pos, int mine) {
+  using Ring = NarrowRing<DEPTH>;
+  if (i >= mine) return;
+  const int s = counts::narrow_slot(wave, i);
+  const uint32_t kbyte = (uint32_t)s * K_SLOT;
+  unsigned char* base = ring.slot(pos);
+  if ((i & 1) == 0) {
+    unsigned char* sc = ring.pair(i >> 1);
+    buf4_to_lds(ld.wsc[0], ld.wscsrc[0], (uint32_t)(s >> 1) * ld.wsc_pair_pitch, sc);
+    buf4_to_lds(ld.wsc[1], ld.wscsrc[1], (uint32_t)(s >> 1) * ld.wsc_pair_pitch, sc + 256);
+    buf4_to_lds_device_scope(ld.xsc, c.xscsrc, kbyte >> 5, sc + 512);
+  }
+  // (narrow gate/up tiles of one row share its cache lines and may run on different XCDs: a line of `hidden` that an L2
+  // holds can be out of date, so the down op does not trust it)
+  unsigned char* x = base + 2 * Ring::HALF_BYTES;
+  if (ld.written) {
+    buf16_to_lds_device_scope(ld.x, c.xsrc[0], kbyte, x);
+    buf16_to_lds_device_scope(ld.x, c.xsrc[1], kbyte, x + 1024);
+  } else {
+    buf16_to_lds(ld.x, c.xsrc[0], kbyte, x);
+    buf16_to_lds(ld.x, c.xsrc[1], kbyte, x + 1024);
+  }
+  const uint32_t wslot = (uint32_t)s * ld.w_slot_pitch;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) buf16_to_lds(ld.w[h], ld.wsrc[h][k], wslot, base + h * Ring::HALF_BYTES + k * 1024);
+}
+// the counts narrow_younger can give: 6 loads a slot, 9 with scales, behind up to four slots
+__device__ __forceinline__ void wait_narrow(int loads) {
+  switch (__builtin_amdgcn_readfirstlane(loads)) {
+    case 6: wait_loads_and_reads<6>(); break;
+    case 9: wait_loads_and_reads<9>(); break;
+    case 15: wait_loads_and_reads<15>(); break;
+    case 21: wait_loads_and_reads<21>(); break;
+    case 24: wait_loads_and_reads<24>(); break;
+    case 30: wait_loads_and_reads<30>(); break;
+    default: wait_loads_and_reads<0>(); break;  // waiting for everything is always right
+  }
+  asm volatile("" ::: "memory");  // (no barrier follows that would keep the reads behind the wait)
+}
+
+template <int DEPTH>
+__device__ __forceinline__ void prefetch_narrow(const MokGemmResidue& g, const MokGemmTask& t, GemmCarry& c) {
+  const int wave = __builtin_amdgcn_readfirstlane(fresh_tid() >> 6);
+  const int mine = counts::narrow_slots(wave, (t.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? g.x : g.hidden).k / K_SLOT);
+  gather_narrow(g, t, c);
+  const NarrowLoader ld = make_narrow_loader(g, t);
+  const NarrowRing<DEPTH> ring(wave);
+#pragma unroll
+  for (int i = 0; i < NarrowRing<DEPTH>::HEAD_SLOTS; ++i) issue_narrow(ld, c, ring, wave, i, i, mine);
 }
 
 template <int DEPTH>
 __device__ __forceinline__ void prefetch(const MokGemmResidue& g, const MokGemmTask& t, GemmCarry& c) {
+  if (__builtin_expect(t.flags & MOK_TASK_QUARTER, 0)) return prefetch_narrow<DEPTH>(g, t, c);
   const Views v = views_of(g, t);
   const int n = v.act.k / K_SLOT;
   if constexpr (DEPTH >= 4) {
@@ -590,10 +743,7 @@ __device__ __forceinline__ void mainloop(const MokGemmResidue& g, const MokGemmT
   // The accumulator is cleared further down, on each of the two paths by itself (an idle wave's as well: one it left
   // unwritten would be the previous tile's, kept alive across the loop).
   auto clear_accumulator = [&]() {
-#pragma unroll
-    for (int a = 0; a < WFRAGS; ++a)
-#pragma unroll
-      for (int b = 0; b < XFRAGS; ++b) acc.v[a][b] = zero_fragment();
+    zero_fragments(acc);
   };
 
   static_assert(DEPTH % 2 == 0, "routed-row pairs start on even steps");
@@ -818,11 +968,9 @@ __device__ __forceinline__ void mainloop_small(const MokGemmResidue& g, const Mo
     woff[a] = wl * K_SLOT + 16 * (half ^ swizzle(wl));
     wscoff[a] = wl * 4;
   }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-      if (used(a)) acc.v[a][b] = zero_fragment();
+  constexpr int A1 = FRAGS & 2 ? 1 : 2;  // two of the four weight fragments are used, or all
+  zero_fragments(acc.v[0][0], acc.v[0][1], acc.v[A1][0], acc.v[A1][1]);
+  if constexpr (FRAGS == SMALL_COLS_FRAGS_GATE_UP) zero_fragments(acc.v[2][0], acc.v[2][1], acc.v[3][0], acc.v[3][1]);
 
   // the prologue of the full tile: steps -DEPTH and 1 - DEPTH were issued by `prefetch`
 #pragma unroll
@@ -929,10 +1077,7 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
     woff[a] = wl * K_SLOT + 16 * (half ^ swizzle(wl));
     wscoff[a] = wl * 4;
   }
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc.v[2 * a][b] = zero_fragment();
+  zero_fragments(acc.v[0][0], acc.v[0][1], acc.v[2][0], acc.v[2][1]);
 
   // slots 0 .. FEW_HEAD_SLOTS - 1 were asked for by `prefetch`; the rest of the ring now
 #pragma unroll
@@ -997,6 +1142,101 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
   wg_barrier();  // every wave holds its last operands in registers: the ring is free
 }
 
+// The mainloop of a narrow tile: leaves the sums in wave 0's fragments [0][0] and [2][0].
+template <int DEPTH>
+__device__ __forceinline__ void mainloop_narrow(const MokGemmResidue& g, const MokGemmTask& t, AccFrag& acc, const GemmCarry& carry,
+                                                const MokGemmTask* upcoming, const MokCounters& counters) {
+  const int tid = fresh_tid();
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r32 = lane & 31, half = lane >> 5;
+  using Ring = NarrowRing<DEPTH>;
+  constexpr int RING = Ring::SLOTS;
+  const int mine = counts::narrow_slots(wave, (t.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? g.x : g.hidden).k / K_SLOT);
+  const NarrowLoader ld = make_narrow_loader(g, t);
+  const Ring ring(wave);
+#pragma unroll
+  for (int i = Ring::HEAD_SLOTS; i < RING; ++i) issue_narrow(ld, carry, ring, wave, i, i, mine);
+  if (upcoming->op != 0) stage(g, *upcoming, counters);
+  const int off = r32 * K_SLOT + 16 * (half ^ swizzle(r32));
+  v16f sum[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[h][r] = 0.0f;
+  struct NarrowOperands {
+    v8i x, w[2];
+  } even, odd;
+  int sx = 0, sw[2] = {0, 0};
+  auto read_operands_narrow = [&](NarrowOperands& o, const unsigned char* slot) {
+    o.x = read_frag(slot + 2 * Ring::HALF_BYTES, off);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) o.w[h] = read_frag(slot + h * Ring::HALF_BYTES, off);
+  };
+  auto scales_of = [&](int p) {
+    const unsigned char* sc = ring.pair(p) + 4 * r32;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) sw[h] = (int)(*reinterpret_cast<const uint32_t*>(sc + 256 * h) >> (8 * half));
+    sx = (int)(*reinterpret_cast<const uint32_t*>(sc + 512) >> (8 * half));
+  };
+  auto multiply = [&](auto ODD_, const NarrowOperands& o) {
+    constexpr bool ODD = decltype(ODD_)::value;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      sum[h] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(o.w[h], o.x, sum[h], 0, 0, ODD ? 2 : 0, sw[h], ODD ? 2 : 0, sx);
+  };
+  if (mine > 0) {
+    wait_narrow(counts::narrow_younger(0, RING - 1, mine));
+    read_operands_narrow(even, ring.slot(0));
+    int pos = 0;
+    // step i: slot i + 1 has landed and slot i is in registers, whose place takes slot i + RING
+    auto advance = [&](int i, NarrowOperands& next) {
+      wait_narrow(counts::narrow_younger(i + 1, i + RING - 1, mine));
+      issue_narrow(ld, carry, ring, wave, i + RING, pos, mine);
+      pos = pos + 1 == RING ? 0 : pos + 1;
+      read_operands_narrow(next, ring.slot(pos));
+    };
+    int i = 0;
+    for (; i + 1 < mine; i += 2) {
+      scales_of(i >> 1);
+      advance(i, odd);
+      multiply(std::false_type{}, even);
+      if (i + 2 < mine) advance(i + 1, even);
+      multiply(std::true_type{}, odd);
+    }
+    if (mine & 1) {
+      scales_of(i >> 1);
+      multiply(std::false_type{}, even);
+    }
+  }
+  // The partial sums meet in wave 0, in the waves' own parts of the head (their last slots are in registers).
+  if (wave != 0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v4f f = {sum[h][4 * q], sum[h][4 * q + 1], sum[h][4 * q + 2], sum[h][4 * q + 3]};
+        *reinterpret_cast<v4f*>(ring.head + (h * 4 + q) * 1024 + lane * 16) = f;
+      }
+  }
+  lds_barrier();
+  if (wave == 0) {
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const v4f f = *reinterpret_cast<const v4f*>(ring.head + w * BUF_BYTES + (h * 4 + q) * 1024 + lane * 16);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[h][4 * q + e] += f[e];
+        }
+  }
+  acc.v[0][0] = sum[0];
+  acc.v[2][0] = sum[1];
+  lds_barrier();  // the partial sums have been read: the head is free
+}
+
 // bf16 epilogue of the down op.  The accumulator is transposed through the arena buffers (idle
 // by now; the head may already hold the next tile's first slots) so that the global stores
 // are 16 bytes per lane and 512 contiguous bytes per routed row; an arena too small for the
@@ -1010,6 +1250,29 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   const f32x2 v = {a, b};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));  // v_cvt_pk_bf16_f32, nearest even
+}
+
+__device__ __forceinline__ void store_narrow(const MokGemmResidue& g, const MokGemmTask& t, const AccFrag& acc) {
+  const int tid = fresh_tid();
+  const int lane = tid & 63;
+  const int row = t.row_begin + (lane & 31);
+  if (tid < 64) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const v16f f = from_acc(acc.v[2 * h][0]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int col = t.col_begin + 32 * h + 8 * q + 4 * (lane >> 5);
+        if (row < t.row_end && col < g.w_down.rows) {
+          uint2 pk;
+          pk.x = pack_bf16x2(f[4 * q + 0], f[4 * q + 1]);
+          pk.y = pack_bf16x2(f[4 * q + 2], f[4 * q + 3]);
+          *reinterpret_cast<uint2*>(g.y + (int64_t)row * g.ld_y + col) = pk;
+        }
+      }
+    }
+  }
+  lds_barrier();  // (as every epilogue ends: the waves leave together)
 }
 
 template <int DEPTH, int FRAGS>  // FRAGS: 0 for a full tile, else the fragments a small tile's waves hold
@@ -1202,9 +1465,17 @@ extern "C" __device__ void mok_gemm_fwd_small(const void* view, const MokGemmTas
 #define PL_SMALL(D, F) case F: mok_gemm_owner::mainloop_small<D, F>(g, *task, placement, *acc, *carry, upcoming, *counters); break;
   switch (pipelink_mok_gemm_depth()) {
     case 2:
+      if (__builtin_expect(placement == mok::TILE_NARROW, 0)) {
+        mok_gemm_owner::mainloop_narrow<2>(g, *task, *acc, *carry, upcoming, *counters);
+        break;
+      }
       switch (frags) { PL_SMALL(2, mok::SMALL_ROWS_FRAGS) PL_SMALL(2, mok::SMALL_COLS_FRAGS_GATE_UP) PL_SMALL(2, mok::SMALL_COLS_FRAGS_DOWN) }
       break;
     default:
+      if (__builtin_expect(placement == mok::TILE_NARROW, 0)) {
+        mok_gemm_owner::mainloop_narrow<4>(g, *task, *acc, *carry, upcoming, *counters);
+        break;
+      }
       if (placement == mok::TILE_SMALL_ROWS) {  // (the deep ring needs the arena of depth 4; mok_gemm_prefetch decides alike)
         mok_gemm_owner::mainloop_few_rows(g, *task, *acc, *carry, upcoming, *counters);
         break;
@@ -1229,6 +1500,7 @@ extern "C" __device__ void mok_gemm_store(const void* view, const MokGemmTask* t
 extern "C" __device__ void mok_gemm_store_small(const void* view, const MokGemmTask* task, const mok::AccFrag* acc) {
   const auto& g = mok_gemm_residue(view);
   const int placement = mok_gemm_owner::placement_of(g, *task);
+  if (__builtin_expect(placement == mok::TILE_NARROW, 0)) return mok_gemm_owner::store_narrow(g, *task, *acc);
 #define PL_STORE(D)                                                                                                  \
   if (placement == mok::TILE_SMALL_ROWS) mok_gemm_owner::store_down<D, mok::SMALL_ROWS_FRAGS>(g, *task, placement, *acc); \
   else mok_gemm_owner::store_down<D, mok::SMALL_COLS_FRAGS_DOWN>(g, *task, placement, *acc);

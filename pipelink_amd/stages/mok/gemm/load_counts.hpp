@@ -52,6 +52,24 @@ MOK_COUNT_FN int few_younger(int slot, int last, int n) {
   return younger;
 }
 
+// A narrow tile's waves split the contraction: wave w takes the pairs of slots w, w + 4, w + 8, ... for itself, through a
+// ring of its own.  Its i-th slot; how many it has of a contraction of n slots; the loads of one
+// (a pair's block scales come with its first slot); the loads behind slot `slot` when slots up to `last` have been issued.
+constexpr int NARROW_SCALE_LOADS = 3;  // two halves of the weight rows, the routed rows
+constexpr int NARROW_LOADS = 6;        // two groups of 16 routed rows, two of each half
+MOK_COUNT_FN int narrow_slot(int wave, int i) { return ((i >> 1) * 4 + wave) * 2 + (i & 1); }
+MOK_COUNT_FN int narrow_slots(int wave, int n) {
+  const int pairs = (n + 1) / 2;
+  const int mine = (pairs - wave + 3) / 4;  // pairs of this wave (wave <= 3: not negative)
+  // the contraction's last pair may be half a pair
+  return mine > 0 && (n & 1) && (mine - 1) * 4 + wave == pairs - 1 ? 2 * mine - 1 : 2 * mine;
+}
+MOK_COUNT_FN int narrow_younger(int slot, int last, int mine) {
+  int younger = 0;
+  for (int k = slot + 1; k <= last; ++k) younger += k < mine ? NARROW_LOADS + (k & 1 ? 0 : NARROW_SCALE_LOADS) : 0;
+  return younger;
+}
+
 }  // namespace counts
 }  // namespace mok_gemm_owner
 

@@ -34,6 +34,9 @@ enum { MOK_ACT_FWD_ROUTED = 1 };
 
 #ifndef MOKGEMMTASK_DEFINED
 #define MOKGEMMTASK_DEFINED
+/* MokGemmTask.flags, MokActTask.flags */
+enum { MOK_TASK_QUARTER = 1 }; /* a quarter of a column tile (32 gate + 32 up columns, or 64 down columns) of at most 32 rows */
+
 typedef struct MokGemmTask {
   int32_t op;        /* MOK_GEMM_FWD_ROUTED_GATE_UP or MOK_GEMM_FWD_ROUTED_DOWN */
   int32_t expert;    /* local expert whose weights this tile multiplies */

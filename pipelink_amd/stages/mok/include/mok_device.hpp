@@ -69,15 +69,20 @@ __device__ __forceinline__ int xrow0(int wave, int b) { return wave_x(wave) * 12
 // wave takes 64 routed rows and up to four 32-row weight fragments, in the accumulator's fragments [a][b] with b < 2.
 //   SMALL_ROWS: all four waves share routed rows 0..63; wave w owns weight fragments a = 0 and a = 2, tile rows
 //               32 w and 128 + 32 w (for the gate/up op: 32 gate columns and the same 32 up columns).
+//   NARROW:     (a task that is a quarter of a column tile, MOK_TASK_QUARTER: at most 32 rows) the waves split the
+//               contraction; the sums are in wave 0, fragments a = 0 and a = 2, b = 0: rows 0..31 of the task's gate and up
+//               rows, or its rows 0..31 and 32..63 of the down matrix.  The other waves hold nothing.
 //   SMALL_COLS: wave w owns routed rows 64 w .. 64 w + 63; the weight fragments are tile rows 0, 32 (a = 0, 1) and,
 //               for the gate/up op, 128, 160 (a = 2, 3): 64 gate columns and the same 64 up columns.
 // Element (reg r, lane l) of fragment (a, b) is weight row wr[a] + 8 (r / 4) + 4 (l / 32) + r % 4, routed row
-// xr0 + 32 b + l % 32.  Which placement a tile has follows from its extent alone, so every owner works it out for itself.
-enum { TILE_FULL = 0, TILE_SMALL_ROWS = 1, TILE_SMALL_COLS = 2 };
+// xr0 + 32 b + l % 32.  Which placement a tile has follows from its extent and its flags alone, so every owner works it
+// out for itself.
+enum { TILE_FULL = 0, TILE_SMALL_ROWS = 1, TILE_SMALL_COLS = 2, TILE_NARROW = 3 };
 constexpr int SMALL_EXTENT = 64;
 // rows: routed rows of the tile that exist; cols: output columns (per weight matrix) from the tile's first that exist
-__device__ __forceinline__ int tile_placement(int rows, int cols) {
-  return rows <= SMALL_EXTENT ? TILE_SMALL_ROWS : cols <= SMALL_EXTENT ? TILE_SMALL_COLS : TILE_FULL;
+__device__ __forceinline__ int tile_placement(int rows, int cols, uint32_t flags) {
+  return flags & MOK_TASK_QUARTER ? TILE_NARROW
+         : rows <= SMALL_EXTENT ? TILE_SMALL_ROWS : cols <= SMALL_EXTENT ? TILE_SMALL_COLS : TILE_FULL;
 }
 struct SmallPlacement {
   int xr0;    // first tile-local routed row of the wave

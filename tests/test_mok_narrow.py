@@ -1,0 +1,140 @@
+"""Column tiles cut in parts for launches of few rows: the schedule and the wait counts on the CPU, the forward on the GPU."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+STAGE = os.path.join(ROOT, "pipelink_amd", "stages", "mok")
+
+SCHEDULE = r"""
+#define MOK_SCHED_FN inline
+#define MOK_SCHED_UNIFORM(x) (x)
+#include "framework/schedule.hpp"
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+using namespace mok_framework;
+int main(int argc, char** argv) {
+  const int op = atoi(argv[1]), gu = atoi(argv[2]), dn = atoi(argv[3]);
+  std::vector<int32_t> counts;
+  for (int a = 4; a < argc; ++a) counts.push_back(atoi(argv[a]));
+  const int ne = (int)counts.size();
+  // the tables a wave's lanes make, by 64 lanes one after the other
+  static Tables tab, want;
+  want.fill(counts.data(), ne);
+  int lane_c[64], lane_t[64];
+  for (int pass = 0; pass < 2; ++pass)   // the second pass has every lane's scan at hand
+    for (int lane = 0; lane < 64; ++lane) {
+      int call = 0;
+      tab.fill_by_wave(counts.data(), ne < 64 ? ne : 64, lane,
+        [&](int v) { int* mine = call++ % 2 ? lane_t : lane_c; if (!pass) mine[lane] = v; int s = 0; for (int l = 0; l <= lane; ++l) s += mine[l]; return s; },
+        [&](int) { return 0; }, [&](bool) { bool more = false; for (int c : counts) more = more || c > NARROW_ROWS; return more; });
+    }
+  for (int e = 0; e < ne; ++e) if (tab.row_begin[e] != want.row_begin[e] || tab.tile_begin[e] != want.tile_begin[e]) { printf("table differs at %d\n", e); return 2; }
+  const int narrow = (int)tab.last;
+  const MokFrameworkParams g{counts.data(), nullptr, ne, op, gu, dn};
+  Schedule sched{g, want, want.tile_begin[ne], op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : gu, op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : dn};
+  if (narrow) sched.cut();
+  printf("%d %d %d\n", narrow, 1 << sched.gate_up_cut, 1 << sched.down_cut);
+  for (int q = 0; q < NUM_XCD; ++q)
+    for (int i = 0, cursor = 0; i < sched.length(q); ++i) {
+      const MokGemmTask t = sched.decode(q, i, cursor);
+      printf("%d %d %d %d %d %d %u\n", t.op, t.expert, t.row_begin, t.row_end, t.col_begin, t.wait_target, t.flags);
+    }
+}
+"""
+
+COUNTS = r"""
+#define MOK_COUNT_FN constexpr inline
+#include "gemm/load_counts.hpp"
+#include <cstdio>
+#include <vector>
+using namespace mok_gemm_owner::counts;
+int main() {
+  int bad = 0;
+  for (int n = 1; n <= 64; ++n) {
+    std::vector<int> seen(n, 0);
+    for (int wave = 0; wave < 4; ++wave) {
+      const int mine = narrow_slots(wave, n);
+      for (int i = 0; i < mine; ++i) { const int s = narrow_slot(wave, i); if (s >= n) { ++bad; continue; } ++seen[s]; }
+      for (int ring : {2, 5})
+        for (int i = -1; i + 1 < mine; ++i) {
+          std::vector<int> order;   // which slot each load is of, in issue order, when the wave waits for slot i + 1
+          for (int k = 0; k < mine && k <= (i < 0 ? ring - 1 : i + ring - 1); ++k)
+            for (int l = 0; l < 6 + (k % 2 ? 0 : 3); ++l) order.push_back(k);
+          int behind = 0;
+          for (int k : order) behind += k > i + 1;
+          const int got = i < 0 ? narrow_younger(0, ring - 1, mine) : narrow_younger(i + 1, i + ring - 1, mine);
+          if (got != behind) { if (bad++ < 5) printf("n %d wave %d ring %d slot %d: %d, not %d\n", n, wave, ring, i + 1, got, behind); }
+        }
+    }
+    for (int s = 0; s < n; ++s) if (seen[s] != 1) { if (bad++ < 5) printf("n %d: slot %d taken %d times\n", n, s, seen[s]); }
+  }
+  return bad != 0;
+}
+"""
+
+
+def _compile(tmp_path, source):
+    if shutil.which("g++") is None:
+        pytest.skip("needs g++")
+    (tmp_path / "t.cpp").write_text(source)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", f"-I{STAGE}", str(tmp_path / "t.cpp"), "-o", str(tmp_path / "t")], check=True)
+    return str(tmp_path / "t")
+
+
+def test_narrow_waves_share_the_slots_and_count_their_loads(tmp_path):
+    res = subprocess.run([_compile(tmp_path, COUNTS)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
+
+
+def test_parts_cover_every_column_tile_once(tmp_path):
+    exe = _compile(tmp_path, SCHEDULE)
+    for op, gu, dn, counts, parts in [(0, 23, 12, [0, 1, 0, 1, 1, 1] + [0] * 26, (1, 4)), (0, 23, 12, [1] * 8 + [0] * 24, (1, 1)),
+                                      (0, 23, 12, [1] * 11, (1, 1)), (0, 6, 2, [32, 1, 0, 7], (4, 4)), (0, 6, 2, [33, 1, 0, 7], (1, 1)),
+                                      (3, 23, 12, [1, 1], (4, 4)), (5, 23, 12, [1, 1, 1, 1], (1, 4)),
+                                      (0, 2, 12, [5] * 22, (1, 1))]:   # whole down tiles: the gate/up tiles stay whole too
+        out = subprocess.run([exe, str(op), str(gu), str(dn), *map(str, counts)], check=True, capture_output=True, text=True).stdout.splitlines()
+        narrow, *got = map(int, out[0].split())
+        assert narrow == (max(counts) <= 32) and tuple(got) == parts
+        want = set()
+        for e, c in enumerate(counts):
+            first = sum(counts[:e])
+            for top, cols, width, p in ((3, gu, 128, parts[0]), (5, dn, 256, parts[1])):
+                if c and op in (0, top):
+                    target = gu * parts[0] if top == 5 and op == 0 else 0
+                    want |= {(top, e, first, first + c, col * (width // p), target, int(p == 4)) for col in range(cols * p)}
+        items = [tuple(map(int, line.split())) for line in out[1:]]
+        assert len(items) == len(want) and set(items) == want
+
+
+# one to 32 rows an expert (33: whole tiles); a contraction of one slot, fewer pairs than waves, an odd number of slots, one
+# more pair than a ring; columns that end inside a column tile; gate/up and down tiles cut, down tiles only, none; rows of whole cache lines (one launch) or not
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,I,counts", [(64, 64, [1]), (128, 320, [32, 0, 5]), (576, 192, [31, 17, 1, 32]), (704, 1088, [2] * 5),
+                                        (2880, 2880, [1, 0, 1, 1, 1]), (2880, 2880, [3, 2, 1, 1, 32, 9, 1]), (1536, 2048, [4] * 7),
+                                        (448, 704, [33, 2, 1]), (320, 128, [20] * 8)])
+def test_forward_of_few_rows_matches_the_oracle(H, I, counts):
+    from oracle import moe_ffn
+    from pipelink_amd.host import mok_inputs
+    from pipelink_amd.host.mok import MoKSession, code_pitch
+    from pipelink_amd.stages.mok import build as mok_build
+    from test_gpu_moe import TOL, _oracle, _run
+
+    paths = mok_build.images()
+    inp = mok_inputs.generate(max(counts) + 3, H, I, len(counts), 1, seed=H + len(counts), counts=counts)
+    ref = _oracle(inp)
+    ys = []
+    for image in ("linked", "one_unit"):
+        with MoKSession(paths[image].read_bytes(), str(paths["link_json"])) as sess:
+            for launches in (1, 2):
+                sess.launches(launches)
+                for pitch in (None, code_pitch(I)):
+                    hq, hsc, y = _run(sess, inp, H, I, pitch_i=pitch)
+                    yy = y.float().numpy()
+                    assert not np.isnan(yy).any() and moe_ffn.rel_frobenius(yy, ref["y"]) <= TOL
+                    ys.append(yy)
+    assert all(np.array_equal(ys[0], other) for other in ys[1:])   # one launch and two, linked and one unit: the same sums
