@@ -10,8 +10,8 @@ from ..stages.attention.params import params_blobs
 
 HEAD_DIM = 128
 Q_TILE = 128
-# A grid of at most this many tiles of 128 queries is launched as twice as many of 64, each with a wave per half of the
-# keys: us whole / half at 256 compute units: 256 tiles 25.7 / 22.3, 384 tiles 41.4 / 35.4, 480 tiles 54.3 / 54.2, 512 tiles
+# A grid of at most this many tiles of 128 queries is launched as twice as many of 64 through the link's image for that,
+# `half` beside it: us whole / half at 256 compute units: 256 tiles 25.7 / 22.3, 384 tiles 41.4 / 35.4, 480 tiles 54.3 / 54.2, 512 tiles
 # 57.6 / 61.4 and 24.8 / 28.8
 HALF_TILES_UP_TO = 384
 
@@ -37,5 +37,10 @@ def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, 
         raise ValueError("one head of K or V must stay below 2 GiB")
     tiles = b * hq * (s // Q_TILE)
     buffers = {"q": q_bits, "k": k_bits, "v": v_bits, "o": ((b, s, hq * d), np.uint16)}
+    half = Path(link_json).parent.parent / "half" / "link" / "link.json"
+    if tiles <= HALF_TILES_UP_TO and image is None and half.exists():   # (an image of the caller's own is of whole tiles)
+        link_json, grid = half, 2 * tiles
+    else:
+        grid = tiles
     return open_hostless(link_json, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
-                         grid=(tiles if tiles > HALF_TILES_UP_TO else 2 * tiles,), backend=backend, image=image)
+                         grid=(grid,), backend=backend, image=image)

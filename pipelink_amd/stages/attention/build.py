@@ -25,19 +25,38 @@ def build(out: Path = BUILD, one_unit: bool = True) -> dict:
     (out / "pipeline.json").write_text((HERE / "pipeline.json").read_text())
     link = linker.link(out / "pipeline.json", out / "link")
     control = linker.build_one_unit(out / "pipeline.json", out / "link", out / "one_unit.hsaco") if one_unit else None
+    _link_half(out)
     window = out / "window"   # the same core package with the other mask package: only the link is redone
     window.mkdir(exist_ok=True)
     for f in out.glob("*.plink"):
         shutil.copy(f, window / f.name)
     (window / "pipeline.json").write_text((HERE / "pipeline_window.json").read_text())
     windowed = linker.link(window / "pipeline.json", window / "link")
+    _link_half(window)
     for junk in list(out.glob("*.bc")) + list((out / "link").glob("*.bc")) + list(window.glob("*.bc")) + list((window / "link").glob("*.bc")):
         junk.unlink()
     return {"packages": reports, "link": link, "one_unit": control, "window": windowed}
 
 
+def _link_half(cell: Path) -> None:
+    """The cell's link for small grids beside it (``half/``): the same packages with the core's half tiles bound."""
+    from ...pipec import linker
+
+    half = cell / "half"
+    half.mkdir(exist_ok=True)
+    for f in cell.glob("*.plink"):
+        shutil.copy(f, half / f.name)
+    pipeline = json.loads((cell / "pipeline.json").read_text())
+    pipeline["pipeline"]["forced_bindings"]["pipelink_fa_half"] = 1
+    (half / "pipeline.json").write_text(json.dumps(pipeline, indent=1))
+    linker.link(half / "pipeline.json", half / "link")
+    for junk in list(half.glob("*.bc")) + list((half / "link").glob("*.bc")):
+        junk.unlink()
+
+
 def images(out: Path = BUILD) -> dict:
     paths = {"link_json": out / "link" / "link.json", "linked": out / "link" / "pipeline.hsaco", "one_unit": out / "one_unit.hsaco",
+             "half_linked": out / "half" / "link" / "pipeline.hsaco", "window_half_linked": out / "window" / "half" / "link" / "pipeline.hsaco",
              "window_link_json": out / "window" / "link" / "link.json", "window_linked": out / "window" / "link" / "pipeline.hsaco"}
     missing = [str(p) for p in paths.values() if not p.exists()]
     if missing:

@@ -1,5 +1,5 @@
-// Package fa.core: flash-attention forward for one tile of 128 queries of one head, or, in a launch of twice as many
-// workgroups, of 64 (half tiles).
+// Package fa.core: flash-attention forward for one tile of 128 queries of one head, or, as the link decides
+// (pipelink_fa_half), of 64 (half tiles).
 //
 // Orientation.  Scores are computed transposed, S^T = K . Q^T (keys are the MFMA rows, queries the
 // columns), so that a lane holds ONE query (column lane % 32) and 16 of the block's 32 keys: row maxima
@@ -31,6 +31,7 @@
 #include "include/fa_abi.h"
 
 extern "C" __device__ int pipelink_fa_kv();  // byte offset of the K / V^T buffers in dynamic LDS
+extern "C" __device__ int pipelink_fa_half();  // link-time variant: 1 = half tiles
 extern "C" __device__ int pipelink_call_mask_key_count(const void* view, int q_first, int q_last);
 extern "C" __device__ int pipelink_call_mask_key_begin(const void* view, int q_first, int q_last);
 extern "C" __device__ int pipelink_call_mask_all_visible(const void* view, int q_first, int q_last, int k_first, int k_last);
@@ -96,11 +97,11 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
   const pipelink_host_view view{params, nullptr};
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
-  // the host launches a workgroup per tile of 128 queries, or two: which one, the grid says
   const int heads = p.batch * p.q_heads;
-  const bool split = (int64_t)gridDim.x > (int64_t)heads * (p.seq / FA_Q_TILE);
+  const bool split = pipelink_fa_half() != 0;
   const int tile_queries = split ? FA_Q_TILE / 2 : FA_Q_TILE;
   const int q_tiles = p.seq / tile_queries;
+  if (blockIdx.x >= (uint32_t)heads * (uint32_t)q_tiles) return;  // (a grid made for the half tiles runs the whole ones too)
   // Causal tiles cost in proportion to their position: the latest (longest) tiles of every head are
   // dispatched first, so that the grid does not end on a few long ones.  bh = batch * q_heads + head.
   const int tile = q_tiles - 1 - (int)(blockIdx.x / heads), bh = blockIdx.x % heads;
@@ -332,7 +333,8 @@ PL_STAGE("fa.core", "0.1.0");
 PL_PARAMS(FaCoreParams);
 PL_ROLE(core, fa_core_role_core, 4);
 PL_TOPOLOGY(false, "static");
-PL_VARIANT(0, {});
+PL_VARIANT(0, {{"pipelink_fa_half", 0}});
+PL_VARIANT(1, {{"pipelink_fa_half", 1}});
 PL_CALL(mask_key_count, "mask_key_count",
         "extern \"C\" __device__ int pipelink_call_mask_key_count(const void* view, int q_first, int q_last);");
 PL_CALL(mask_key_begin, "mask_key_begin",
@@ -344,6 +346,7 @@ PL_CALL(mask_visible, "mask_visible",
 // two buffers of (K block 16 KB + V block 16 KB)
 PL_CLAIM("pipelink_fa_kv", "smem", 2 * 2 * (64 * 128 * 2), 1024, "kernel");
 PL_USES("pipelink_fa_kv");
+PL_USES("pipelink_fa_half");
 // two workgroups per CU (two waves per SIMD, 256 registers per lane each): one multiplies while the other
 // is in its softmax or waits at its barrier; 2 x 67.6 KB of LDS fit
 PL_FACT("launch.waves_per_simd", 2);
