@@ -14,7 +14,8 @@ from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 BUILD = HERE / "build"
-STAGES = [("fa.core", "core.hip"), ("fa.mask.causal", "mask_causal.hip"), ("fa.mask.window", "mask_window.hip")]
+# package file -> source; fa.core_half is fa.core too, with half tiles
+STAGES = [("fa.core", "core.hip"), ("fa.core_half", "core_half.hip"), ("fa.mask.causal", "mask_causal.hip"), ("fa.mask.window", "mask_window.hip")]
 
 
 def build(out: Path = BUILD, one_unit: bool = True) -> dict:
@@ -39,7 +40,7 @@ def build(out: Path = BUILD, one_unit: bool = True) -> dict:
 
 
 def _link_half(cell: Path) -> None:
-    """The cell's link for small grids beside it (``half/``): the same packages with the core's half tiles bound."""
+    """The cell's link for small grids beside it (``half/``): the same pipeline with the core package of half tiles."""
     from ...pipec import linker
 
     half = cell / "half"
@@ -47,7 +48,9 @@ def _link_half(cell: Path) -> None:
     for f in cell.glob("*.plink"):
         shutil.copy(f, half / f.name)
     pipeline = json.loads((cell / "pipeline.json").read_text())
-    pipeline["pipeline"]["forced_bindings"]["pipelink_fa_half"] = 1
+    for stage in pipeline["pipeline"]["stages"]:
+        if stage["stage_id"] == "fa.core":
+            stage["artifact_path"] = "fa.core_half.plink"
     (half / "pipeline.json").write_text(json.dumps(pipeline, indent=1))
     linker.link(half / "pipeline.json", half / "link")
     for junk in list(half.glob("*.bc")) + list((half / "link").glob("*.bc")):

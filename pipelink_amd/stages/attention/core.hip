@@ -1,5 +1,5 @@
-// Package fa.core: flash-attention forward for one tile of 128 queries of one head, or, as the link decides
-// (pipelink_fa_half), of 64 (half tiles).
+// Package fa.core: flash-attention forward for one tile of 128 queries of one head; compiled by core_half.hip with
+// FA_HALF_TILES, of 64 (half tiles).
 //
 // Orientation.  Scores are computed transposed, S^T = K . Q^T (keys are the MFMA rows, queries the
 // columns), so that a lane holds ONE query (column lane % 32) and 16 of the block's 32 keys: row maxima
@@ -25,13 +25,15 @@
 //
 // Two LDS buffers per operand: block i + 1 is in flight while block i is multiplied; one barrier per block.
 #include <pipelink/stage.hpp>
+#ifndef FA_HALF_TILES
+#define FA_HALF_TILES 0
+#endif
 #ifndef PIPELINK_EMIT
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include "include/fa_abi.h"
 
 extern "C" __device__ int pipelink_fa_kv();  // byte offset of the K / V^T buffers in dynamic LDS
-extern "C" __device__ int pipelink_fa_half();  // link-time variant: 1 = half tiles
 extern "C" __device__ int pipelink_call_mask_key_count(const void* view, int q_first, int q_last);
 extern "C" __device__ int pipelink_call_mask_key_begin(const void* view, int q_first, int q_last);
 extern "C" __device__ int pipelink_call_mask_all_visible(const void* view, int q_first, int q_last, int k_first, int k_last);
@@ -98,7 +100,7 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
   const int heads = p.batch * p.q_heads;
-  const bool split = pipelink_fa_half() != 0;
+  constexpr bool split = FA_HALF_TILES;
   const int tile_queries = split ? FA_Q_TILE / 2 : FA_Q_TILE;
   const int q_tiles = p.seq / tile_queries;
   if (blockIdx.x >= (uint32_t)heads * (uint32_t)q_tiles) return;  // (a grid made for the half tiles runs the whole ones too)
@@ -277,7 +279,7 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
       if (i + 1 < blocks) block(i + 1, std::integral_constant<int, 1>{}, tiles);
     }
   };
-  if (split) {
+  if constexpr (split) {
     stream(std::integral_constant<int, 1>{});
     // the other half of the keys: waves 2 and 3 hand what they have to waves 0 and 1.  A half that has seen no key for a
     // query has no maximum, and nothing to add.
@@ -329,12 +331,15 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
 #include "include/fa_abi.h"
 #endif
 
+#if FA_HALF_TILES
+PL_STAGE("fa.core", "0.1.0-half");
+#else
 PL_STAGE("fa.core", "0.1.0");
+#endif
 PL_PARAMS(FaCoreParams);
 PL_ROLE(core, fa_core_role_core, 4);
 PL_TOPOLOGY(false, "static");
-PL_VARIANT(0, {{"pipelink_fa_half", 0}});
-PL_VARIANT(1, {{"pipelink_fa_half", 1}});
+PL_VARIANT(0, {});
 PL_CALL(mask_key_count, "mask_key_count",
         "extern \"C\" __device__ int pipelink_call_mask_key_count(const void* view, int q_first, int q_last);");
 PL_CALL(mask_key_begin, "mask_key_begin",
@@ -346,7 +351,6 @@ PL_CALL(mask_visible, "mask_visible",
 // two buffers of (K block 16 KB + V block 16 KB)
 PL_CLAIM("pipelink_fa_kv", "smem", 2 * 2 * (64 * 128 * 2), 1024, "kernel");
 PL_USES("pipelink_fa_kv");
-PL_USES("pipelink_fa_half");
 // two workgroups per CU (two waves per SIMD, 256 registers per lane each): one multiplies while the other
 // is in its softmax or waits at its barrier; 2 x 67.6 KB of LDS fit
 PL_FACT("launch.waves_per_simd", 2);
