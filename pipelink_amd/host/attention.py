@@ -1,6 +1,8 @@
 """Host side of the flash-attention prefill example on the host-less route."""
 from __future__ import annotations
 
+import hashlib
+import json
 from pathlib import Path
 
 import numpy as np
@@ -10,10 +12,24 @@ from ..stages.attention.params import params_blobs
 
 HEAD_DIM = 128
 Q_TILE = 128
-# A grid of at most this many tiles of 128 queries is launched as twice as many of 64 through the link's image for that,
+# A grid of at most this many tiles of 128 queries is launched as twice as many of 64 through the link made for that,
 # `half` beside it: us whole / half at 256 compute units: 256 tiles 25.7 / 22.3, 384 tiles 41.4 / 35.4, 480 tiles 54.3 / 54.2, 512 tiles
 # 57.6 / 61.4 and 24.8 / 28.8
 HALF_TILES_UP_TO = 384
+
+
+def _half_of(link_json: str | Path) -> Path | None:
+    """The half-tile link that was made for exactly this link (``stages.attention.build.link_half``), if there is one: a link
+    redone since, with another mask for instance, has other bytes than the one recorded."""
+    link = Path(link_json)
+    half = link.parent.parent / "half"
+    try:
+        of = json.loads((half / "of.json").read_text())
+        same = all(hashlib.sha256(path.read_bytes()).hexdigest() == of[name]
+                   for name, path in (("whole", link), ("half", half / "link" / "link.json")))
+    except (OSError, ValueError, KeyError, TypeError):
+        return None
+    return half / "link" / "link.json" if same else None
 
 
 def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, v_bits: np.ndarray, *, scale: float | None = None,
@@ -37,8 +53,8 @@ def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, 
         raise ValueError("one head of K or V must stay below 2 GiB")
     tiles = b * hq * (s // Q_TILE)
     buffers = {"q": q_bits, "k": k_bits, "v": v_bits, "o": ((b, s, hq * d), np.uint16)}
-    half = Path(link_json).parent.parent / "half" / "link" / "link.json"
-    if tiles <= HALF_TILES_UP_TO and image is None and half.exists():   # (an image of the caller's own is of whole tiles)
+    half = _half_of(link_json) if tiles <= HALF_TILES_UP_TO and image is None else None   # (an image of the caller's own is of whole tiles)
+    if half is not None:
         link_json, grid = half, 2 * tiles
     else:
         grid = tiles

@@ -26,22 +26,24 @@ def build(out: Path = BUILD, one_unit: bool = True) -> dict:
     (out / "pipeline.json").write_text((HERE / "pipeline.json").read_text())
     link = linker.link(out / "pipeline.json", out / "link")
     control = linker.build_one_unit(out / "pipeline.json", out / "link", out / "one_unit.hsaco") if one_unit else None
-    _link_half(out)
+    link_half(out)
     window = out / "window"   # the same core package with the other mask package: only the link is redone
     window.mkdir(exist_ok=True)
     for f in out.glob("*.plink"):
         shutil.copy(f, window / f.name)
     (window / "pipeline.json").write_text((HERE / "pipeline_window.json").read_text())
     windowed = linker.link(window / "pipeline.json", window / "link")
-    _link_half(window)
+    link_half(window)
     for junk in list(out.glob("*.bc")) + list((out / "link").glob("*.bc")) + list(window.glob("*.bc")) + list((window / "link").glob("*.bc")):
         junk.unlink()
     return {"packages": reports, "link": link, "one_unit": control, "window": windowed}
 
 
-def _link_half(cell: Path) -> None:
-    """The cell's link for small grids beside it (``half/``): the same pipeline with the core package of half tiles."""
-    from ...pipec import linker
+def link_half(cell: Path) -> None:
+    """The cell's link for few tiles beside it (``half/``): the same pipeline with the core package of half tiles.  ``half/of.json``
+    holds the sha256 of the two link.json: a session takes this link only in the place of the one it was made for, so a cell
+    that is linked anew runs its own link at every size until this has been called again."""
+    from ...pipec import linker, plink
 
     half = cell / "half"
     half.mkdir(exist_ok=True)
@@ -53,6 +55,8 @@ def _link_half(cell: Path) -> None:
             stage["artifact_path"] = "fa.core_half.plink"
     (half / "pipeline.json").write_text(json.dumps(pipeline, indent=1))
     linker.link(half / "pipeline.json", half / "link")
+    of = {name: plink.sha256_hex((d / "link" / "link.json").read_bytes()) for name, d in (("whole", cell), ("half", half))}
+    (half / "of.json").write_text(json.dumps(of))
     for junk in list(half.glob("*.bc")) + list((half / "link").glob("*.bc")):
         junk.unlink()
 

@@ -3,6 +3,7 @@ import json
 import shutil
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 from pipelink_amd.stages.attention import build as fa_build
@@ -36,3 +37,49 @@ def test_a_pipeline_file_names_core_and_mask_and_nothing_of_their_inside(built, 
     link = linker.link(tmp_path / "pipeline.json", tmp_path / "link")
     assert set(link["bindings"]) == {"pipelink_fa_kv"} and link["observed"]["mfma"] == mfma and link["observed"]["calls"] == 0
     assert [(e["stage_id"], e["bytes"]) for e in link["params"]["entries"]] == [("fa.core", 56), ("fa.mask.causal", 8)]
+
+
+class Recorder:
+    """Device memory on the host; keeps the images that were loaded and the launches."""
+
+    def __init__(self):
+        self.images, self.launches, self.uploads = [], [], 0
+
+    def current(self): pass
+    def allocate(self, size, align=256): return 4096 * (1 + self.uploads)
+    def free(self, addr): pass
+    def zero(self, addr, size, stream=None): pass
+    def upload(self, addr, data, stream=None): self.uploads += 1
+    def synchronize(self, stream=None): pass
+    def module_load(self, image): return self.images.append(image)
+    def module_unload(self, module): pass
+    def module_function(self, module, name, lds=0): return 1
+    def launch(self, fn, params, grid, block, lds, stream=None): self.launches.append(grid[0])
+
+
+def _open(link_json, tiles=4, **kw):
+    """What a session of `tiles` tiles of 128 queries loads and launches: image bytes, workgroups."""
+    from pipelink_amd.host.attention import open_session
+
+    be = Recorder()
+    q, kv = np.zeros((1, tiles, 128, 128), np.uint16), np.zeros((1, 1, 128, 128), np.uint16)
+    open_session(link_json, q, kv, kv, backend=be, **kw).launch()
+    return be.images[0], be.launches[0]
+
+
+def test_few_tiles_run_the_half_tile_link_made_for_their_link_and_no_other(built, tmp_path):
+    from pipelink_amd.pipec import linker
+
+    cell = tmp_path / "cell"
+    shutil.copytree(built, cell)
+    link_json = cell / "link" / "link.json"
+    assert _open(link_json) == ((cell / "half" / "link" / "pipeline.hsaco").read_bytes(), 8)
+    assert _open(link_json, tiles=400) == ((cell / "link" / "pipeline.hsaco").read_bytes(), 400)
+    # another mask in the pipeline and only the link redone: few tiles run it too, not what was linked before
+    (cell / "pipeline.json").write_text(json.dumps(_pipeline(mask="fa.mask.window")))
+    linker.link(cell / "pipeline.json", cell / "link")
+    relinked = (cell / "link" / "pipeline.hsaco").read_bytes()
+    assert relinked != (built / "link" / "pipeline.hsaco").read_bytes()
+    assert _open(link_json, window=7) == (relinked, 4)
+    fa_build.link_half(cell)   # and the half tiles of the new link, once asked for
+    assert _open(link_json, window=7) == ((cell / "half" / "link" / "pipeline.hsaco").read_bytes(), 8)
