@@ -53,10 +53,8 @@ def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, 
         raise ValueError("one head of K or V must stay below 2 GiB")
     tiles = b * hq * (s // Q_TILE)
     buffers = {"q": q_bits, "k": k_bits, "v": v_bits, "o": ((b, s, hq * d), np.uint16)}
-    half = _half_of(link_json) if tiles <= HALF_TILES_UP_TO and image is None else None   # (an image of the caller's own is of whole tiles)
-    if half is not None:
-        link_json, grid = half, 2 * tiles
-    else:
-        grid = tiles
-    return open_hostless(link_json, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
+    half = _half_of(link_json) if tiles <= HALF_TILES_UP_TO and image is None else None   # (an image of the caller's own is run as it is)
+    facts = json.loads(Path(half or link_json).read_text()).get("facts", {})
+    grid = b * hq * (s // facts.get("fa.core.tile_queries", Q_TILE))
+    return open_hostless(half or link_json, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
                          grid=(grid,), backend=backend, image=image)

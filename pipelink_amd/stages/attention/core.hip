@@ -90,25 +90,21 @@ __device__ __forceinline__ float sum_with_other_half(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-}  // namespace fa_core
 
-extern "C" __device__ void fa_core_role_core(const void* params, unsigned variant) {
-  (void)variant;
-  using namespace fa_core;
-  const FaCoreParams& p = *static_cast<const FaCoreParams*>(params);
-  const pipelink_host_view view{params, nullptr};
+constexpr bool split = FA_HALF_TILES;
+constexpr int TILE_QUERIES = split ? FA_Q_TILE / 2 : FA_Q_TILE;
+
+// one tile; `index` counts them with the longest ones first
+__device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_host_view& view, uint32_t index) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
   const int heads = p.batch * p.q_heads;
-  constexpr bool split = FA_HALF_TILES;
-  const int tile_queries = split ? FA_Q_TILE / 2 : FA_Q_TILE;
-  const int q_tiles = p.seq / tile_queries;
-  if (blockIdx.x >= (uint32_t)heads * (uint32_t)q_tiles) return;  // (a grid made for the half tiles runs the whole ones too)
+  const int q_tiles = p.seq / TILE_QUERIES;
   // Causal tiles cost in proportion to their position: the latest (longest) tiles of every head are
   // dispatched first, so that the grid does not end on a few long ones.  bh = batch * q_heads + head.
-  const int tile = q_tiles - 1 - (int)(blockIdx.x / heads), bh = blockIdx.x % heads;
+  const int tile = q_tiles - 1 - (int)(index / heads), bh = index % heads;
   const int b = bh / p.q_heads, h = bh % p.q_heads, kvh = h / (p.q_heads / p.kv_heads);
-  const int q0 = tile * tile_queries, qw = q0 + 32 * (split ? wave & 1 : wave);  // the wave's first query
+  const int q0 = tile * TILE_QUERIES, qw = q0 + 32 * (split ? wave & 1 : wave);  // the wave's first query
   const int key0 = split ? 32 * (wave >> 1) : 0;                                 // its first key of every block
   const uint32_t head_bytes = (uint32_t)p.seq * FA_D * 2;
   const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
@@ -133,8 +129,8 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
   bool seen = false;  // this lane's query has met a key it may see (decided on unscaled scores: the scale is the caller's)
 
   // the mask package says which stretch of keys the tile's queries may see at all: blocks [first_block, blocks)
-  const int keys = pipelink_call_mask_key_count(&view, q0, q0 + tile_queries - 1);
-  const int first_block = pipelink_call_mask_key_begin(&view, q0, q0 + tile_queries - 1) / FA_K_BLOCK;
+  const int keys = pipelink_call_mask_key_count(&view, q0, q0 + TILE_QUERIES - 1);
+  const int first_block = pipelink_call_mask_key_begin(&view, q0, q0 + TILE_QUERIES - 1) / FA_K_BLOCK;
   const int blocks = (keys + FA_K_BLOCK - 1) / FA_K_BLOCK;
   const int wave_keys = pipelink_call_mask_key_count(&view, qw, qw + 31), wave_begin = pipelink_call_mask_key_begin(&view, qw, qw + 31);
   // Schedule.  Two LDS buffers per operand: block i + 1 is in flight while block i is multiplied; one barrier per
@@ -327,6 +323,25 @@ extern "C" __device__ void fa_core_role_core(const void* params, unsigned varian
       *reinterpret_cast<v2i*>(orow + 32 * db + 8 * q4 + 4 * half) = __builtin_bit_cast(v2i, packed);
     }
 }
+}  // namespace fa_core
+
+extern "C" __device__ void fa_core_role_core(const void* params, unsigned variant) {
+  (void)variant;
+  using namespace fa_core;
+  const FaCoreParams& p = *static_cast<const FaCoreParams*>(params);
+  const pipelink_host_view view{params, nullptr};
+  const uint32_t tiles = (uint32_t)(p.batch * p.q_heads) * (uint32_t)(p.seq / TILE_QUERIES);
+  // The image a session is given beside its link may be of the other tile size than the link its grid was made for: whole
+  // tiles leave workgroups of a larger grid idle, half tiles take several of a smaller one.
+  uint32_t index = blockIdx.x;
+  if (index >= tiles) return;
+  for (;;) {
+    attend(p, view, index);
+    if (!split || tiles - index <= gridDim.x) break;
+    index += gridDim.x;
+    __syncthreads();  // nobody reads this tile's keys, values or partial sums any more
+  }
+}
 #else
 #include "include/fa_abi.h"
 #endif
@@ -354,5 +369,10 @@ PL_USES("pipelink_fa_kv");
 // two workgroups per CU (two waves per SIMD, 256 registers per lane each): one multiplies while the other
 // is in its softmax or waits at its barrier; 2 x 67.6 KB of LDS fit
 PL_FACT("launch.waves_per_simd", 2);
+#if FA_HALF_TILES
+PL_FACT("fa.core.tile_queries", 64);
+#else
+PL_FACT("fa.core.tile_queries", 128);
+#endif
 PL_PRELUDE("include/fa_abi.h");
 PL_EMIT_MAIN()

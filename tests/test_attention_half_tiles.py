@@ -37,3 +37,34 @@ def test_half_tiles_match_attention_in_64_bits(b, hq, hkv, s, window):
             want = score.softmax(-1) @ v[n, kv].double()
             # probabilities and result in bf16 (2^-9 each, relative): the bar the other attention tests use
             assert (got[n, :, head] - want).norm() / want.norm() <= 5e-3
+
+
+def test_an_image_of_the_other_tile_size_covers_the_whole_output():
+    """An image beside a link (a session's second one, or one the caller names) has the link's grid, not its own."""
+    from pathlib import Path
+
+    from pipelink_amd.host.attention import open_session
+    from pipelink_amd.stages.attention import build as fa_build
+
+    images = fa_build.images()
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (_bits(torch.randn(2, h, 640, 128, generator=g).to(torch.bfloat16)) for h in (4, 2, 2))
+
+    def run(sess):
+        sess.write("o", np.full((2, 640, 512), 0x7FC0, dtype=np.uint16))
+        sess.launch()
+        sess.synchronize()
+        return sess.read("o")
+
+    sess = open_session(images["link_json"], q, k, v)                                   # 40 tiles: half tiles
+    half = run(sess)
+    whole = run(sess.with_image(images["linked"]))
+    sess.close()
+    sess = open_session(images["link_json"], q, k, v, image=images["linked"])
+    assert np.array_equal(run(sess), whole) and np.array_equal(run(sess.with_image(images["half_linked"])), half)
+    sess.close()
+    for link, image in ((images["link_json"], images["half_linked"]), (Path(images["half_linked"]).parent / "link.json", None)):
+        sess = open_session(link, q, k, v, image=image)
+        assert np.array_equal(run(sess), half)
+        sess.close()
+    assert not np.array_equal(whole, half) and not (half == 0x7FC0).any() and not (whole == 0x7FC0).any()

@@ -83,3 +83,10 @@ def test_few_tiles_run_the_half_tile_link_made_for_their_link_and_no_other(built
     assert _open(link_json, window=7) == (relinked, 4)
     fa_build.link_half(cell)   # and the half tiles of the new link, once asked for
     assert _open(link_json, window=7) == ((cell / "half" / "link" / "pipeline.hsaco").read_bytes(), 8)
+
+
+def test_the_grid_is_of_the_tiles_of_the_link_that_is_opened(built):
+    half = built / "half" / "link" / "pipeline.hsaco"
+    assert _open(built / "half" / "link" / "link.json") == (half.read_bytes(), 8)
+    assert _open(built / "half" / "link" / "link.json", tiles=400) == (half.read_bytes(), 800)
+    assert _open(built / "half" / "link" / "link.json", image=half) == (half.read_bytes(), 8)
