@@ -32,7 +32,7 @@ def _half_of(link_json: str | Path) -> Path | None:
     return half / "link" / "link.json" if same else None
 
 
-def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, v_bits: np.ndarray, *, scale: float | None = None,
+def open_session(link_json: str | Path | dict, q_bits: np.ndarray, k_bits: np.ndarray, v_bits: np.ndarray, *, scale: float | None = None,
                  window: int | None = None, backend=None, image: str | Path | None = None) -> HostlessSession:
     """q_bits [B, Hq, S, 128], k_bits / v_bits [B, Hkv, S, 128]: bf16 bit patterns (uint16).  Buffers: q, k, v and
     o ([B, S, Hq * 128] uint16, zeroed).  `window`: for a link with fa.mask.window, the number of keys a query sees.
@@ -53,8 +53,10 @@ def open_session(link_json: str | Path, q_bits: np.ndarray, k_bits: np.ndarray, 
         raise ValueError("one head of K or V must stay below 2 GiB")
     tiles = b * hq * (s // Q_TILE)
     buffers = {"q": q_bits, "k": k_bits, "v": v_bits, "o": ((b, s, hq * d), np.uint16)}
-    half = _half_of(link_json) if tiles <= HALF_TILES_UP_TO and image is None else None   # (an image of the caller's own is run as it is)
-    facts = json.loads(Path(half or link_json).read_text()).get("facts", {})
-    grid = b * hq * (s // facts.get("fa.core.tile_queries", Q_TILE))
-    return open_hostless(half or link_json, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
+    # (an image of the caller's own, and a link handed over as an object, are run as they are)
+    whole = isinstance(link_json, dict) or image is not None or tiles > HALF_TILES_UP_TO
+    chosen = link_json if whole else _half_of(link_json) or link_json
+    link = chosen if isinstance(chosen, dict) else json.loads(Path(chosen).read_text())
+    grid = b * hq * (s // link.get("facts", {}).get("fa.core.tile_queries", Q_TILE))
+    return open_hostless(chosen, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
                          grid=(grid,), backend=backend, image=image)

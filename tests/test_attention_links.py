@@ -90,3 +90,9 @@ def test_the_grid_is_of_the_tiles_of_the_link_that_is_opened(built):
     assert _open(built / "half" / "link" / "link.json") == (half.read_bytes(), 8)
     assert _open(built / "half" / "link" / "link.json", tiles=400) == (half.read_bytes(), 800)
     assert _open(built / "half" / "link" / "link.json", image=half) == (half.read_bytes(), 8)
+
+
+def test_a_link_may_be_handed_over_as_an_object(built):
+    image = built / "link" / "pipeline.hsaco"
+    link = json.loads((built / "link" / "link.json").read_text())
+    assert _open(link, image=image) == (image.read_bytes(), 4) and _open(link, tiles=400, image=image) == (image.read_bytes(), 400)
