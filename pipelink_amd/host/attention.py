@@ -12,10 +12,29 @@ from ..stages.attention.params import params_blobs
 
 HEAD_DIM = 128
 Q_TILE = 128
-# A grid of at most this many tiles of 128 queries is launched as twice as many of 64 through the link made for that,
-# `half` beside it: us whole / half at 256 compute units: 256 tiles 25.7 / 22.3, 384 tiles 41.4 / 35.4, 480 tiles 54.3 / 54.2, 512 tiles
-# 57.6 / 61.4 and 24.8 / 28.8
+K_BLOCK = 64
+COMPUTE_UNITS = 256
 HALF_TILES_UP_TO = 384
+
+
+def _half_tiles_pay(heads: int, s: int, window: int | None) -> bool:
+    """Whether tiles of 64 queries, twice as many workgroups with a wave per half of each key block, take less time than tiles
+    of 128.  Half tiles shorten a tile's chain of key blocks, which is all a launch takes while compute units are left over;
+    they cost a start and a merge per workgroup, which short chains do not earn back, and loads twice once every compute unit
+    has two workgroups.  us half / us whole over 3700 random shapes (1 to 384 tiles, S 128 to 4096, causal and windows of 20
+    keys up; a launch against itself: 0.95 .. 1.05), by the longest chain L of a whole tile in blocks, the average A and the load F = tiles * A / (256 L):
+      up to 128 tiles    0.69 .. 0.98 whatever the chains
+      129 to 256 tiles   L 2: 1.2, L 4: 0.97 to 1.04, L 6: 0.97 (up to 1.16), L 8: 0.93 (up to 1.08); from L 10 on and F up to 0.78:
+                         0.79 .. 0.98, two shapes of 460 above 1 (1.01 and 1.03, L 10); beyond: up to 1.11
+      257 to 384 tiles   from L 12 on and F up to 0.78: 0.81 .. 0.98; beyond: up to 1.26; L 10: 0.9 to 1.13, L 7 and
+                         less: 1.03 to 1.37
+      512 tiles          1.07 (S 2048), 1.16 (S 512)"""
+    tiles = heads * (s // Q_TILE)
+    if tiles <= COMPUTE_UNITS // 2 or tiles > HALF_TILES_UP_TO:
+        return tiles <= COMPUTE_UNITS // 2
+    chains = [(q + Q_TILE) // K_BLOCK - (max(0, q - window + 1) // K_BLOCK if window else 0) for q in range(0, s, Q_TILE)]
+    longest = max(chains)
+    return longest >= (10 if tiles <= COMPUTE_UNITS else 12) and heads * sum(chains) <= 0.78 * COMPUTE_UNITS * longest
 
 
 def _half_of(link_json: str | Path) -> Path | None:
@@ -51,10 +70,9 @@ def open_session(link_json: str | Path | dict, q_bits: np.ndarray, k_bits: np.nd
         raise ValueError("operands are uint16 bf16 bit patterns")
     if s * d * 2 >= 1 << 31:
         raise ValueError("one head of K or V must stay below 2 GiB")
-    tiles = b * hq * (s // Q_TILE)
     buffers = {"q": q_bits, "k": k_bits, "v": v_bits, "o": ((b, s, hq * d), np.uint16)}
     # (an image of the caller's own, and a link handed over as an object, are run as they are)
-    whole = isinstance(link_json, dict) or image is not None or tiles > HALF_TILES_UP_TO
+    whole = isinstance(link_json, dict) or image is not None or not _half_tiles_pay(b * hq, s, window)
     chosen = link_json if whole else _half_of(link_json) or link_json
     link = chosen if isinstance(chosen, dict) else json.loads(Path(chosen).read_text())
     grid = b * hq * (s // link.get("facts", {}).get("fa.core.tile_queries", Q_TILE))

@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 # one and two query tiles; one block of keys and an odd number; windows that leave one half of the first block's keys
-# invisible to some queries, that are one key, that are longer than the sequence; the last grid that takes half tiles (384)
-# and the first that does not
+# invisible to some queries, that are one key, that are longer than the sequence; more tiles than a launch by itself would
+# run as half tiles
 @pytest.mark.parametrize("b,hq,hkv,s,window", [(1, 1, 1, 128, None), (2, 4, 2, 128, 1), (1, 4, 4, 256, 33), (1, 8, 2, 384, 97), (1, 4, 1, 640, None),
                                                (1, 2, 2, 512, 5000), (3, 32, 4, 512, None), (5, 7, 1, 1408, 200)])
 def test_half_tiles_match_attention_in_64_bits(b, hq, hkv, s, window):
@@ -19,8 +19,8 @@ def test_half_tiles_match_attention_in_64_bits(b, hq, hkv, s, window):
 
     g = torch.Generator().manual_seed(s + b)
     q, k, v = (torch.randn(b, h, s, 128, generator=g).to(torch.bfloat16) for h in (hq, hkv, hkv))
-    images = fa_build.images()
-    sess = open_session(images["window_link_json" if window else "link_json"], _bits(q), _bits(k), _bits(v), window=window)
+    link_json = fa_build.images()["window_half_linked" if window else "half_linked"].parent / "link.json"
+    sess = open_session(link_json, _bits(q), _bits(k), _bits(v), window=window)
     sess.write("o", np.full((b, s, hq * 128), 0x7FC0, dtype=np.uint16))
     sess.launch()
     sess.synchronize()

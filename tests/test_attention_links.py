@@ -96,3 +96,17 @@ def test_a_link_may_be_handed_over_as_an_object(built):
     image = built / "link" / "pipeline.hsaco"
     link = json.loads((built / "link" / "link.json").read_text())
     assert _open(link, image=image) == (image.read_bytes(), 4) and _open(link, tiles=400, image=image) == (image.read_bytes(), 400)
+
+
+# heads, S, window -> half tiles; the shapes that are not were measured slower with them (us half / whole in the comments)
+@pytest.mark.parametrize("heads,s,window,half", [
+    (128, 128, None, True), (192, 128, None, False), (32, 128 * 4, 64, True),                     # 0.96, 1.20, 0.79
+    (128, 256, None, False), (45, 384, None, False), (51, 640, None, True), (32, 1024, None, True),  # 1.02, 1.07, 0.91, 0.86
+    (28, 1152, 64, False), (32, 1152, 700, True), (35, 1152, 300, False), (42, 1152, 300, False),  # 1.05, 0.79, 1.15, 1.28
+    (128, 384, None, False), (96, 512, None, False), (80, 512, 64, False), (76, 640, None, False),  # 1.16, 1.11, 1.24, 1.04
+    (29, 1536, None, True), (12, 4096, None, True), (12, 4096, 300, False), (9, 3584, 942, False),  # 0.80, 0.79, 1.12, 1.11
+    (32, 2048, None, False), (1, 4096, 1, True)])                                                 # 1.07, 0.7
+def test_half_tiles_only_where_they_are_faster(heads, s, window, half):
+    from pipelink_amd.host.attention import _half_tiles_pay
+
+    assert _half_tiles_pay(heads, s, window) == half
