@@ -129,12 +129,12 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
   // exclusive prefix sums of rows and row tiles per expert (every workgroup computes its own copy)
   if (threadIdx.x < 64)
     tab.fill_by_wave(g.tokens_per_expert, ne, threadIdx.x, [](int v) { return wave_scan(v); },
-                     [](int v) { return __builtin_amdgcn_readlane(v, 63); }, [](bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; });
+                     [](int v) { return __builtin_amdgcn_readlane(v, 63); });
   __syncthreads();
 
   Schedule sched{g, tab, tab.tile_begin[ne], g.op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : g.num_col_tiles_gate_up,
                  g.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : g.num_col_tiles_down};
-  if (__builtin_amdgcn_readfirstlane((int)tab.last)) sched.cut();
+  sched.cut();
   const MokCounters counters{g.op == MOK_FWD_BOTH ? reinterpret_cast<int32_t*>(g.workspace + MOK_WS_COUNTERS) : nullptr,
                              g.workspace + MOK_WS_STATUS};
   uint32_t phase = 0;

@@ -49,7 +49,8 @@ MOK_SCHED_FN int count_by_wave(int n, Holds holds) {
 struct Tables {
   int row_begin[MAX_EXPERTS + 1];
   int tile_begin[MAX_EXPERTS + 1];
-  uint32_t last;   // at first: no expert has more than NARROW_ROWS rows; then: 1 + the list `claim` is of, or 0 if every list has been handed out; in the end: 1 in the workgroup
+  // (nothing here may be written by a workgroup that has no tile and read by it before: no barrier lies between)
+  uint32_t last;   // 1 + the list `claim` is of, or 0 if every list has been handed out; in the end: 1 in the workgroup
                    // that leaves the launch last
   uint32_t claim;  // what the list's queue answered this workgroup's last request
 
@@ -70,11 +71,9 @@ struct Tables {
   // inclusive sum over the lanes up to this one, `last_lane` lane 63's value.  fill() by one thread is a chain of `ne`
   // memory reads, one after the other, in front of everything else a launch does: a launch of one token and 32 experts
   // took 54.4 us with it and takes 53.2 us.
-  // `any` is true if its argument is in any lane.  Leaves in `last` whether every expert has at most NARROW_ROWS rows.
-  template <class Scan, class Last, class Any>
-  MOK_SCHED_FN void fill_by_wave(const int32_t* tokens_per_expert, int ne, int lane, Scan scan, Last last_lane, Any any) {
+  template <class Scan, class Last>
+  MOK_SCHED_FN void fill_by_wave(const int32_t* tokens_per_expert, int ne, int lane, Scan scan, Last last_lane) {
     int rows = 0, tiles = 0;
-    bool more = false;
     for (int e0 = 0; e0 < ne; e0 += 64) {
       const int e = e0 + lane;
       const int c = e < ne ? tokens_per_expert[e] : 0, t = (c + TILE_X - 1) / TILE_X;
@@ -85,10 +84,8 @@ struct Tables {
       }
       rows += last_lane(c_sum);
       tiles += last_lane(t_sum);
-      more = more || any(c > NARROW_ROWS);
     }
     if (lane == 0) {
-      last = more ? 0u : 1u;
       row_begin[ne] = rows;
       tile_begin[ne] = tiles;
     }
@@ -102,14 +99,15 @@ struct Schedule {
   int gate_up_cols, down_cols;  // column tiles of the GEMMs this launch runs (0: not run)
   int gate_up_cut = 0, down_cut = 0;  // a column tile is 2^cut tasks (one or four)
 
-  // Narrow tiles (for launches all of whose experts have at most NARROW_ROWS rows): a GEMM's column tiles are cut in four
-  // if the quarters still run at once.  More of them than that would take a second turn, whose start costs more than the
+  // Narrow tiles, for launches all of whose experts have at most NARROW_ROWS rows (every wave looks at the tables itself): a
+  // GEMM's column tiles are cut in four if the quarters still run at once.  More of them than that would take a second turn, whose start costs more than the
   // finer cut gives, us per forward: one token of 2880 x 2880, top 4 of 32, is 92 gate/up and 48 down tiles: 53.2 whole,
   // 44.2 with the down tiles cut, 49.4 with both (368 and 192 quarters); two tokens (184 and 96): 53.4 whole, 63.2 cut;
   // 1024 x 1536, top 2 of 16, one token: 31.1 whole, 21.6 cut.  (Halves as well, where quarters do not fit, are 39.7 for
   // the one token, but their code beside this costs every launch of whole small tiles 1 to 2 %.)
   // (From the numbers of both GEMMs whatever this launch runs: one launch and two give the same sums.)
   MOK_SCHED_FN void cut() {
+    if (MOK_SCHED_COUNT(g.num_experts, [&](int e) { return tab.row_begin[e + 1] - tab.row_begin[e] > NARROW_ROWS; }) != 0) return;
     down_cut = cut_of(row_tiles * g.num_col_tiles_down);
     // (the parts of a gate/up tile share cache lines of `hidden`, which only narrow down tiles read at device scope)
     gate_up_cut = down_cut ? cut_of(row_tiles * g.num_col_tiles_gate_up) : 0;

@@ -22,23 +22,24 @@ int main(int argc, char** argv) {
   std::vector<int32_t> counts;
   for (int a = 4; a < argc; ++a) counts.push_back(atoi(argv[a]));
   const int ne = (int)counts.size();
-  // the tables a wave's lanes make, by 64 lanes one after the other
+  // the tables a wave's lanes make: its 64 lanes one after the other, a scan from what the lanes handed in the pass before
   static Tables tab, want;
   want.fill(counts.data(), ne);
-  int lane_c[64], lane_t[64];
-  for (int pass = 0; pass < 2; ++pass)   // the second pass has every lane's scan at hand
+  tab.last = tab.claim = 0xA5u;   // the words the launch's end and the queues write are none of the tables'
+  std::vector<std::vector<int>> handed(2 * ((ne + 63) / 64), std::vector<int>(64, 0));
+  for (int pass = 0; pass < 2; ++pass)   // the second pass has every lane's numbers at hand
     for (int lane = 0; lane < 64; ++lane) {
-      int call = 0;
-      tab.fill_by_wave(counts.data(), ne < 64 ? ne : 64, lane,
-        [&](int v) { int* mine = call++ % 2 ? lane_t : lane_c; if (!pass) mine[lane] = v; int s = 0; for (int l = 0; l <= lane; ++l) s += mine[l]; return s; },
-        [&](int) { return 0; }, [&](bool) { bool more = false; for (int c : counts) more = more || c > NARROW_ROWS; return more; });
+      int scans = 0, totals = 0;
+      tab.fill_by_wave(counts.data(), ne, lane,
+        [&](int v) { auto& of = handed.at(scans++); if (!pass) of[lane] = v; int s = 0; for (int l = 0; l <= lane; ++l) s += of[l]; return s; },
+        [&](int) { int s = 0; for (int v : handed.at(totals++)) s += v; return s; });
     }
-  for (int e = 0; e < ne; ++e) if (tab.row_begin[e] != want.row_begin[e] || tab.tile_begin[e] != want.tile_begin[e]) { printf("table differs at %d\n", e); return 2; }
-  const int narrow = (int)tab.last;
+  for (int e = 0; e <= ne; ++e) if (tab.row_begin[e] != want.row_begin[e] || tab.tile_begin[e] != want.tile_begin[e]) { printf("table differs at %d\n", e); return 2; }
+  if (tab.last != 0xA5u || tab.claim != 0xA5u) { printf("the tables write the queues' words\n"); return 3; }
   const MokFrameworkParams g{counts.data(), nullptr, ne, op, gu, dn};
-  Schedule sched{g, want, want.tile_begin[ne], op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : gu, op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : dn};
-  if (narrow) sched.cut();
-  printf("%d %d %d\n", narrow, 1 << sched.gate_up_cut, 1 << sched.down_cut);
+  Schedule sched{g, tab, tab.tile_begin[ne], op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : gu, op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : dn};
+  sched.cut();
+  printf("%d %d\n", 1 << sched.gate_up_cut, 1 << sched.down_cut);
   for (int q = 0; q < NUM_XCD; ++q)
     for (int i = 0, cursor = 0; i < sched.length(q); ++i) {
       const MokGemmTask t = sched.decode(q, i, cursor);
@@ -98,8 +99,7 @@ def test_parts_cover_every_column_tile_once(tmp_path):
                                       (3, 23, 12, [1, 1], (4, 4)), (5, 23, 12, [1, 1, 1, 1], (1, 4)),
                                       (0, 2, 12, [5] * 22, (1, 1))]:   # whole down tiles: the gate/up tiles stay whole too
         out = subprocess.run([exe, str(op), str(gu), str(dn), *map(str, counts)], check=True, capture_output=True, text=True).stdout.splitlines()
-        narrow, *got = map(int, out[0].split())
-        assert narrow == (max(counts) <= 32) and tuple(got) == parts
+        assert tuple(map(int, out[0].split())) == parts
         want = set()
         for e, c in enumerate(counts):
             first = sum(counts[:e])
