@@ -163,6 +163,9 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
       if (!early) {
         if (!pipelink_call_gemm_ready(&view, &task, &counters)) pipelink_call_gemm_wait(&view, &task, &counters);
         pipelink_call_gemm_prefetch(&view, &task, &carry);
+        // The mainloop stages the next task where this one's tokens and counter are, and no wave may do that before every
+        // wave has read them.  (A tile whose prefetch was early has its predecessor's epilogue and barriers in between.)
+        mok::lds_barrier();
       }
       if (i >= 0) {  // the first tile's loads are on their way: the second turn
         if (i + turn < items) next = sched.decode(q, i + turn, cursor);
