@@ -4,9 +4,11 @@
 #ifndef PLK_MOK_RESIDUES_HPP
 #define PLK_MOK_RESIDUES_HPP
 
+#include <algorithm>
 #include <cstdint>
 #include <vector>
 
+#include "../stages/mok/framework/cut.hpp"
 #include "../stages/mok/include/mok_abi.h"
 
 namespace plk_mok {
@@ -115,11 +117,20 @@ inline MokFrameworkParams framework_params(const Dims& d, uint64_t tokens_per_ex
 }
 
 // an upper bound of the number of tiles of the launch: more workgroups than this would idle, and cost the others time when
-// they start and leave (a layer of 448 x 704 with 509 tokens: 38 us with 72 workgroups, 41 with 256).  A launch none of
-// whose experts has more than 32 rows may cut its column tiles into four.
+// they start and leave (a layer of 448 x 704 with 509 tokens: 38 us with 72 workgroups, 41 with 256).  A launch that may cut
+// its column tiles in four (mok_framework::cut_for) is bounded by its parts: every expert with rows is one row tile then, and
+// holds 32 rows at most.
 inline int64_t max_workgroups(const Dims& d) {
-  const int parts = d.routed_rows <= 32 * (int64_t)d.experts ? 4 : 1;
-  return parts * max_row_tiles(d) * ((d.pass != 2 ? num_col_tiles_gate_up(d) : 0) + (d.pass != 1 ? num_col_tiles_down(d) : 0));
+  const int gu = num_col_tiles_gate_up(d), down = num_col_tiles_down(d);
+  auto launched = [&](int64_t row_tiles, mok_framework::Cut cut) {
+    return row_tiles * ((d.pass != 2 ? gu << cut.gate_up : 0) + (d.pass != 1 ? down << cut.down : 0));
+  };
+  int64_t most = launched(max_row_tiles(d), {0, 0});
+  for (int t = (d.routed_rows + mok_framework::NARROW_ROWS - 1) / mok_framework::NARROW_ROWS; t <= d.experts && t <= d.routed_rows; ++t) {
+    const mok_framework::Cut cut = mok_framework::cut_for(d.routed_rows, d.experts, t, gu, down);
+    most = std::max(most, launched(t, cut));
+  }
+  return most;
 }
 
 }  // namespace plk_mok

@@ -8,6 +8,7 @@
 #define PIPELINK_MOK_FRAMEWORK_SCHEDULE_HPP
 #include <stdint.h>
 #include "../include/mok_abi.h"
+#include "cut.hpp"
 
 #ifndef MOK_SCHED_FN
 #define MOK_SCHED_FN __device__ __forceinline__
@@ -24,8 +25,6 @@ constexpr int MAX_EXPERTS = 256;
 constexpr int NUM_XCD = 8;       // lists
 constexpr int TILE_X = 256;      // routed rows of a tile   (the GEMM owner's published facts; the stage source
 constexpr int TILE_W = 256;      // weight rows of a tile    checks them against the owner's header)
-constexpr int NARROW_ROWS = 32;  // routed rows a quarter of a column tile (MOK_TASK_QUARTER) holds at most
-constexpr int CHIP = 256;        // workgroups that run at once (one per compute unit)
 
 // how many of the first n numbers a condition holds for: one after the other; by a wave (all of its lanes take part and get
 // the answer), where the reads behind the condition are 64 at a time instead of a chain of LDS latencies
@@ -99,20 +98,15 @@ struct Schedule {
   int gate_up_cols, down_cols;  // column tiles of the GEMMs this launch runs (0: not run)
   int gate_up_cut = 0, down_cut = 0;  // a column tile is 2^cut tasks (one or four)
 
-  // Narrow tiles, for launches all of whose experts have at most NARROW_ROWS rows (every wave looks at the tables itself): a
-  // GEMM's column tiles are cut in four if the quarters still run at once.  More of them than that would take a second turn, whose start costs more than the
-  // finer cut gives, us per forward: one token of 2880 x 2880, top 4 of 32, is 92 gate/up and 48 down tiles: 53.2 whole,
-  // 44.2 with the down tiles cut, 49.4 with both (368 and 192 quarters); two tokens (184 and 96): 53.4 whole, 63.2 cut;
-  // 1024 x 1536, top 2 of 16, one token: 31.1 whole, 21.6 cut.  (Halves as well, where quarters do not fit, are 39.7 for
-  // the one token, but their code beside this costs every launch of whole small tiles 1 to 2 %.)
-  // (From the numbers of both GEMMs whatever this launch runs: one launch and two give the same sums.)
+  // Narrow tiles, for launches all of whose experts have at most NARROW_ROWS rows (every wave looks at the tables itself):
+  // cut_for says whose column tiles are cut in four.
   MOK_SCHED_FN void cut() {
+    const Cut c = cut_for(tab.row_begin[g.num_experts], g.num_experts, row_tiles, g.num_col_tiles_gate_up, g.num_col_tiles_down);
+    if (c.down == 0) return;
     if (MOK_SCHED_COUNT(g.num_experts, [&](int e) { return tab.row_begin[e + 1] - tab.row_begin[e] > NARROW_ROWS; }) != 0) return;
-    down_cut = cut_of(row_tiles * g.num_col_tiles_down);
-    // (the parts of a gate/up tile share cache lines of `hidden`, which only narrow down tiles read at device scope)
-    gate_up_cut = down_cut ? cut_of(row_tiles * g.num_col_tiles_gate_up) : 0;
+    down_cut = c.down;
+    gate_up_cut = c.gate_up;
   }
-  MOK_SCHED_FN static int cut_of(int tiles) { return 4 * tiles <= CHIP ? 2 : 0; }
   MOK_SCHED_FN int gate_up_items() const { return row_tiles * gate_up_cols << gate_up_cut; }
   MOK_SCHED_FN int down_items() const { return row_tiles * down_cols << down_cut; }
 

@@ -95,9 +95,13 @@ def test_narrow_waves_share_the_slots_and_count_their_loads(tmp_path):
 def test_parts_cover_every_column_tile_once(tmp_path):
     exe = _compile(tmp_path, SCHEDULE)
     for op, gu, dn, counts, parts in [(0, 23, 12, [0, 1, 0, 1, 1, 1] + [0] * 26, (1, 4)), (0, 23, 12, [1] * 8 + [0] * 24, (1, 1)),
-                                      (0, 23, 12, [1] * 11, (1, 1)), (0, 6, 2, [32, 1, 0, 7], (4, 4)), (0, 6, 2, [33, 1, 0, 7], (1, 1)),
+                                      (0, 23, 12, [1] * 11, (1, 1)), (0, 6, 4, [32, 1, 0, 7], (4, 4)), (0, 6, 4, [33, 1, 0, 7], (1, 1)),
+                                      (0, 6, 2, [32, 1, 0, 7], (1, 4)),   # 5 slots of gate/up contraction for 96 tasks
                                       (3, 23, 12, [1, 1], (4, 4)), (5, 23, 12, [1, 1, 1, 1], (1, 4)),
-                                      (0, 2, 12, [5] * 22, (1, 1))]:   # whole down tiles: the gate/up tiles stay whole too
+                                      (0, 2, 12, [5] * 22, (1, 1)),   # whole down tiles: the gate/up tiles stay whole too
+                                      # layers where quarters were measured slower (us cut / whole 1.2, 1.4, 1.06, 1.05)
+                                      (0, 2, 1, [1] * 28 + [0] * 4, (1, 1)), (0, 1, 2, [12, 13] * 16, (1, 1)),
+                                      (0, 2, 1, [2, 3] * 4, (1, 1)), (0, 6, 2, [27, 28] * 4, (1, 1))]:
         out = subprocess.run([exe, str(op), str(gu), str(dn), *map(str, counts)], check=True, capture_output=True, text=True).stdout.splitlines()
         assert tuple(map(int, out[0].split())) == parts
         want = set()
@@ -111,12 +115,56 @@ def test_parts_cover_every_column_tile_once(tmp_path):
         assert len(items) == len(want) and set(items) == want
 
 
+GRID = r"""
+#define MOK_SCHED_FN inline
+#define MOK_SCHED_UNIFORM(x) (x)
+#include "framework/schedule.hpp"
+#include "../../csrc/plk_mok_residues.hpp"
+#include <cstdio>
+#include <random>
+using namespace mok_framework;
+int main() {
+  std::mt19937 rng(1);
+  auto upto = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
+  for (int it = 0; it < 200000; ++it) {
+    plk_mok::Dims d;
+    d.hidden = 64 * upto(1, 48), d.intermediate = 64 * upto(1, 48), d.experts = upto(1, 64), d.pass = upto(0, 2);
+    std::vector<int32_t> counts(d.experts);
+    const int most = upto(0, 40);
+    for (auto& c : counts) { c = rng() % 2 ? upto(0, most) : 0; d.routed_rows += c; }
+    if (!d.routed_rows) continue;
+    Tables tab;
+    tab.fill(counts.data(), d.experts);
+    const MokFrameworkParams g = plk_mok::framework_params(d, (uint64_t)(uintptr_t)counts.data(), 0);
+    Schedule sched{g, tab, tab.tile_begin[d.experts], d.pass == 2 ? 0 : g.num_col_tiles_gate_up, d.pass == 1 ? 0 : g.num_col_tiles_down};
+    sched.cut();
+    const long long tasks = sched.gate_up_items() + sched.down_items();
+    if (tasks > plk_mok::max_workgroups(d)) { printf("%lld tasks, %lld workgroups\n", tasks, (long long)plk_mok::max_workgroups(d)); return 1; }
+  }
+  // a layer of 448 x 704, top 2 of 8: nothing is cut from 65 tokens on, and the grid has no room for it
+  for (int tokens : {4, 64, 65, 110, 128, 129}) {
+    plk_mok::Dims d;
+    d.hidden = 448, d.intermediate = 704, d.experts = 8, d.routed_rows = 2 * tokens;
+    printf("%d\n", (int)plk_mok::max_workgroups(d));
+  }
+}
+"""
+
+
+def test_the_grid_has_room_for_the_tasks_and_for_quarters_only_where_they_may_be(tmp_path):
+    res = subprocess.run([_compile(tmp_path, GRID)], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
+    assert list(map(int, res.stdout.split())) == [112, 112, 72, 72, 72, 80]
+
+
 # one to 32 rows an expert (33: whole tiles); a contraction of one slot, fewer pairs than waves, an odd number of slots, one
-# more pair than a ring; columns that end inside a column tile; gate/up and down tiles cut, down tiles only, none; rows of whole cache lines (one launch) or not
+# more pair than a ring; columns that end inside a column tile; gate/up and down tiles cut, down tiles only, none; rows of whole
+# cache lines (one launch) or not; from `(448, 256` on: quarters of the shortest contractions that are cut
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,I,counts", [(64, 64, [1]), (128, 320, [32, 0, 5]), (576, 192, [31, 17, 1, 32]), (704, 1088, [2] * 5),
                                         (2880, 2880, [1, 0, 1, 1, 1]), (2880, 2880, [3, 2, 1, 1, 32, 9, 1]), (1536, 2048, [4] * 7),
-                                        (448, 704, [33, 2, 1]), (320, 128, [20] * 8)])
+                                        (448, 704, [33, 2, 1]), (320, 128, [20] * 8),
+                                        (448, 256, [16]), (512, 192, [5]), (320, 192, [7]), (576, 384, [9, 0, 31, 1]), (1088, 448, [31, 1]), (1536, 64, [3])])
 def test_forward_of_few_rows_matches_the_oracle(H, I, counts):
     from oracle import moe_ffn
     from pipelink_amd.host import mok_inputs
