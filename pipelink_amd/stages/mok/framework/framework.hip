@@ -113,30 +113,16 @@ __device__ __attribute__((noinline)) SmallTileResult small_tile(const void* para
   return SmallTileResult{carry, early ? 1 : 0, answer};
 }
 
-}  // namespace mok_framework
 
-extern "C" __device__ void mok_framework_worker(const void* params, unsigned variant) {
-  (void)variant;
-  using namespace mok_framework;
+// The workgroup's tiles.  PARTS: a launch whose column tiles are cut, all of whose tiles are small ones; without it no task is
+// a part, and the compiler leaves out what parts need.  One loop for both costs launches without parts 0.2 to 0.7 us (the
+// parts' code between the others' and three times the scalar spills): 448 x 704, 160 tokens 20.4 / 20.7 us, 256 x 2048, 250
+// tokens 28.6 / 29.7, 27 tokens of 2880 x 2880 163.9 / 165.5.
+template <bool PARTS>
+__device__ __forceinline__ void run_tiles(const void* params, const MokFrameworkParams& g, Tables& tab, Schedule sched,
+                                          const MokCounters& counters) {
   const pipelink_host_view view{params, nullptr};
-  const MokFrameworkParams& g = *static_cast<const MokFrameworkParams*>(params);
-  Tables& tab = *reinterpret_cast<Tables*>(pipelink_smem + pipelink_mok_fw_sched());
-  const int ne = g.num_experts;
-
-  pipelink_call_gemm_init(&view);
-  pipelink_call_act_init(&view);
-
-  // exclusive prefix sums of rows and row tiles per expert (every workgroup computes its own copy)
-  if (threadIdx.x < 64)
-    tab.fill_by_wave(g.tokens_per_expert, ne, threadIdx.x, [](int v) { return wave_scan(v); },
-                     [](int v) { return __builtin_amdgcn_readlane(v, 63); });
-  __syncthreads();
-
-  Schedule sched{g, tab, tab.tile_begin[ne], g.op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : g.num_col_tiles_gate_up,
-                 g.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : g.num_col_tiles_down};
-  sched.cut();
-  const MokCounters counters{g.op == MOK_FWD_BOTH ? reinterpret_cast<int32_t*>(g.workspace + MOK_WS_COUNTERS) : nullptr,
-                             g.workspace + MOK_WS_STATUS};
+  if (!PARTS) sched.gate_up_cut = sched.down_cut = 0;
   uint32_t phase = 0;
 
   const int q = blockIdx.x % NUM_XCD;
@@ -175,7 +161,7 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
       const bool has_next = next.op != 0;
       const bool asks = has_next && asking;
       uint32_t answer = 0;
-      if (pipelink_call_gemm_placement(&view, &task) != mok::TILE_FULL) {
+      if (PARTS || pipelink_call_gemm_placement(&view, &task) != mok::TILE_FULL) {
         const SmallTileResult res = small_tile(params, task, next, counters.base, counters.status, asks ? g.workspace + MOK_WS_QUEUE + list : nullptr, carry);
         carry = res.carry;
         early = __builtin_amdgcn_readfirstlane(res.early) != 0;
@@ -190,11 +176,7 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
         // The next tile's first loads fly while this tile's epilogue computes -- unless its rows are not complete yet:
         // then this tile is finished (and counted) first, so that nobody waits for a workgroup that waits.
         early = has_next && pipelink_call_gemm_ready(&view, &next, &counters);
-        if (early) {
-          MokGemmTask whole = next;
-          whole.flags = 0u;  // (a launch with full tiles cuts none: the code for parts is not needed here)
-          pipelink_call_gemm_prefetch(&view, &whole, &carry);
-        }
+        if (early) pipelink_call_gemm_prefetch(&view, &next, &carry);
         if (task.op == MOK_GEMM_FWD_ROUTED_GATE_UP) {
           const MokActTask act{MOK_ACT_FWD_ROUTED, task.row_begin, task.row_end, task.col_begin, task.task_idx, task.counter_idx, task.flags};
           pipelink_call_act_fwd(&view, &act, &counters, &phase, &acc);
@@ -248,6 +230,34 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
       next = after;
     }
   }
+}
+
+}  // namespace mok_framework
+
+extern "C" __device__ void mok_framework_worker(const void* params, unsigned variant) {
+  (void)variant;
+  using namespace mok_framework;
+  const pipelink_host_view view{params, nullptr};
+  const MokFrameworkParams& g = *static_cast<const MokFrameworkParams*>(params);
+  Tables& tab = *reinterpret_cast<Tables*>(pipelink_smem + pipelink_mok_fw_sched());
+  const int ne = g.num_experts;
+
+  pipelink_call_gemm_init(&view);
+  pipelink_call_act_init(&view);
+
+  // exclusive prefix sums of rows and row tiles per expert (every workgroup computes its own copy)
+  if (threadIdx.x < 64)
+    tab.fill_by_wave(g.tokens_per_expert, ne, threadIdx.x, [](int v) { return wave_scan(v); },
+                     [](int v) { return __builtin_amdgcn_readlane(v, 63); });
+  __syncthreads();
+
+  Schedule sched{g, tab, tab.tile_begin[ne], g.op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : g.num_col_tiles_gate_up,
+                 g.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : g.num_col_tiles_down};
+  sched.cut();
+  const MokCounters counters{g.op == MOK_FWD_BOTH ? reinterpret_cast<int32_t*>(g.workspace + MOK_WS_COUNTERS) : nullptr,
+                             g.workspace + MOK_WS_STATUS};
+  if (sched.down_cut) run_tiles<true>(params, g, tab, sched, counters);
+  else run_tiles<false>(params, g, tab, sched, counters);
   pipelink_call_gemm_fini(&view);
 
   // The last workgroup to leave puts the queues and the counters back to zero for the next launch: by then nobody
@@ -259,7 +269,7 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
   __syncthreads();
   if (tab.last) {
     if (g.op == MOK_FWD_BOTH)
-      for (int w = threadIdx.x; w < sched.row_tiles; w += blockDim.x)
+      for (int w = threadIdx.x; w < sched.row_tiles; w += mok::THREADS)
         __hip_atomic_store(g.workspace + MOK_WS_COUNTERS + w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (threadIdx.x < NUM_XCD) __hip_atomic_store(g.workspace + MOK_WS_QUEUE + threadIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (threadIdx.x == 0) {

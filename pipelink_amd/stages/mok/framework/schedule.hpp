@@ -102,10 +102,10 @@ struct Schedule {
   // cut_for says whose column tiles are cut in four.
   MOK_SCHED_FN void cut() {
     const Cut c = cut_for(tab.row_begin[g.num_experts], g.num_experts, row_tiles, g.num_col_tiles_gate_up, g.num_col_tiles_down);
-    if (c.down == 0) return;
+    if (MOK_SCHED_UNIFORM(c.down) == 0) return;
     if (MOK_SCHED_COUNT(g.num_experts, [&](int e) { return tab.row_begin[e + 1] - tab.row_begin[e] > NARROW_ROWS; }) != 0) return;
-    down_cut = c.down;
-    gate_up_cut = c.gate_up;
+    down_cut = MOK_SCHED_UNIFORM(c.down);
+    gate_up_cut = MOK_SCHED_UNIFORM(c.gate_up);
   }
   MOK_SCHED_FN int gate_up_items() const { return row_tiles * gate_up_cols << gate_up_cut; }
   MOK_SCHED_FN int down_items() const { return row_tiles * down_cols << down_cut; }

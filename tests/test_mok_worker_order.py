@@ -62,7 +62,7 @@ void pipelink_call_gemm_store(const void*, const MokGemmTask*, const mok::AccFra
 void pipelink_call_gemm_store_small(const void*, const MokGemmTask*, const mok::AccFrag*) {}
 void pipelink_call_act_fwd(const void*, const MokActTask*, const MokCounters*, uint32_t*, const mok::AccFrag*) {}
 void pipelink_call_act_fwd_small(const void*, const MokActTask*, const MokCounters*, uint32_t*, const mok::AccFrag*) {}
-int pipelink_call_gemm_placement(const void*, const MokGemmTask* t) { return mok::tile_placement(t->row_end - t->row_begin, 1 << 20, t->flags); }
+int pipelink_call_gemm_placement(const void*, const MokGemmTask* t) { puts("placement"); return mok::tile_placement(t->row_end - t->row_begin, 1 << 20, t->flags); }
 }
 int main(int argc, char** argv) {
   const int rows = atoi(argv[1]), gu = atoi(argv[2]), dn = atoi(argv[3]), workgroups = atoi(argv[4]);
@@ -112,6 +112,9 @@ def test_a_barrier_lies_between_staging_a_task_and_reading_it_and_back(trace, ro
     cut = [4 if rows <= 32 and 4 * n <= 256 else 1 for n in (gu, dn)]
     if cut[1] == 1:
         cut[0] = 1
+    # launches with parts and launches without have a loop each: only the one without looks whether a tile is a full one
+    assert ("placement" in events) == (cut[1] == 1)
+    events = [e for e in events if e != "placement"]
     assert tiles == f"tiles {-(-rows // 256) * (gu * cut[0] + dn * cut[1])}"   # every tile has been run
     since = set()   # what has happened to the staged area since the last barrier
     for n, event in enumerate(events):
