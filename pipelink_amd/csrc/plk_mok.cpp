@@ -453,10 +453,12 @@ extern "C" int plk_mxfp8_quantize_zero_pad(uint64_t src, int src_is_bf16, int64_
 // ---- weight code layout conversion: row-major [rows, ld_q] -> K-tiled [K/64, rows, 64], expert by expert ------
 // A permutation of 64-byte pieces, so its cost is memory traffic: a workgroup takes two neighbouring 64-byte columns of
 // LAYOUT_ROWS rows, so that every row is read 128 bytes at a time (one column at a time asks for each cache line twice,
-// far apart) and written 512 contiguous bytes per wave and column; a lane has LAYOUT_ROWS / 32 loads in flight.  All
-// experts in one launch: 32 experts of 2880 x 2880 take 106 us (5.0 TB/s, what a plain copy reaches); one column at a time,
-// a launch per expert, was 32 x 5.5 us and the gaps between them.
-constexpr int LAYOUT_ROWS = 128;
+// far apart) and written 512 contiguous bytes per wave and column.  A lane has LAYOUT_ROWS / 32 loads in flight: rows past the
+// last are the last once more, because a load or a store under a condition of its own makes the compiler wait for each load
+// before the next one.  All experts in one launch.
+// us: 32 experts of 2880 x 2880 97 (5.5 TB/s) with 64 rows, 97 with 32 and 128, 105 with 256; one expert of 2880 x 2880 3.9
+// (with 128 rows and loads under conditions 108 and 17.6; one column at a time, a launch per expert, 32 x 5.6 and 5.6).
+constexpr int LAYOUT_ROWS = 64;
 __global__ void __launch_bounds__(256) codes_to_k64_tiled_kernel(const uint8_t* __restrict__ src, int experts, int64_t rows, int ktiles,
                                                                   int64_t ld_q, uint8_t* __restrict__ dst) {
   const int lane8 = threadIdx.x & 7, c = lane8 & 3;  // a row's 128 bytes: eight lanes, four per column
@@ -468,12 +470,14 @@ __global__ void __launch_bounds__(256) codes_to_k64_tiled_kernel(const uint8_t* 
       const uint8_t* const from = src + e * rows * ld_q + kt * 64 + c * 16;
       uint8_t* const to = dst + (e * ktiles + kt) * rows * 64 + c * 16;
       uint4 v[LAYOUT_ROWS / 32];
+      int64_t row[LAYOUT_ROWS / 32];
 #pragma unroll
-      for (int u = 0; u < LAYOUT_ROWS / 32; ++u)
-        if (row0 + 32 * u < rows) v[u] = *reinterpret_cast<const uint4*>(from + (row0 + 32 * u) * ld_q);
+      for (int u = 0; u < LAYOUT_ROWS / 32; ++u) {
+        row[u] = row0 + 32 * u < rows ? row0 + 32 * u : rows - 1;
+        v[u] = *reinterpret_cast<const uint4*>(from + row[u] * ld_q);
+      }
 #pragma unroll
-      for (int u = 0; u < LAYOUT_ROWS / 32; ++u)
-        if (row0 + 32 * u < rows) *reinterpret_cast<uint4*>(to + (row0 + 32 * u) * 64) = v[u];
+      for (int u = 0; u < LAYOUT_ROWS / 32; ++u) *reinterpret_cast<uint4*>(to + row[u] * 64) = v[u];
     }
   }
 }
