@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -450,6 +451,11 @@ extern "C" int plk_mxfp8_quantize_zero_pad(uint64_t src, int src_is_bf16, int64_
   return quantize(src, src_is_bf16, rows, k, dst_q, ld_q, dst_sc, ld_sc, 1, stream);
 }
 
+// Workgroups that take `per` rows each.  A launch holds fewer than 2^32 threads: at most this many, the rows behind them are
+// further turns (code layout) or launches (scale layout, whose kernel a loop over rows slows down: 6.3 us / 7.3 us).
+constexpr int64_t MOST_ROW_GROUPS = 1 << 20;
+static unsigned row_groups(int64_t rows, int per) { return (unsigned)std::min((rows + per - 1) / per, MOST_ROW_GROUPS); }
+
 // ---- weight code layout conversion: row-major [rows, ld_q] -> K-tiled [K/64, rows, 64], expert by expert ------
 // A permutation of 64-byte pieces, so its cost is memory traffic: a workgroup takes two neighbouring 64-byte columns of
 // LAYOUT_ROWS rows, so that every row is read 128 bytes at a time (one column at a time asks for each cache line twice,
@@ -462,22 +468,24 @@ constexpr int LAYOUT_ROWS = 64;
 __global__ void __launch_bounds__(256) codes_to_k64_tiled_kernel(const uint8_t* __restrict__ src, int experts, int64_t rows, int ktiles,
                                                                   int64_t ld_q, uint8_t* __restrict__ dst) {
   const int lane8 = threadIdx.x & 7, c = lane8 & 3;  // a row's 128 bytes: eight lanes, four per column
-  const int64_t row0 = (int64_t)blockIdx.x * LAYOUT_ROWS + (threadIdx.x >> 3);
   for (int64_t e = blockIdx.z; e < experts; e += gridDim.z) {
     for (int64_t pair = blockIdx.y; 2 * pair < ktiles; pair += gridDim.y) {
       const int64_t kt = 2 * pair + (lane8 >> 2);
       if (kt >= ktiles) continue;
       const uint8_t* const from = src + e * rows * ld_q + kt * 64 + c * 16;
       uint8_t* const to = dst + (e * ktiles + kt) * rows * 64 + c * 16;
-      uint4 v[LAYOUT_ROWS / 32];
-      int64_t row[LAYOUT_ROWS / 32];
+      for (int64_t first = (int64_t)blockIdx.x * LAYOUT_ROWS; first < rows; first += (int64_t)gridDim.x * LAYOUT_ROWS) {
+        uint4 v[LAYOUT_ROWS / 32];
+        int64_t row[LAYOUT_ROWS / 32];
 #pragma unroll
-      for (int u = 0; u < LAYOUT_ROWS / 32; ++u) {
-        row[u] = row0 + 32 * u < rows ? row0 + 32 * u : rows - 1;
-        v[u] = *reinterpret_cast<const uint4*>(from + row[u] * ld_q);
+        for (int u = 0; u < LAYOUT_ROWS / 32; ++u) {
+          const int64_t r = first + 32 * u + (threadIdx.x >> 3);
+          row[u] = r < rows ? r : rows - 1;
+          v[u] = *reinterpret_cast<const uint4*>(from + row[u] * ld_q);
+        }
+#pragma unroll
+        for (int u = 0; u < LAYOUT_ROWS / 32; ++u) *reinterpret_cast<uint4*>(to + row[u] * 64) = v[u];
       }
-#pragma unroll
-      for (int u = 0; u < LAYOUT_ROWS / 32; ++u) *reinterpret_cast<uint4*>(to + row[u] * 64) = v[u];
     }
   }
 }
@@ -489,7 +497,7 @@ extern "C" int plk_mxfp8_codes_to_k64_tiled_experts(uint64_t src, int32_t expert
   if (rows == 0 || experts == 0) return PLK_OK;
   if (!src || !dst) return plk_hip_set_error(PLK_E_ARGUMENT, "plk_mxfp8_codes_to_k64_tiled: null device address");
   const int ktiles = k / 64, pairs = (ktiles + 1) / 2;
-  const dim3 grid((unsigned)((rows + LAYOUT_ROWS - 1) / LAYOUT_ROWS), (unsigned)(pairs < 65535 ? pairs : 65535),
+  const dim3 grid(row_groups(rows, LAYOUT_ROWS), (unsigned)(pairs < 65535 ? pairs : 65535),
                   (unsigned)(experts < 65535 ? experts : 65535));
   codes_to_k64_tiled_kernel<<<grid, dim3(256), 0, (hipStream_t)stream>>>((const uint8_t*)(uintptr_t)src, experts, rows, ktiles, ld_q,
                                                                         (uint8_t*)(uintptr_t)dst);
@@ -507,10 +515,10 @@ extern "C" int plk_mxfp8_codes_to_k64_tiled(uint64_t src, int64_t rows, int32_t 
 // written contiguously.  Rows whose bytes are whole dwords (`words`) are read so, others byte by byte.  32 experts of
 // 2880 x 2880: 10 us, 32 x 3.0 us before as a launch per expert and byte loads a row pitch apart.
 constexpr int SCALE_ROWS = 64, SCALE_SLOTS = 32;
-__global__ void __launch_bounds__(256) scales_to_slot_major_kernel(const uint8_t* __restrict__ src, int experts, int64_t rows, int nblocks,
+__global__ void __launch_bounds__(256) scales_to_slot_major_kernel(const uint8_t* __restrict__ src, int experts, int64_t first_row, int64_t rows, int nblocks,
                                                                     int ld_sc, uint32_t* __restrict__ dst, int nslots, int words) {
   __shared__ uint32_t tile[SCALE_ROWS][SCALE_SLOTS + 1];
-  const int64_t row0 = (int64_t)blockIdx.x * SCALE_ROWS;
+  const int64_t row0 = first_row + (int64_t)blockIdx.x * SCALE_ROWS;
   for (int64_t e = blockIdx.z; e < experts; e += gridDim.z) {
     for (int s0 = blockIdx.y * SCALE_SLOTS; s0 < nslots; s0 += gridDim.y * SCALE_SLOTS) {
       const int s = s0 + (threadIdx.x & (SCALE_SLOTS - 1));
@@ -548,10 +556,11 @@ extern "C" int plk_mxfp8_scales_to_slot_major_experts(uint64_t src, int32_t expe
   if (!src || !dst) return plk_hip_set_error(PLK_E_ARGUMENT, "plk_mxfp8_scales_to_slot_major: null device address");
   const int nslots = (k + 127) / 128, groups = (nslots + SCALE_SLOTS - 1) / SCALE_SLOTS;
   const int words = src % 4 == 0 && ld_sc % 4 == 0;
-  const dim3 grid((unsigned)((rows + SCALE_ROWS - 1) / SCALE_ROWS), (unsigned)(groups < 65535 ? groups : 65535),
-                  (unsigned)(experts < 65535 ? experts : 65535));
-  scales_to_slot_major_kernel<<<grid, dim3(256), 0, (hipStream_t)stream>>>((const uint8_t*)(uintptr_t)src, experts, rows, k / 32, ld_sc,
-                                                                          (uint32_t*)(uintptr_t)dst, nslots, words);
+  for (int64_t first = 0; first < rows; first += MOST_ROW_GROUPS * SCALE_ROWS) {
+    const dim3 grid(row_groups(rows - first, SCALE_ROWS), (unsigned)(groups < 65535 ? groups : 65535), (unsigned)(experts < 65535 ? experts : 65535));
+    scales_to_slot_major_kernel<<<grid, dim3(256), 0, (hipStream_t)stream>>>((const uint8_t*)(uintptr_t)src, experts, first, rows, k / 32, ld_sc,
+                                                                            (uint32_t*)(uintptr_t)dst, nslots, words);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return plk_hip_set_error(PLK_E_RESOURCE, hipGetErrorString(e));
   return PLK_OK;

@@ -69,3 +69,14 @@ def test_quantiser_of_the_plain_entry_leaves_the_pad_alone():
     oq, osc = mxfp8.mx_quantize(x.cpu().numpy())
     assert np.array_equal(q[:, :96].cpu().numpy(), oq) and bool((q[:, 96:] == 0xA5).all())
     assert np.array_equal(sc.cpu().numpy(), osc[:, :3])
+
+
+def test_scale_layout_of_more_rows_than_one_launch_has_threads_for():
+    """2^30 rows and a few: four threads a row are 2^32 (1 GB of scale bytes, 4 GB of dwords)."""
+    from pipelink_amd.host.mok import weight_scales_to_slot_major
+
+    n = (1 << 30) + 65
+    sc = torch.randint(0, 256, (1, n, 1), dtype=torch.uint8, device="cuda")
+    got = weight_scales_to_slot_major(sc, 32).view(n, 4)
+    for first in range(0, n, 1 << 28):
+        assert torch.equal(got[first:first + (1 << 28), 0], sc[0, first:first + (1 << 28), 0]) and not got[first:first + (1 << 28), 1:].any()
