@@ -101,7 +101,12 @@ def test_parts_cover_every_column_tile_once(tmp_path):
                                       (0, 2, 12, [5] * 22, (1, 1)),   # whole down tiles: the gate/up tiles stay whole too
                                       # layers where quarters were measured slower (us cut / whole 1.2, 1.4, 1.06, 1.05)
                                       (0, 2, 1, [1] * 28 + [0] * 4, (1, 1)), (0, 1, 2, [12, 13] * 16, (1, 1)),
-                                      (0, 2, 1, [2, 3] * 4, (1, 1)), (0, 6, 2, [27, 28] * 4, (1, 1))]:
+                                      (0, 2, 1, [2, 3] * 4, (1, 1)), (0, 6, 2, [27, 28] * 4, (1, 1)),
+                                      # tables of a wave's 64 lanes and more: the totals carried from group to group, an expert of
+                                      # too many rows in a later one, down tiles only
+                                      *((0, 23, 12, [1] + [0] * (n - 2) + [last], parts) for n in (63, 64, 65, 128, 129, 256)
+                                        for last, parts in ((32, (4, 4)), (33, (1, 1)))),
+                                      (0, 3, 2, [0, 1, 200, 2] * 64, (1, 1)), (5, 23, 12, ([1] + [0] * 51) * 4 + [0] * 40, (1, 4))]:
         out = subprocess.run([exe, str(op), str(gu), str(dn), *map(str, counts)], check=True, capture_output=True, text=True).stdout.splitlines()
         assert tuple(map(int, out[0].split())) == parts
         want = set()
@@ -157,6 +162,24 @@ def test_the_grid_has_room_for_the_tasks_and_for_quarters_only_where_they_may_be
     assert list(map(int, res.stdout.split())) == [112, 112, 72, 72, 72, 80]
 
 
+@pytest.mark.skipif(not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs the ROCm toolchain")
+def test_the_packages_link_with_the_short_ring(tmp_path):
+    """Ring depth 2 is the other value pipelines may bind: the code for parts must leave that link's register allocation possible
+    (with parts and whole tiles in one loop the compiler did not survive it)."""
+    import json
+
+    from pipelink_amd.pipec import linker, pack
+    from pipelink_amd.stages.mok import build as mok_build
+
+    for stage_id, rel in mok_build.STAGES:
+        pack.pack_stage(mok_build.HERE / rel, tmp_path / f"{stage_id}.plink")
+    pipeline = json.loads((mok_build.HERE / "pipelines_fwd.json").read_text())
+    pipeline["pipeline"]["forced_bindings"]["pipelink_mok_gemm_depth"] = 2
+    (tmp_path / "pipeline.json").write_text(json.dumps(pipeline))
+    link = linker.link(tmp_path / "pipeline.json", tmp_path / "link")
+    assert link["bindings"]["pipelink_mok_gemm_depth"] == [2, "forced"] and link["observed"]["calls"] == 0
+
+
 # one to 32 rows an expert (33: whole tiles); a contraction of one slot, fewer pairs than waves, an odd number of slots, one
 # more pair than a ring; columns that end inside a column tile; gate/up and down tiles cut, down tiles only, none; rows of whole
 # cache lines (one launch) or not; from `(448, 256` on: quarters of the shortest contractions that are cut
@@ -164,7 +187,9 @@ def test_the_grid_has_room_for_the_tasks_and_for_quarters_only_where_they_may_be
 @pytest.mark.parametrize("H,I,counts", [(64, 64, [1]), (128, 320, [32, 0, 5]), (576, 192, [31, 17, 1, 32]), (704, 1088, [2] * 5),
                                         (2880, 2880, [1, 0, 1, 1, 1]), (2880, 2880, [3, 2, 1, 1, 32, 9, 1]), (1536, 2048, [4] * 7),
                                         (448, 704, [33, 2, 1]), (320, 128, [20] * 8),
-                                        (448, 256, [16]), (512, 192, [5]), (320, 192, [7]), (576, 384, [9, 0, 31, 1]), (1088, 448, [31, 1]), (1536, 64, [3])])
+                                        (448, 256, [16]), (512, 192, [5]), (320, 192, [7]), (576, 384, [9, 0, 31, 1]), (1088, 448, [31, 1]), (1536, 64, [3]),
+                                        # more experts than a wave has lanes: the expert of a task found beyond the first 64, parts and none
+                                        (512, 512, [0] * 100 + [3] + [0] * 28 + [1]), (256, 192, [1, 0, 2] * 43 + [70]), (128, 128, [1, 0, 2] * 85 + [5])])
 def test_forward_of_few_rows_matches_the_oracle(H, I, counts):
     from oracle import moe_ffn
     from pipelink_amd.host import mok_inputs
@@ -186,3 +211,48 @@ def test_forward_of_few_rows_matches_the_oracle(H, I, counts):
                     assert not np.isnan(yy).any() and moe_ffn.rel_frobenius(yy, ref["y"]) <= TOL
                     ys.append(yy)
     assert all(np.array_equal(ys[0], other) for other in ys[1:])   # one launch and two, linked and one unit: the same sums
+
+
+@pytest.mark.gpu
+def test_parts_through_the_static_entry_point_and_in_a_graph():
+    """Gate/up and down tiles in parts, one launch (rows of whole cache lines) and two, without a session's own buffers: the
+    bytes of the plain forward, also on every replay of a captured graph."""
+    import json
+
+    import torch
+    from pipelink_amd.host import mok_inputs
+    from pipelink_amd.host.backend import HipBackend
+    from pipelink_amd.host.mok import MoKSession
+    from pipelink_amd.stages.mok import build as mok_build
+    from test_zz_no_alloc import _device_problem, _poison, _snapshot
+
+    paths = mok_build.images()
+    link = json.loads(paths["link_json"].read_text())
+    with MoKSession(paths["linked"].read_bytes(), link) as sess, MoKSession(paths["linked"].read_bytes(), link) as fresh:
+        cases = [_device_problem(sess, mok_inputs.generate(40, H, I, len(c), 1, seed=H, counts=c), H, I, pitch)
+                 for H, I, c, pitch in ((1088, 704, [31, 1, 0, 7], 768), (1088, 704, [31, 1, 0, 7], None), (1536, 64, [3], 128))]
+        expected = []
+        for prob, out, _ in cases:
+            _poison(out)
+            sess.forward(prob)
+            expected.append(_snapshot(out))
+        be = HipBackend(0, 0)
+        stream = be.stream_create()
+        graph = be.capture(stream, lambda: [fresh.forward_static(prob, stream=stream) for prob, _, _ in cases])
+        try:
+            for replay in range(4):   # the first turn is the plain call
+                for _, out, _ in cases:
+                    _poison(out)
+                torch.cuda.synchronize()
+                if replay:
+                    graph.launch(stream)
+                    be.synchronize(stream)
+                else:
+                    for prob, _, _ in cases:
+                        sess.forward_static(prob)
+                for (_, out, _), want in zip(cases, expected):
+                    assert all(torch.equal(g, w) for g, w in zip(_snapshot(out), want)), replay
+            assert fresh.status() == 0 and sess.status() == 0
+        finally:
+            graph.close()
+            be.close()
