@@ -37,18 +37,18 @@ def _half_tiles_pay(heads: int, s: int, window: int | None) -> bool:
     return longest >= (10 if tiles <= COMPUTE_UNITS else 12) and heads * sum(chains) <= 0.78 * COMPUTE_UNITS * longest
 
 
-def _half_of(link_json: str | Path) -> Path | None:
-    """The half-tile link that was made for exactly this link (``stages.attention.build.link_half``), if there is one: a link
-    redone since, with another mask for instance, has other bytes than the one recorded."""
-    link = Path(link_json)
-    half = link.parent.parent / "half"
+def _half_of(link_json: Path, link_bytes: bytes) -> tuple[dict, Path] | None:
+    """The half-tile link that was made for exactly this link (``stages.attention.build.link_half``) and its folder, if there is
+    one: a link redone since, with another mask for instance, has other bytes than the one recorded."""
+    folder = link_json.parent.parent / "half"
     try:
-        of = json.loads((half / "of.json").read_text())
-        same = all(hashlib.sha256(path.read_bytes()).hexdigest() == of[name]
-                   for name, path in (("whole", link), ("half", half / "link" / "link.json")))
+        of = json.loads((folder / "of.json").read_text())
+        if hashlib.sha256(link_bytes).hexdigest() != of["whole"]:
+            return None
+        half_bytes = (folder / "link" / "link.json").read_bytes()
+        return (json.loads(half_bytes), folder / "link") if hashlib.sha256(half_bytes).hexdigest() == of["half"] else None
     except (OSError, ValueError, KeyError, TypeError):
         return None
-    return half / "link" / "link.json" if same else None
 
 
 def open_session(link_json: str | Path | dict, q_bits: np.ndarray, k_bits: np.ndarray, v_bits: np.ndarray, *, scale: float | None = None,
@@ -71,10 +71,15 @@ def open_session(link_json: str | Path | dict, q_bits: np.ndarray, k_bits: np.nd
     if s * d * 2 >= 1 << 31:
         raise ValueError("one head of K or V must stay below 2 GiB")
     buffers = {"q": q_bits, "k": k_bits, "v": v_bits, "o": ((b, s, hq * d), np.uint16)}
-    # (an image of the caller's own, and a link handed over as an object, are run as they are)
-    whole = isinstance(link_json, dict) or image is not None or not _half_tiles_pay(b * hq, s, window)
-    chosen = link_json if whole else _half_of(link_json) or link_json
-    link = chosen if isinstance(chosen, dict) else json.loads(Path(chosen).read_text())
+    if isinstance(link_json, dict):
+        link = link_json
+    else:
+        link_bytes = Path(link_json).read_bytes()
+        link, folder = json.loads(link_bytes), Path(link_json).parent
+        if image is None:   # (an image of the caller's own, and a link handed over as an object, are run as they are)
+            half = _half_of(Path(link_json), link_bytes) if _half_tiles_pay(b * hq, s, window) else None
+            link, folder = half or (link, folder)
+            image = folder / link["target"]["image"]
     grid = b * hq * (s // link.get("facts", {}).get("fa.core.tile_queries", Q_TILE))
-    return open_hostless(chosen, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
+    return open_hostless(link, buffers=buffers, params=lambda addr: params_blobs(addr, b, hq, hkv, s, scale, window),
                          grid=(grid,), backend=backend, image=image)
