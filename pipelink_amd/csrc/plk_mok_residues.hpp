@@ -105,31 +105,38 @@ inline int64_t workspace_words(const Dims& d) { return MOK_WS_COUNTERS + max_row
 // bytes of a row).  Otherwise the forward is two launches.
 inline bool one_launch_ok(const Dims& d, uint64_t hidden_q) { return d.ld_q_i % 128 == 0 && hidden_q % 128 == 0; }
 
+// The launches whose column tiles may be cut in four (mok_framework::cut_for): every expert with rows is one row tile then,
+// and holds 32 rows at most.  f(row tiles, cut) for each number of row tiles that would be cut.
+template <class F>
+inline void each_cut(const Dims& d, F f) {
+  if (d.routed_rows > 16 * (int64_t)d.experts) return;
+  for (int t = (d.routed_rows + mok_framework::NARROW_ROWS - 1) / mok_framework::NARROW_ROWS; t <= d.experts && t <= d.routed_rows; ++t) {
+    const mok_framework::Cut cut = mok_framework::cut_for(d.routed_rows, d.experts, t, num_col_tiles_gate_up(d), num_col_tiles_down(d));
+    if (cut.down != 0) f(t, cut);
+  }
+}
+
 inline MokFrameworkParams framework_params(const Dims& d, uint64_t tokens_per_expert, uint64_t workspace) {
   MokFrameworkParams fw{};
   fw.tokens_per_expert = (const int32_t*)(uintptr_t)tokens_per_expert;
   fw.workspace = (uint32_t*)(uintptr_t)workspace;
   fw.num_experts = d.experts;
   fw.op = d.pass == 0 ? MOK_FWD_BOTH : d.pass == 1 ? MOK_GEMM_FWD_ROUTED_GATE_UP : MOK_GEMM_FWD_ROUTED_DOWN;
+  each_cut(d, [&](int, mok_framework::Cut) { fw.op |= MOK_FWD_MAY_CUT; });
   fw.num_col_tiles_gate_up = num_col_tiles_gate_up(d);
   fw.num_col_tiles_down = num_col_tiles_down(d);
   return fw;
 }
 
 // an upper bound of the number of tiles of the launch: more workgroups than this would idle, and cost the others time when
-// they start and leave (a layer of 448 x 704 with 509 tokens: 38 us with 72 workgroups, 41 with 256).  A launch that may cut
-// its column tiles in four (mok_framework::cut_for) is bounded by its parts: every expert with rows is one row tile then, and
-// holds 32 rows at most.
+// they start and leave (a layer of 448 x 704 with 509 tokens: 38 us with 72 workgroups, 41 with 256).
 inline int64_t max_workgroups(const Dims& d) {
   const int gu = num_col_tiles_gate_up(d), down = num_col_tiles_down(d);
   auto launched = [&](int64_t row_tiles, mok_framework::Cut cut) {
     return row_tiles * ((d.pass != 2 ? gu << cut.gate_up : 0) + (d.pass != 1 ? down << cut.down : 0));
   };
   int64_t most = launched(max_row_tiles(d), {0, 0});
-  for (int t = (d.routed_rows + mok_framework::NARROW_ROWS - 1) / mok_framework::NARROW_ROWS; t <= d.experts && t <= d.routed_rows; ++t) {
-    const mok_framework::Cut cut = mok_framework::cut_for(d.routed_rows, d.experts, t, gu, down);
-    most = std::max(most, launched(t, cut));
-  }
+  each_cut(d, [&](int row_tiles, mok_framework::Cut cut) { most = std::max(most, launched(row_tiles, cut)); });
   return most;
 }
 

@@ -53,7 +53,7 @@ struct Tables {
                    // that leaves the launch last
   uint32_t claim;  // what the list's queue answered this workgroup's last request
 
-  // exclusive prefix sums of rows and row tiles per expert, one expert after the other
+  // exclusive prefix sums of rows and row tiles per expert, one expert after the other (what the tests compare the next with)
   MOK_SCHED_FN void fill(const int32_t* tokens_per_expert, int ne) {
     int rows = 0, tiles = 0;
     for (int e = 0; e < ne; ++e) {
@@ -101,6 +101,7 @@ struct Schedule {
   // Narrow tiles, for launches all of whose experts have at most NARROW_ROWS rows (every wave looks at the tables itself):
   // cut_for says whose column tiles are cut in four.
   MOK_SCHED_FN void cut() {
+    if (!(g.op & MOK_FWD_MAY_CUT)) return;  // (most launches know here: the tables' sums and the rule took them 0.1 us)
     const Cut c = cut_for(tab.row_begin[g.num_experts], g.num_experts, row_tiles, g.num_col_tiles_gate_up, g.num_col_tiles_down);
     if (MOK_SCHED_UNIFORM(c.down) == 0) return;
     if (MOK_SCHED_COUNT(g.num_experts, [&](int e) { return tab.row_begin[e + 1] - tab.row_begin[e] > NARROW_ROWS; }) != 0) return;
@@ -140,7 +141,7 @@ struct Schedule {
     const int col = local / (t1 - t0);
     const int tile = t0 + local - col * (t1 - t0);  // row tile, counted over all experts
     const int first = tab.row_begin[e] + (tile - tab.tile_begin[e]) * TILE_X;
-    const bool both = g.op == MOK_FWD_BOTH;
+    const bool both = (g.op & MOK_FWD_OP_MASK) == MOK_FWD_BOTH;
     // wave-uniform by construction; say so, so that the task lives in scalar registers
     MokGemmTask t;
     t.op = gate_up ? MOK_GEMM_FWD_ROUTED_GATE_UP : MOK_GEMM_FWD_ROUTED_DOWN;

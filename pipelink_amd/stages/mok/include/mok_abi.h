@@ -30,6 +30,9 @@ enum {
   MOK_GEMM_FWD_ROUTED_GATE_UP = 3, /* = MOK_GEMM_FWD_ROUTED_GATE of the reference */
   MOK_GEMM_FWD_ROUTED_DOWN = 5
 };
+/* Beside the op in MokFrameworkParams.op: the grid has room for column tiles cut in parts; whether they are cut the kernel
+ * finds from the experts' rows.  Without it none are. */
+enum { MOK_FWD_MAY_CUT = 0x100, MOK_FWD_OP_MASK = 0xff };
 enum { MOK_ACT_FWD_ROUTED = 1 };
 
 #ifndef MOKGEMMTASK_DEFINED
@@ -107,7 +110,7 @@ typedef struct MokFrameworkParams {
   uint32_t* workspace;              /* MOK_WS_* words + one counter per routed-row tile; all zero before a launch,
                                        and the launch leaves them zero (except the status word and the poll limit) */
   int32_t num_experts;
-  int32_t op;                       /* which GEMM this launch runs, or MOK_FWD_BOTH */
+  int32_t op;                       /* which GEMM this launch runs, or MOK_FWD_BOTH; MOK_FWD_MAY_CUT */
   int32_t num_col_tiles_gate_up;    /* column tiles of the gate/up GEMM (128 gate + 128 up columns each) */
   int32_t num_col_tiles_down;       /* column tiles of the down GEMM (256 columns each) */
 } MokFrameworkParams;

@@ -36,7 +36,7 @@ int main(int argc, char** argv) {
     }
   for (int e = 0; e <= ne; ++e) if (tab.row_begin[e] != want.row_begin[e] || tab.tile_begin[e] != want.tile_begin[e]) { printf("table differs at %d\n", e); return 2; }
   if (tab.last != 0xA5u || tab.claim != 0xA5u) { printf("the tables write the queues' words\n"); return 3; }
-  const MokFrameworkParams g{counts.data(), nullptr, ne, op, gu, dn};
+  const MokFrameworkParams g{counts.data(), nullptr, ne, op | MOK_FWD_MAY_CUT, gu, dn};
   Schedule sched{g, tab, tab.tile_begin[ne], op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : gu, op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : dn};
   sched.cut();
   printf("%d %d\n", 1 << sched.gate_up_cut, 1 << sched.down_cut);
@@ -144,6 +144,12 @@ int main() {
     Schedule sched{g, tab, tab.tile_begin[d.experts], d.pass == 2 ? 0 : g.num_col_tiles_gate_up, d.pass == 1 ? 0 : g.num_col_tiles_down};
     sched.cut();
     const long long tasks = sched.gate_up_items() + sched.down_items();
+    // the same tasks whatever the host says of them, as long as it says that they may be
+    MokFrameworkParams told = g;
+    told.op |= MOK_FWD_MAY_CUT;
+    Schedule asked{told, tab, sched.row_tiles, sched.gate_up_cols, sched.down_cols};
+    asked.cut();
+    if (asked.gate_up_cut != sched.gate_up_cut || asked.down_cut != sched.down_cut) { printf("the host does not expect what the kernel cuts\n"); return 1; }
     if (tasks > plk_mok::max_workgroups(d)) { printf("%lld tasks, %lld workgroups\n", tasks, (long long)plk_mok::max_workgroups(d)); return 1; }
   }
   // a layer of 448 x 704, top 2 of 8: nothing is cut from 65 tokens on, and the grid has no room for it

@@ -27,6 +27,7 @@ inline void barrier() { puts("barrier"); }
 #define __syncthreads() barrier()
 #define __builtin_amdgcn_s_barrier() barrier()
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)
+#define __builtin_amdgcn_sched_barrier(x) ((void)0)
 #define __builtin_amdgcn_update_dpp(old, v, ...) (old)
 #define __builtin_amdgcn_readfirstlane(v) (v)
 #define __builtin_amdgcn_readlane(v, l) (v)
@@ -73,7 +74,7 @@ int main(int argc, char** argv) {
   g.tokens_per_expert = &tokens;
   g.workspace = workspace;
   g.num_experts = 1;
-  g.op = MOK_FWD_BOTH;
+  g.op = MOK_FWD_BOTH | MOK_FWD_MAY_CUT;
   g.num_col_tiles_gate_up = gu;
   g.num_col_tiles_down = dn;
   gridDim.x = workgroups;
