@@ -337,7 +337,7 @@ int plk_mok_forward_static(plk_mok_session* s, const plk_mok_problem* p, void* s
 //
 // A pass over memory (one read of the values, one write of codes and scales), so what counts is how few instructions stand
 // between the two.  A lane takes 16 consecutive bytes of values (8 of bf16, 4 of fp32), four or eight lanes a block of 32, a
-// lane Q_PIECES such pieces at once so that several loads per lane are in flight; magnitudes are compared as integers (an
+// lane Q_PIECES such pieces (the compiler waits for each load; other waves fill that time); magnitudes are compared as integers (an
 // infinity or a NaN is the largest, which is the rule's exponent field 255); the block's maximum is two or three lane
 // permutations; a piece's row comes from one high multiply; NaN codes are patched in a branch that a block without one
 // does not enter.

@@ -109,7 +109,7 @@ __device__ __forceinline__ void forward(const MokActResidue& p, const MokActTask
   // The tile is counted when all of it is in memory: every wave waits until its own stores have been written through (a
   // store leaves the wave's vector-memory count when it is acknowledged; the barrier's workgroup-scope fence does not wait
   // for that), then the workgroup meets, then one thread counts the tile.  The row tile's counter reaches the number of
-  // gate/up column tiles when all of its `hidden` can be read by any workgroup
+  // its gate/up tasks (column tiles, or four parts of each) when all of its `hidden` can be read by any workgroup
   // (campaigns/mok/port/framework/interp_fwd.cu:174-213: the reference's act -> down dependency).
   auto count_tile = [&]() {
     if (t.counter_idx >= 0 && counters.base) __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)

@@ -15,9 +15,9 @@
 // tiles out in list order, one atomic per tile, and a workgroup whose list is handed out asks another list that has tiles left
 // (the reference asks the cluster launch control for its next tile, interp_fwd.cu:137-160).  Tiles differ in cost
 // (full ones, and those of few rows or few columns, which have a placement of their own), and turns of equal length
-// leave the workgroups that drew the full ones tiles behind the others.  A down tile reads rows of `hidden` that up
-// to 23 other workgroups write: it waits until the row tile's readiness counter (MokCounters) has reached the number
-// of gate/up column tiles.  In every list all gate/up tiles come before the first down tile and the queue hands out
+// leave the workgroups that drew the full ones tiles behind the others.  A down tile reads rows of `hidden` that the
+// gate/up tasks of its row tile write (column tiles, or four parts of each): it waits until the row tile's readiness counter
+// (MokCounters) has reached their number.  In every list all gate/up tiles come before the first down tile and the queue hands out
 // in that order, gate/up tiles wait for nothing, and a workgroup only ever waits while it holds no unfinished tile:
 // so the tiles a wait depends on are finished or running, no wait can last, and each is bounded anyway.
 //

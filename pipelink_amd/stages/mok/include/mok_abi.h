@@ -49,7 +49,7 @@ typedef struct MokGemmTask {
   int32_t task_idx;  /* running index of the tile in the schedule */
   int32_t counter_idx; /* readiness counter of the tile's routed-row tile (a launch of both GEMMs), or -1 */
   int32_t wait_target; /* down op: value that counter must have reached before the tile's rows of `hidden` are read
-                          (the number of gate/up column tiles); 0 = the tile waits for nothing */
+                          (the number of the row tile's gate/up tasks); 0 = the tile waits for nothing */
   uint32_t flags;
 } MokGemmTask;
 #endif
