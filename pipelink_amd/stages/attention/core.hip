@@ -170,7 +170,10 @@ __device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_hos
   // constant so that the address tables are registers
   auto block = [&](int i, auto pair, auto tiles) {
     constexpr int PB = decltype(pair)::value, NT = decltype(tiles)::value;
-    __syncthreads();  // blocks i of K and V have landed (the barrier drains every wave's loads); buffers of block i - 1 are free
+    // blocks i of K and V have landed, and the buffers of block i - 1 are free.  (The barrier itself waits for no global -> LDS
+    // load, and a wave that left the last block early, because none of its queries sees a key of it, has met no other wait.)
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __syncthreads();
     if (i + 1 < blocks) {
       issue_block<false>(kres, (uint32_t)(i + 1) * FA_K_BLOCK * FA_D * 2, buf + (1 - PB) * BUF_BYTES, wave, lane);
       issue_block<true>(vres, (uint32_t)(i + 1) * FA_K_BLOCK * FA_D * 2, buf + (1 - PB) * BUF_BYTES + K_BYTES, wave, lane);
