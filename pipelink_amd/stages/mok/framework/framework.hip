@@ -56,6 +56,16 @@ extern __shared__ __attribute__((aligned(1024))) unsigned char pipelink_smem[];
 namespace mok_framework {
 static_assert(TILE_X == mok::TILE_X && TILE_W == mok::TILE_W, "the schedule's tile is the GEMM owner's");
 
+// The queue's answer has arrived.  Said where every wave passes: read only behind a branch of thread 0's, it is on its way for
+// ever as far as the compiler can tell, and whichever later code writes its register waits, in the next tile's mainloop too.
+__device__ __forceinline__ void arrived(uint32_t answer) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" ::"v"(answer));
+#else
+  (void)answer;
+#endif
+}
+
 // inclusive sum over the lanes of a full wave: within rows of 16 lanes, then across them
 __device__ __forceinline__ int wave_scan(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
@@ -189,6 +199,7 @@ __device__ __forceinline__ void run_tiles(const void* params, const MokFramework
       }
       // the queue's answer goes round the workgroup through LDS; the barrier is one every wave reaches at about the
       // same time (the epilogue has just ended with one)
+      arrived(answer);
       if (threadIdx.x == 0) tab.claim = answer;
       mok::lds_barrier();
       MokGemmTask after = next;

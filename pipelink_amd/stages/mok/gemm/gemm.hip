@@ -533,17 +533,6 @@ __device__ __forceinline__ void issue_few(const Loader& ld, const FewRing& ring,
 #pragma unroll
   for (int i = 0; i < W_GROUPS; ++i) buf16_to_lds(ld.w, ld.wsrc[i], wslot, base + ld.dst + i * 1024);
 }
-__device__ __forceinline__ void wait_few(int loads) {  // a multiple of FEW_LOADS, at most (FEW_DEPTH - 1) of them
-  switch (__builtin_amdgcn_readfirstlane(loads) / FEW_LOADS) {
-    case 0: wait_loads_and_reads<0>(); break;
-    case 1: wait_loads_and_reads<FEW_LOADS>(); break;
-    case 2: wait_loads_and_reads<2 * FEW_LOADS>(); break;
-    case 3: wait_loads_and_reads<3 * FEW_LOADS>(); break;
-    case 4: wait_loads_and_reads<4 * FEW_LOADS>(); break;
-    case 5: wait_loads_and_reads<5 * FEW_LOADS>(); break;
-    default: wait_loads_and_reads<6 * FEW_LOADS>(); break;
-  }
-}
 // which placement the task's tile has: its routed rows that exist, its output columns that exist
 __device__ __forceinline__ int placement_of(const MokGemmResidue& g, const MokGemmTask& t) {
   const int cols = (t.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? g.w_gate.rows : g.w_down.rows) - t.col_begin;
@@ -1051,6 +1040,11 @@ __device__ __forceinline__ void mainloop_small(const MokGemmResidue& g, const Mo
 
 // The mainloop of a tile of at most 64 rows in the deep ring (ring depth 4 and up; mainloop_small<DEPTH, SMALL_ROWS_FRAGS>
 // otherwise): the small placement's fragments a = 0 and a = 2, two routed-row fragments, four MFMAs a step.
+// A step has 256 clocks of MFMAs; what bounds it while the memory is not busy is the other instructions one wave issues, about
+// five clocks each.  With the ring position a product, the waits a switch on a computed count and every fragment's address its
+// own (110 instructions and eight branches a step) a step took 0.41 us, whatever its loads were of; with 50 instructions and no
+// branch 0.22.  us before / after: one token of 2880 x 2880, top 4 of 32, 41.7 / 36.3; two 54.0 / 43.0; three 60.3 / 54.0; 128,
+// where all compute units stream at once, 169.0 / 166.8.
 __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const MokGemmTask& t, AccFrag& acc, const GemmCarry& carry,
                                                   const MokGemmTask* upcoming, const MokCounters& counters) {
   const int tid = fresh_tid();  // nothing of this path is to be computed ahead and kept across full tiles
@@ -1063,47 +1057,48 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
   const FewRing ring;
   const Rings<4> r;
   const Loader ld = make_loader(v, t, carry);
-  const SmallPlacement sp = small_placement(TILE_SMALL_ROWS, wave);
-  int xoff[2], xscoff[2], woff[2], wscoff[2];
-#pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    const int row = 32 * b + r32;
-    xoff[b] = BUF_BYTES + row * K_SLOT + 16 * (half ^ swizzle(row));
-    xscoff[b] = row * 16;
-  }
-#pragma unroll
-  for (int a = 0; a < 2; ++a) {
-    const int wl = sp.wr[2 * a] + r32;
-    woff[a] = wl * K_SLOT + 16 * (half ^ swizzle(wl));
-    wscoff[a] = wl * 4;
-  }
+  // Fragment addresses: routed rows 0..31 and 32..63 and weight rows 32 w.. and 128 + 32 w.. are whole multiples of 16 rows
+  // apart, so they share a swizzle and lie constants apart; the second 16 bytes of a lane have bit 5 flipped.
+  const int xoff = BUF_BYTES + r32 * K_SLOT + 16 * (half ^ swizzle(r32));
+  const int woff = wave * 32 * K_SLOT + r32 * K_SLOT + 16 * (half ^ swizzle(r32));
+  const unsigned char* const xsc_at = r.xscale() + r32 * 16;
+  const unsigned char* const wsc_at = r.wscale() + (wave * 32 + r32) * 4;
   zero_fragments(acc.v[0][0], acc.v[0][1], acc.v[2][0], acc.v[2][1]);
 
   // slots 0 .. FEW_HEAD_SLOTS - 1 were asked for by `prefetch`; the rest of the ring now
 #pragma unroll
   for (int s = FEW_HEAD_SLOTS; s < FEW_DEPTH; ++s) issue_few(ld, ring, r, s, s, n);
   if (upcoming->op != 0) stage(g, *upcoming, counters);
-  wait_few(few_younger(0, -1, n));
+  // (the counts below are of a ring full of loads: with fewer slots than it holds they would let some of them go)
+  static_assert(few_younger(0, -1, 1 << 20) == (FEW_DEPTH - 1) * FEW_LOADS && few_younger(101, 99, 1 << 20) == (FEW_DEPTH - 2) * FEW_LOADS,
+                "the waits' counts");
+  if (n < FEW_DEPTH) wait_loads_and_reads<0>();
+  else wait_loads_and_reads<(FEW_DEPTH - 1) * FEW_LOADS>();
   wg_barrier();
 
   struct FewOperands {
     v8i x[2], w[2];
   } even, odd;
   int sx[2], sw[2], sxn[2], swn[2];
+  auto frag = [&](const unsigned char* lo, const unsigned char* hi) {
+    const v4i l = *reinterpret_cast<const v4i*>(lo), h = *reinterpret_cast<const v4i*>(hi);
+    return v8i{l.x, l.y, l.z, l.w, h.x, h.y, h.z, h.w};
+  };
   auto read_operands_few = [&](FewOperands& o, const unsigned char* slot) {
+    const unsigned char *x0 = slot + xoff, *x1 = slot + (xoff ^ 32), *w0 = slot + woff, *w1 = slot + (woff ^ 32);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) o.x[b] = read_frag(slot, xoff[b]);
+    for (int b = 0; b < 2; ++b) o.x[b] = frag(x0 + b * 32 * K_SLOT, x1 + b * 32 * K_SLOT);
 #pragma unroll
-    for (int a = 0; a < 2; ++a) o.w[a] = read_frag(slot, woff[a]);
+    for (int a = 0; a < 2; ++a) o.w[a] = frag(w0 + a * (TILE_W / 2) * K_SLOT, w1 + a * (TILE_W / 2) * K_SLOT);
   };
   auto read_scales_few = [&](int (&sx_)[2], int (&sw_)[2], int j) {  // of the pair of slots that starts at slot j (j even)
     const int c = (j & 7) >> 1;
-    const unsigned char* xbuf = r.xscale() + ((j >> 3) & 1) * (TILE_X * 16);
-    const unsigned char* wbuf = r.wscale() + c * (TILE_W * 4);
+    const unsigned char* xbuf = xsc_at + ((j >> 3) & 1) * (TILE_X * 16) + 4 * c;
+    const unsigned char* wbuf = wsc_at + c * (TILE_W * 4);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) sx_[b] = (int)(*reinterpret_cast<const uint32_t*>(xbuf + 4 * c + xscoff[b]) >> (8 * half));
+    for (int b = 0; b < 2; ++b) sx_[b] = (int)(*reinterpret_cast<const uint32_t*>(xbuf + b * 32 * 16) >> (8 * half));
 #pragma unroll
-    for (int a = 0; a < 2; ++a) sw_[a] = (int)(*reinterpret_cast<const uint32_t*>(wbuf + wscoff[a]) >> (8 * half));
+    for (int a = 0; a < 2; ++a) sw_[a] = (int)(*reinterpret_cast<const uint32_t*>(wbuf + a * (TILE_W / 2) * 4) >> (8 * half));
   };
   auto multiply = [&](auto ODD_, const FewOperands& o) {
     constexpr bool ODD = decltype(ODD_)::value;
@@ -1116,21 +1111,51 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
   };
   read_operands_few(even, ring.slot(0));
   read_scales_few(sx, sw, 0);
-  int pos = 0;  // ring position of slot t_ in `advance`
-  // step t_: slot t_ + 1 has landed for every wave and every wave holds slot t_ in registers, whose place takes slot
-  // t_ + FEW_DEPTH
-  auto advance = [&](int t_, FewOperands& next) {
-    wait_few(few_younger(t_ + 1, t_ - 1, n));
+  // Step t: slot t + 1 has landed for every wave and every wave holds slot t in registers, whose place takes slot
+  // t + FEW_DEPTH.  A step is a quarter of a full tile's MFMAs, so its other instructions count: the ring position is two
+  // offsets that advance, the loads behind the last slot are issued all the same (of an operand without extent: zeros, no
+  // memory traffic), so that the wait is a constant.
+  uint32_t here = 0, ahead = FEW_SLOT_BYTES;  // where slots t and t + 1 are, from the ring's first place
+  const uint32_t arena = (uint32_t)(ring.arena - ring.head);
+  int s = FEW_DEPTH;                          // the slot step t issues
+  const void *const x_base = v.act.q, *const w_base = v.w.q + (int64_t)__builtin_amdgcn_readfirstlane(t.expert) * v.w.expert_pitch_q;
+  uint32_t x_bytes = (uint32_t)v.act.rows * (uint32_t)v.act.ld_q, w_bytes = (uint32_t)v.w.rows * (uint32_t)v.w.k;
+  uint32_t kbyte = FEW_DEPTH * K_SLOT, wslot = FEW_DEPTH * ld.w_slot_pitch;
+  const uint32_t wave_x = BUF_BYTES + wave * 1024;
+  auto issue = [&](auto ODD_) {  // ODD: of step t; slot t + FEW_DEPTH is even then
+    static_assert(FEW_DEPTH % 2 == 1, "an odd step issues an even slot");
+    x_bytes = s < n ? x_bytes : 0;
+    w_bytes = s < n ? w_bytes : 0;
+    const rsrc_t x = make_rsrc(x_base, x_bytes), w = make_rsrc(w_base, w_bytes);
+    unsigned char* const at = ring.head + here;
+    if constexpr (decltype(ODD_)::value) {
+      if (s < n) {
+        if ((s & 7) == 0) buf16_to_lds_device_scope(ld.xsc, ld.xscsrc, kbyte >> 5, r.xscale() + ((s >> 3) & 1) * (TILE_X * 16) + wave * 1024);
+        buf4_to_lds(ld.wsc, ld.wscsrc, (uint32_t)(s >> 1) * ld.wsc_pair_pitch, r.wscale() + ((s & 7) >> 1) * (TILE_W * 4) + wave * 256);
+      }
+    }
+    buf16_to_lds(x, ld.xsrc[0], kbyte, at + wave_x);
+#pragma unroll
+    for (int i = 0; i < W_GROUPS; ++i) buf16_to_lds(w, ld.wsrc[i], wslot, at + ld.dst + i * 1024);
+    ++s;
+    kbyte += K_SLOT;
+    wslot += ld.w_slot_pitch;
+  };
+  auto advance = [&](auto ODD_, FewOperands& next) {
+    wait_loads_and_reads<(FEW_DEPTH - 2) * FEW_LOADS>();
     wg_barrier();
-    issue_few(ld, ring, r, t_ + FEW_DEPTH, pos, n);
-    pos = pos + 1 == FEW_DEPTH ? 0 : pos + 1;
-    read_operands_few(next, ring.slot(pos));
+    issue(ODD_);
+    read_operands_few(next, ring.head + ahead);
+    here = ahead;
+    ahead += FEW_SLOT_BYTES;
+    ahead = ahead == FEW_HEAD_SLOTS * FEW_SLOT_BYTES ? arena : ahead;
+    ahead = ahead == arena + (FEW_DEPTH - FEW_HEAD_SLOTS) * FEW_SLOT_BYTES ? 0u : ahead;
   };
   int j = 0;
   for (; j + 1 < n; j += 2) {
-    advance(j, odd);
+    advance(std::false_type{}, odd);
     multiply(std::false_type{}, even);
-    advance(j + 1, even);
+    advance(std::true_type{}, even);
     read_scales_few(sxn, swn, j + 2);
     multiply(std::true_type{}, odd);
 #pragma unroll
@@ -1139,7 +1164,8 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
     for (int a = 0; a < 2; ++a) sw[a] = swn[a];
   }
   if (n & 1) multiply(std::false_type{}, even);
-  wg_barrier();  // every wave holds its last operands in registers: the ring is free
+  wait_loads_and_reads<0>();  // (the zeros behind the last slot have been written)
+  wg_barrier();               // every wave holds its last operands in registers: the ring is free
 }
 
 // The mainloop of a narrow tile: leaves the sums in wave 0's fragments [0][0] and [2][0].
