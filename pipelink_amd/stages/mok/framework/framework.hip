@@ -56,6 +56,19 @@ extern __shared__ __attribute__((aligned(1024))) unsigned char pipelink_smem[];
 namespace mok_framework {
 static_assert(TILE_X == mok::TILE_X && TILE_W == mok::TILE_W, "the schedule's tile is the GEMM owner's");
 
+// Asks a queue for its next number, without waiting for the answer.  (An addition of one lane is made one of a wave by the
+// compiler, which has the answer spread over the lanes at once: 1 to 2 us in front of the next tile's first loads.  A wrapping
+// increment it leaves alone.)  us with the addition / this, and the two accesses of LDS that waited for everything: one token of
+// 2880 x 2880, top 4 of 32, 36.3 / 34.8; 27 160.1 / 158.2; 128 167.0 / 164.7; 448 x 704, 60 tokens 19.7 / 18.9.  Full tiles keep
+// the addition: there the increment's register is the one that makes the next mainloop wait (2000 tokens 277.0 / 279.5).
+__device__ __forceinline__ uint32_t take_one(uint32_t* queue) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_atomic_inc32(queue, 0xFFFFFFFFu, __ATOMIC_RELAXED, "agent");
+#else
+  return __hip_atomic_fetch_add(queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#endif
+}
+
 // The queue's answer has arrived.  Said where every wave passes: read only behind a branch of thread 0's, it is on its way for
 // ever as far as the compiler can tell, and whichever later code writes its register waits, in the next tile's mainloop too.
 __device__ __forceinline__ void arrived(uint32_t answer) {
@@ -111,7 +124,7 @@ __device__ __attribute__((noinline)) SmallTileResult small_tile(const void* para
   mok::AccFrag acc;
   pipelink_call_gemm_fwd_small(&view, &task, &counters, &phase, &acc, &carry, &next);
   uint32_t answer = 0;
-  if (queue && threadIdx.x == 0) answer = __hip_atomic_fetch_add(queue, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (queue && threadIdx.x == 0) answer = take_one(queue);
   const bool early = next.op != 0 && pipelink_call_gemm_ready(&view, &next, &counters);
   if (early) pipelink_call_gemm_prefetch(&view, &next, &carry);
   if (task.op == MOK_GEMM_FWD_ROUTED_GATE_UP) {

@@ -356,7 +356,8 @@ __device__ __forceinline__ void stage(const MokGemmResidue& g, const MokGemmTask
 __device__ __forceinline__ bool staged_ready(const MokGemmTask& t, const MokCounters& counters) {
   if (!waits(t, counters)) return true;
   const Rings<2> r;
-  return *reinterpret_cast<const volatile int32_t*>(r.peek()) >= t.wait_target;
+  // (as an LDS access: a volatile read through a generic pointer is one of any memory, and waits for all loads there are)
+  return *(const volatile __attribute__((address_space(3))) int32_t*)r.peek() >= t.wait_target;
 }
 // Waits until the rows the task reads are complete: one thread polls the counter at device scope, the others wait at
 // the barrier.  A bounded poll: after WAIT_POLLS probes (a few tens of milliseconds; a wait that can be met takes
@@ -1270,6 +1271,9 @@ __device__ __forceinline__ void mainloop_narrow(const MokGemmResidue& g, const M
 // half a tile (depth 2) falls back to 8-byte stores straight from the registers.
 constexpr int Y_PITCH = TILE_W * 2 + 16;  // bytes per staged row: 256 bf16 + pad against bank conflicts
 
+// LDS is written here while the next tile's loads into LDS fly.  The compiler waits for all of those in front of an LDS access of
+// which it does not know that it is of another type than theirs: a struct like uint2 says nothing, a vector type does.
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
@@ -1374,10 +1378,7 @@ __device__ __forceinline__ void store_down(const MokGemmResidue& g, const MokGem
 #pragma unroll
               for (int q = 0; q < 4; ++q) {
                 const int col = sp.wr[a] + 8 * q + 4 * (lane >> 5);
-                uint2 pk;
-                pk.x = pack_bf16x2(f[4 * q + 0], f[4 * q + 1]);
-                pk.y = pack_bf16x2(f[4 * q + 2], f[4 * q + 3]);
-                *reinterpret_cast<uint2*>(rowp + col * 2) = pk;
+                *reinterpret_cast<v2u*>(rowp + col * 2) = v2u{pack_bf16x2(f[4 * q + 0], f[4 * q + 1]), pack_bf16x2(f[4 * q + 2], f[4 * q + 3])};
               }
             }
           }
@@ -1392,10 +1393,7 @@ __device__ __forceinline__ void store_down(const MokGemmResidue& g, const MokGem
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const int col = wrow0(wave, a) + 8 * q + 4 * (lane >> 5);
-              uint2 pk;
-              pk.x = pack_bf16x2(f[4 * q + 0], f[4 * q + 1]);
-              pk.y = pack_bf16x2(f[4 * q + 2], f[4 * q + 3]);
-              *reinterpret_cast<uint2*>(rowp + col * 2) = pk;
+              *reinterpret_cast<v2u*>(rowp + col * 2) = v2u{pack_bf16x2(f[4 * q + 0], f[4 * q + 1]), pack_bf16x2(f[4 * q + 2], f[4 * q + 3])};
             }
           }
         }
@@ -1406,8 +1404,8 @@ __device__ __forceinline__ void store_down(const MokGemmResidue& g, const MokGem
         const int srow = wave * (ROWS / WAVES) + it * 2 + (lane >> 5);
         const int row = t.row_begin + pass * ROWS + srow;
         if (row < t.row_end && col_ok) {
-          const uint4 v = *reinterpret_cast<const uint4*>(stage + srow * Y_PITCH + chunk * 16);
-          *reinterpret_cast<uint4*>(g.y + (int64_t)row * g.ld_y + t.col_begin + chunk * 8) = v;
+          const v4i v = *reinterpret_cast<const v4i*>(stage + srow * Y_PITCH + chunk * 16);
+          *reinterpret_cast<v4i*>(g.y + (int64_t)row * g.ld_y + t.col_begin + chunk * 8) = v;
         }
       }
       __syncthreads();  // the arena is reused by the next pass or the next tile's loads
