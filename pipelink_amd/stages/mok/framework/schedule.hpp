@@ -112,11 +112,25 @@ struct Schedule {
   MOK_SCHED_FN int down_items() const { return row_tiles * down_cols << down_cut; }
 
   // List q: the q-th eighth of the gate/up tiles (all experts' tiles in one sequence: expert by expert, column tile by
-  // column tile, row tiles innermost), then the q-th eighth of the down tiles.
+  // column tile, row tiles innermost), then the q-th eighth of the down tiles, from its second expert on (`rotated`).
   MOK_SCHED_FN int share(int q, int total) const { return (int)((long long)q * total / NUM_XCD); }
   MOK_SCHED_FN int length(int q) const {
     const int gu = gate_up_items(), d = down_items();
     return share(q + 1, gu) - share(q, gu) + share(q + 1, d) - share(q, d);
+  }
+
+  // The down tile list q runs in the place of `item` (launches of both GEMMs): the rest of the expert in whose middle the list
+  // begins comes last.  That expert's gate/up tiles are divided alike, some of them the end of the list before, which run last
+  // of all gate/up tiles: its down tiles, first in this list, held workgroups for up to a tile's time.  us in the old order /
+  // this: 14 tokens of 2880 x 2880, top 4 of 32, 152.4 / 138.9; 10 142.0 / 135.8; 20 and 27 157.9 / 159.1; 1003 212.7 / 210.8;
+  // 4000 429 / 421; 8192 801 / 794.  (Launches of parts are one turn of the chip: one token 34.6 / 35.8.)
+  MOK_SCHED_FN int rotated(int q, int d, int item) const {
+    const int first = share(q, d), end = share(q + 1, d);
+    const int e = MOK_SCHED_COUNT(g.num_experts, [&](int x) { return tab.tile_begin[x] * down_cols <= first; }) - 1;  // of item `first`
+    const int next = MOK_SCHED_UNIFORM(tab.tile_begin[e + 1]) * down_cols;  // the next expert's first item
+    if (MOK_SCHED_UNIFORM(tab.tile_begin[e]) * down_cols == first || next >= end) return item;
+    const int at = item + next - first;
+    return at < end ? at : at - (end - first);
   }
 
   // item i of list q -> task.  `cursor` is the expert of the item this workgroup decoded last: a workgroup's items
@@ -125,7 +139,8 @@ struct Schedule {
     const int gu = gate_up_items(), d = down_items();
     const int mine = share(q + 1, gu) - share(q, gu);
     const bool gate_up = i < mine;
-    const int item = gate_up ? share(q, gu) + i : share(q, d) + i - mine;  // in the sequence of its GEMM's items
+    int item = gate_up ? share(q, gu) + i : share(q, d) + i - mine;  // in the sequence of its GEMM's items
+    if (!gate_up && gu != 0 && down_cut == 0) item = rotated(q, d, item);
     const int cut = gate_up ? gate_up_cut : down_cut;                      // a column tile's parts are neighbours
     const int idx = item >> cut, part = item - (idx << cut);
     const int cols = gate_up ? gate_up_cols : down_cols;
