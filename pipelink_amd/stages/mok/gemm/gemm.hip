@@ -1046,6 +1046,7 @@ __device__ __forceinline__ void mainloop_small(const MokGemmResidue& g, const Mo
 // own (110 instructions and eight branches a step) a step took 0.41 us, whatever its loads were of; with 50 instructions and no
 // branch 0.22.  us before / after: one token of 2880 x 2880, top 4 of 32, 41.7 / 36.3; two 54.0 / 43.0; three 60.3 / 54.0; 128,
 // where all compute units stream at once, 169.0 / 166.8.
+template <int B>  // routed-row fragments
 __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const MokGemmTask& t, AccFrag& acc, const GemmCarry& carry,
                                                   const MokGemmTask* upcoming, const MokCounters& counters) {
   const int tid = fresh_tid();  // nothing of this path is to be computed ahead and kept across full tiles
@@ -1078,9 +1079,9 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
   wg_barrier();
 
   struct FewOperands {
-    v8i x[2], w[2];
+    v8i x[B], w[2];
   } even, odd;
-  int sx[2], sw[2], sxn[2], swn[2];
+  int sx[B], sw[2], sxn[B], swn[2];
   auto frag = [&](const unsigned char* lo, const unsigned char* hi) {
     const v4i l = *reinterpret_cast<const v4i*>(lo), h = *reinterpret_cast<const v4i*>(hi);
     return v8i{l.x, l.y, l.z, l.w, h.x, h.y, h.z, h.w};
@@ -1088,16 +1089,16 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
   auto read_operands_few = [&](FewOperands& o, const unsigned char* slot) {
     const unsigned char *x0 = slot + xoff, *x1 = slot + (xoff ^ 32), *w0 = slot + woff, *w1 = slot + (woff ^ 32);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) o.x[b] = frag(x0 + b * 32 * K_SLOT, x1 + b * 32 * K_SLOT);
+    for (int b = 0; b < B; ++b) o.x[b] = frag(x0 + b * 32 * K_SLOT, x1 + b * 32 * K_SLOT);
 #pragma unroll
     for (int a = 0; a < 2; ++a) o.w[a] = frag(w0 + a * (TILE_W / 2) * K_SLOT, w1 + a * (TILE_W / 2) * K_SLOT);
   };
-  auto read_scales_few = [&](int (&sx_)[2], int (&sw_)[2], int j) {  // of the pair of slots that starts at slot j (j even)
+  auto read_scales_few = [&](int (&sx_)[B], int (&sw_)[2], int j) {  // of the pair of slots that starts at slot j (j even)
     const int c = (j & 7) >> 1;
     const unsigned char* xbuf = xsc_at + ((j >> 3) & 1) * (TILE_X * 16) + 4 * c;
     const unsigned char* wbuf = wsc_at + c * (TILE_W * 4);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) sx_[b] = (int)(*reinterpret_cast<const uint32_t*>(xbuf + b * 32 * 16) >> (8 * half));
+    for (int b = 0; b < B; ++b) sx_[b] = (int)(*reinterpret_cast<const uint32_t*>(xbuf + b * 32 * 16) >> (8 * half));
 #pragma unroll
     for (int a = 0; a < 2; ++a) sw_[a] = (int)(*reinterpret_cast<const uint32_t*>(wbuf + a * (TILE_W / 2) * 4) >> (8 * half));
   };
@@ -1106,7 +1107,7 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < B; ++b)
         acc.v[2 * a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(o.w[a], o.x[b], acc.v[2 * a][b], 0, 0, ODD ? 2 : 0, sw[a],
                                                                           ODD ? 2 : 0, sx[b]);
   };
@@ -1145,8 +1146,9 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
   auto advance = [&](auto ODD_, FewOperands& next) {
     wait_loads_and_reads<(FEW_DEPTH - 2) * FEW_LOADS>();
     wg_barrier();
-    issue(ODD_);
     read_operands_few(next, ring.head + ahead);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(ODD_);
     here = ahead;
     ahead += FEW_SLOT_BYTES;
     ahead = ahead == FEW_HEAD_SLOTS * FEW_SLOT_BYTES ? arena : ahead;
@@ -1160,7 +1162,7 @@ __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const
     read_scales_few(sxn, swn, j + 2);
     multiply(std::true_type{}, odd);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) sx[b] = sxn[b];
+    for (int b = 0; b < B; ++b) sx[b] = sxn[b];
 #pragma unroll
     for (int a = 0; a < 2; ++a) sw[a] = swn[a];
   }
@@ -1501,7 +1503,10 @@ extern "C" __device__ void mok_gemm_fwd_small(const void* view, const MokGemmTas
         break;
       }
       if (placement == mok::TILE_SMALL_ROWS) {  // (the deep ring needs the arena of depth 4; mok_gemm_prefetch decides alike)
-        mok_gemm_owner::mainloop_few_rows(g, *task, *acc, *carry, upcoming, *counters);
+        // (32 rows, one fragment of them: half the MFMAs and three quarters of the LDS reads.  us with two fragments / this: one
+        // token of 2880 x 2880, top 4 of 32, 34.7 / 32.5; two 42.3 / 39.8; 128 164.8 / 164.1; 448 x 704, 60 tokens 18.9 / 18.6)
+        if (task->row_end - task->row_begin <= 32) mok_gemm_owner::mainloop_few_rows<1>(g, *task, *acc, *carry, upcoming, *counters);
+        else mok_gemm_owner::mainloop_few_rows<2>(g, *task, *acc, *carry, upcoming, *counters);
         break;
       }
       switch (frags) { PL_SMALL(4, mok::SMALL_COLS_FRAGS_GATE_UP) PL_SMALL(4, mok::SMALL_COLS_FRAGS_DOWN) }
