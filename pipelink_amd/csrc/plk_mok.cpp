@@ -102,7 +102,8 @@ static int make_workspace(plk_mok_session* s, int64_t words) {
 // One pass's params image: the three owners' records at their linked offsets, zeros between them.
 static void fill_image(const plk_mok_link_info& link, const plk_mok_problem* p, int pass, uint64_t workspace, unsigned char* image) {
   const plk_mok::Dims d = dims_of(p, pass);
-  const MokFrameworkParams fw = plk_mok::framework_params(d, p->tokens_per_expert, workspace);
+  MokFrameworkParams fw = plk_mok::framework_params(d, p->tokens_per_expert, workspace);
+  plk_mok::offer_parts(d, fw);
   const MokGemmResidue g = plk_mok::gemm_residue(
       d, plk_mok::GemmAddresses{p->x_q, p->x_sc, p->w_gate_q, p->w_gate_sc, p->w_up_q, p->w_up_sc, p->w_down_q, p->w_down_sc,
                                 p->hidden_q, p->hidden_sc, p->y, p->row_token});
@@ -116,7 +117,7 @@ static void fill_image(const plk_mok_link_info& link, const plk_mok_problem* p, 
 // on every CU, a multiple of the XCD count, but no more workgroups than there can be tiles.
 static int launch_pass(plk_mok_session* s, const plk_mok_problem* p, int pass, void* stream, uint64_t params_dev) {
   const plk_mok::Dims d = dims_of(p, pass);
-  const int64_t max_tiles = plk_mok::max_workgroups(d);
+  const int64_t max_tiles = plk_mok::useful_workgroups(d);
   int64_t wgs = (int64_t)s->compute_units * s->link.workgroups_per_cu;
   if (wgs > max_tiles) wgs = max_tiles;
   wgs = (wgs + NUM_XCD - 1) / NUM_XCD * NUM_XCD;

@@ -116,6 +116,21 @@ inline void each_cut(const Dims& d, F f) {
   }
 }
 
+// Parts of 64 columns (mok_framework::parts_for): of `cols` columns, and of the last column tile of `tile` columns.
+inline int32_t parts(int32_t cols) { return (cols + mok_framework::PART_COLS - 1) / mok_framework::PART_COLS; }
+inline int32_t last_parts(int32_t cols, int tile) { return parts(cols - (cols - 1) / tile * tile); }
+// The most row tiles with which the launch may run parts, or 0 where it does not: where the number that is to be expected, half
+// a tile more than full ones for each expert, is too many already, a grid with room for parts would mostly be idle workgroups
+// (2500 tokens of 448 x 704, top 2 of 8: 38.3 us, 40.2 with it).
+inline int64_t part_row_tiles(const Dims& d) {
+  auto run = [&](int64_t t) { return mok_framework::parts_for(d.routed_rows, d.experts, (int)t, parts(d.intermediate), parts(d.hidden)); };
+  const int64_t full = ((int64_t)d.routed_rows + TILE_X - 1) / TILE_X;
+  if (!run(full + d.experts / 2)) return 0;
+  int64_t t = max_row_tiles(d);
+  while (!run(t)) --t;
+  return t;
+}
+
 inline MokFrameworkParams framework_params(const Dims& d, uint64_t tokens_per_expert, uint64_t workspace) {
   MokFrameworkParams fw{};
   fw.tokens_per_expert = (const int32_t*)(uintptr_t)tokens_per_expert;
@@ -128,7 +143,7 @@ inline MokFrameworkParams framework_params(const Dims& d, uint64_t tokens_per_ex
   return fw;
 }
 
-// an upper bound of the number of tiles of the launch: more workgroups than this would idle, and cost the others time when
+// an upper bound of the number of tiles of a launch that runs no parts: more workgroups than this would idle, and cost the others time when
 // they start and leave (a layer of 448 x 704 with 509 tokens: 38 us with 72 workgroups, 41 with 256).
 inline int64_t max_workgroups(const Dims& d) {
   const int gu = num_col_tiles_gate_up(d), down = num_col_tiles_down(d);
@@ -138,6 +153,18 @@ inline int64_t max_workgroups(const Dims& d) {
   int64_t most = launched(max_row_tiles(d), {0, 0});
   each_cut(d, [&](int row_tiles, mok_framework::Cut cut) { most = std::max(most, launched(row_tiles, cut)); });
   return most;
+}
+
+// What the forward entry adds: it sizes the grid itself, so its launches may run parts.  (Owners of a launch whose geometry the
+// caller chose do not offer them.)
+inline void offer_parts(const Dims& d, MokFrameworkParams& fw) {
+  if (part_row_tiles(d) != 0)
+    fw.op |= last_parts(d.intermediate, TILE_W / 2) << MOK_FWD_LAST_GATE_UP_SHIFT | last_parts(d.hidden, TILE_W) << MOK_FWD_LAST_DOWN_SHIFT;
+}
+
+// The launch's workgroups: as many as may have a tile of their own, whole or a part.
+inline int64_t useful_workgroups(const Dims& d) {
+  return std::max(max_workgroups(d), part_row_tiles(d) * ((d.pass != 2 ? parts(d.intermediate) : 0) + (d.pass != 1 ? parts(d.hidden) : 0)));
 }
 
 }  // namespace plk_mok

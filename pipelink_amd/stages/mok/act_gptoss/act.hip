@@ -105,7 +105,8 @@ __device__ __forceinline__ void forward(const MokActResidue& p, const MokActTask
     if (half == 0) stage[STAGE_SCALE_OFF + trow * 4 + (tcol >> 5)] = (uint8_t)e;
   };
   // ---- activation + requant into an LDS tile [256 rows][128 codes] + [256 rows][4 scales] ----
-  const int placement = tile_placement(t.row_end - t.row_begin, p.cols - t.col_begin, t.flags);
+  const int col_end = SMALL ? cols_end(t.col_begin, t.flags, p.cols) : p.cols;
+  const int placement = tile_placement(t.row_end - t.row_begin, col_end - t.col_begin, t.flags);
   // The tile is counted when all of it is in memory: every wave waits until its own stores have been written through (a
   // store leaves the wave's vector-memory count when it is acknowledged; the barrier's workgroup-scope fence does not wait
   // for that), then the workgroup meets, then one thread counts the tile.  The row tile's counter reaches the number of
@@ -163,7 +164,7 @@ __device__ __forceinline__ void forward(const MokActResidue& p, const MokActTask
   // Stores of `hidden` are device-scope (cache policy bit 4, sc1): they go through to memory, where a workgroup on
   // another XCD -- a down tile of the same launch, once the row tile's counter says so -- reads them.
   const int chunk = lane & 7;
-  const bool col_ok = t.col_begin + chunk * 16 < p.cols;  // column extents are multiples of 32
+  const bool col_ok = t.col_begin + chunk * 16 < col_end;  // column extents are multiples of 32
 #pragma unroll
   for (int it = 0; it < TILE_X / (THREADS / 64) / 8; ++it) {
     const int trow = wave * (TILE_X / (THREADS / 64)) + it * 8 + (lane >> 3);
@@ -180,11 +181,11 @@ __device__ __forceinline__ void forward(const MokActResidue& p, const MokActTask
     if (row < t.row_end) {
       const uint32_t sc = *reinterpret_cast<const uint32_t*>(stage + STAGE_SCALE_OFF + tid * 4);
       uint8_t* out = p.hidden_sc + (int64_t)row * p.ld_sc + (t.col_begin >> 5);
-      if (t.col_begin + TILE_W / 2 <= p.cols) {
+      if (t.col_begin + TILE_W / 2 <= col_end) {
         // col_begin is a multiple of 128: dword aligned
         __hip_atomic_store(reinterpret_cast<uint32_t*>(out), sc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       } else {
-        for (int j = 0; t.col_begin + 32 * j < p.cols; ++j)
+        for (int j = 0; t.col_begin + 32 * j < col_end; ++j)
           __hip_atomic_store(out + j, (uint8_t)(sc >> (8 * j)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }

@@ -48,6 +48,19 @@ constexpr Cut cut_for(long long rows, int experts, int row_tiles, int gate_up_co
   if (both_pay) c.gate_up = 2;
   return c;
 }
+
+// Launches of more rows: every column tile is parts of 64 columns (MOK_TASK_PART) if all the parts of each GEMM run at once and
+// an expert has more than 64 rows on average.  A layer of few column tiles leaves most of the chip idle, and a launch takes as
+// long as one tile: its steps, which wait for 16 MFMAs each, and an epilogue of 128 x 128 values a wave.  A part has half the
+// MFMAs and epilogue (gate/up) or a quarter (down), spread over waves of 64 rows.  us whole / parts: 448 x 704, top 2 of 8, 257
+// tokens 33.4 / 27.6, 509 36.0 / 27.9, 2000 38.3 / 32.3; 256 x 256, top 1 of 4, 300 tokens 23.4 / 19.4; 704 x 448, 600 tokens of
+// one expert in four 34.4 / 26.1; 2048 x 512, 400 tokens 45.4 / 40.7; 2880 x 768, 500 tokens 50.1 / 49.9 (long contractions: the
+// whole tile's placed loop makes up for it).  With 16 to 64 rows on average tiles are mostly small ones already, which parts only
+// make more of: 140 tokens of the first layer 19.6 / 22.4, of 640 x 2560 with 50 rows an expert 27.1 / 34.3.
+constexpr int PART_COLS = 64;
+constexpr bool parts_for(long long rows, int experts, int row_tiles, int gate_up_parts, int down_parts) {
+  return rows > 64 * (long long)experts && row_tiles * gate_up_parts <= CHIP && row_tiles * down_parts <= CHIP;
+}
 }  // namespace mok_framework
 
 #endif

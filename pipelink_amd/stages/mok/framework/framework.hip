@@ -137,7 +137,7 @@ __device__ __attribute__((noinline)) SmallTileResult small_tile(const void* para
 }
 
 
-// The workgroup's tiles.  PARTS: a launch whose column tiles are cut, all of whose tiles are small ones; without it no task is
+// The workgroup's tiles.  PARTS: a launch whose column tiles are cut or parts, all of whose tiles are small ones; without it no task is
 // a part, and the compiler leaves out what parts need.  One loop for both costs launches without parts 0.2 to 0.7 us (the
 // parts' code between the others' and three times the scalar spills): 448 x 704, 160 tokens 20.4 / 20.7 us, 256 x 2048, 250
 // tokens 28.6 / 29.7, 27 tokens of 2880 x 2880 163.9 / 165.5.
@@ -148,7 +148,11 @@ __device__ __forceinline__ void run_tiles(const void* params, const MokFramework
   // one that is taken: 168 scalar spills, 144 with this)
   if (PARTS) __builtin_amdgcn_sched_barrier(0);
   const pipelink_host_view view{params, nullptr};
-  if (!PARTS) sched.gate_up_cut = sched.down_cut = 0;
+  if (!PARTS) {
+    sched.gate_up_cut = sched.down_cut = 0;
+    sched.gate_up_width = TILE_W / 2;
+    sched.down_width = TILE_W;
+  }
   uint32_t phase = 0;
 
   const int q = blockIdx.x % NUM_XCD;
@@ -281,9 +285,11 @@ extern "C" __device__ void mok_framework_worker(const void* params, unsigned var
   Schedule sched{g, tab, tab.tile_begin[ne], op == MOK_GEMM_FWD_ROUTED_DOWN ? 0 : g.num_col_tiles_gate_up,
                  op == MOK_GEMM_FWD_ROUTED_GATE_UP ? 0 : g.num_col_tiles_down};
   sched.cut();
+  sched.part();
   const MokCounters counters{op == MOK_FWD_BOTH ? reinterpret_cast<int32_t*>(g.workspace + MOK_WS_COUNTERS) : nullptr,
                              g.workspace + MOK_WS_STATUS};
-  if (sched.down_cut) run_tiles<true>(params, g, tab, sched, counters);
+  const bool small_only = sched.down_cut != 0 || sched.down_width == PART_COLS;  // (every tile is a small one then)
+  if (small_only) run_tiles<true>(params, g, tab, sched, counters);
   else run_tiles<false>(params, g, tab, sched, counters);
   pipelink_call_gemm_fini(&view);
 

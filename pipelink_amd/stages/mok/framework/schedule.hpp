@@ -97,6 +97,7 @@ struct Schedule {
   int row_tiles;  // of all experts
   int gate_up_cols, down_cols;  // column tiles of the GEMMs this launch runs (0: not run)
   int gate_up_cut = 0, down_cut = 0;  // a column tile is 2^cut tasks (one or four)
+  int gate_up_width = TILE_W / 2, down_width = TILE_W;  // columns of a column tile; PART_COLS: every task is a part
 
   // Narrow tiles, for launches all of whose experts have at most NARROW_ROWS rows (every wave looks at the tables itself):
   // cut_for says whose column tiles are cut in four.
@@ -107,6 +108,16 @@ struct Schedule {
     if (MOK_SCHED_COUNT(g.num_experts, [&](int e) { return tab.row_begin[e + 1] - tab.row_begin[e] > NARROW_ROWS; }) != 0) return;
     down_cut = MOK_SCHED_UNIFORM(c.down);
     gate_up_cut = MOK_SCHED_UNIFORM(c.gate_up);
+  }
+  // Parts of 64 columns, for launches of more rows that leave most of the chip idle: the column tiles are that narrow then.
+  MOK_SCHED_FN void part() {
+    const int last_gate_up = g.op >> MOK_FWD_LAST_GATE_UP_SHIFT & MOK_FWD_LAST_MASK, last_down = g.op >> MOK_FWD_LAST_DOWN_SHIFT & MOK_FWD_LAST_MASK;
+    if (last_gate_up == 0) return;
+    const int gu = (g.num_col_tiles_gate_up - 1) * (TILE_W / 2 / PART_COLS) + last_gate_up, d = (g.num_col_tiles_down - 1) * (TILE_W / PART_COLS) + last_down;
+    if (!MOK_SCHED_UNIFORM(parts_for(tab.row_begin[g.num_experts], g.num_experts, row_tiles, gu, d))) return;
+    if (gate_up_cols) gate_up_cols = gu;
+    if (down_cols) down_cols = d;
+    gate_up_width = down_width = PART_COLS;
   }
   MOK_SCHED_FN int gate_up_items() const { return row_tiles * gate_up_cols << gate_up_cut; }
   MOK_SCHED_FN int down_items() const { return row_tiles * down_cols << down_cut; }
@@ -163,11 +174,11 @@ struct Schedule {
     t.expert = e;
     t.row_begin = MOK_SCHED_UNIFORM(first);
     t.row_end = MOK_SCHED_UNIFORM(tab.row_begin[e + 1]);
-    t.col_begin = MOK_SCHED_UNIFORM(((col << cut) + part) * ((gate_up ? TILE_W / 2 : TILE_W) >> cut));
+    t.col_begin = MOK_SCHED_UNIFORM(((col << cut) + part) * ((gate_up ? gate_up_width : down_width) >> cut));
     t.task_idx = MOK_SCHED_UNIFORM(q << 24 | i);
     t.counter_idx = MOK_SCHED_UNIFORM(both ? tile : -1);
     t.wait_target = gate_up ? 0 : gate_up_cols << gate_up_cut;
-    t.flags = (uint32_t)MOK_SCHED_UNIFORM(cut != 0 ? MOK_TASK_QUARTER : 0);
+    t.flags = (uint32_t)MOK_SCHED_UNIFORM(cut != 0 ? MOK_TASK_QUARTER : down_width == PART_COLS ? MOK_TASK_PART : 0);
     return t;
   }
 };

@@ -101,6 +101,7 @@ struct Loader {
   uint32_t xsrc[X_GROUPS];        // this lane's 16 bytes of its row in each group, at k = 0
   uint32_t wsrc[W_GROUPS];
   int dst;                        // buffer-relative LDS byte offset of the wave's first group (both rings)
+  bool written;                   // the routed rows are `hidden` of this launch, whose cache lines two workgroups wrote: read at device scope
 };
 
 // LDS areas of one workgroup.  The first two buffers of each ring and the scale buffers (the
@@ -166,11 +167,20 @@ __device__ __forceinline__ void issue_w(const Loader& ld, const Rings<DEPTH>& r,
 
 // Issue row groups G0 .. G1-1 of the routed rows of slots j and j+1 (j even: the two halves of a
 // 128-byte line) into routed-row buffers buf0 and buf1, the two loads of a row group back to back.
-template <int G0, int G1, int DEPTH>
+// PARTS: the task may be a part of a column tile (a small tile's, or one of which the caller does not know).
+template <int G0, int G1, bool PARTS, int DEPTH>
 __device__ __forceinline__ void issue_x_groups(const Loader& ld, const Rings<DEPTH>& r, int j, int buf0, int buf1) {
   const uint32_t kbyte = (uint32_t)j * K_SLOT;
   unsigned char* dst0 = r.x(buf0) + ld.dst;
   unsigned char* dst1 = r.x(buf1) + ld.dst;
+  if (PARTS && ld.written) {
+#pragma unroll
+    for (int i = G0; i < G1; ++i) {
+      buf16_to_lds_device_scope(ld.x, ld.xsrc[i], kbyte, dst0 + i * 1024);
+      buf16_to_lds_device_scope(ld.x, ld.xsrc[i], kbyte + K_SLOT, dst1 + i * 1024);
+    }
+    return;
+  }
 #pragma unroll
   for (int i = G0; i < G1; ++i) {
     buf16_to_lds(ld.x, ld.xsrc[i], kbyte, dst0 + i * 1024);
@@ -452,11 +462,13 @@ __device__ __forceinline__ Loader make_loader(const Views& v, const MokGemmTask&
   ld.dst = wave * X_GROUPS * 1024;
   static_assert(X_GROUPS == W_GROUPS, "one wave offset serves both rings");
   const MokMxView& wv = v.w;
+  const int col_end = cols_end(t.col_begin, t.flags, wv.rows);
+  ld.written = !gate_up && t.flags & MOK_TASK_PART;
 #pragma unroll
   for (int i = 0; i < W_GROUPS; ++i) {
     const int wl = (wave * W_GROUPS + i) * 16 + lrow;  // tile-local weight row
     const int col = t.col_begin + (gate_up ? (wl & (TILE_W / 2 - 1)) : wl);
-    ld.wsrc[i] = col < wv.rows ? (uint32_t)col * (uint32_t)K_SLOT + chunk : PAST_THE_END;  // weights are K-tiled: [K/64][rows][64]
+    ld.wsrc[i] = col < col_end ? (uint32_t)col * (uint32_t)K_SLOT + chunk : PAST_THE_END;  // weights are K-tiled: [K/64][rows][64]
   }
   ld.w = make_rsrc(wv.q + (int64_t)expert * wv.expert_pitch_q, (uint32_t)wv.rows * (uint32_t)wv.k);
   ld.w_slot_pitch = (uint32_t)wv.rows * (uint32_t)K_SLOT;
@@ -465,7 +477,7 @@ __device__ __forceinline__ Loader make_loader(const Views& v, const MokGemmTask&
   const int col = t.col_begin + (gate_up ? (tid & (TILE_W / 2 - 1)) : tid);
   ld.wsc = make_rsrc(wv.sc + (int64_t)expert * wv.expert_pitch_sc,
                      (uint32_t)((wv.k + K_PAIR - 1) / K_PAIR) * (uint32_t)wv.rows * 4u);
-  ld.wscsrc = col < wv.rows ? (uint32_t)col * 4u : PAST_THE_END;
+  ld.wscsrc = col < col_end ? (uint32_t)col * 4u : PAST_THE_END;
   ld.wsc_pair_pitch = (uint32_t)wv.rows * 4u;
   return ld;
 }
@@ -477,18 +489,18 @@ __device__ __forceinline__ Loader make_loader(const Views& v, const MokGemmTask&
 // step after it.  With DEPTH == 2 the whole pair is issued on the even step.  Steps -DEPTH and
 // 1 - DEPTH only touch head buffers: `prefetch` issues them, and may run while the previous
 // tile's epilogue still uses the arena.
-template <int DEPTH>
+template <bool PARTS = false, int DEPTH>
 __device__ __forceinline__ void issue_step(const Loader& ld, const Rings<DEPTH>& r, int u, int n, int xb0, int xb1, int wb) {
   constexpr bool SPLIT = DEPTH >= 4;
   const int s = u + DEPTH;
   const int pair = (u & 1) ? s - 1 : s;
   if (pair < n) {
     if (!SPLIT) {
-      if ((u & 1) == 0) issue_x_groups<0, X_GROUPS>(ld, r, pair, xb0, xb1);
+      if ((u & 1) == 0) issue_x_groups<0, X_GROUPS, PARTS>(ld, r, pair, xb0, xb1);
     } else if ((u & 1) == 0) {
-      issue_x_groups<0, X_GROUPS / 2>(ld, r, pair, xb0, xb1);
+      issue_x_groups<0, X_GROUPS / 2, PARTS>(ld, r, pair, xb0, xb1);
     } else {
-      issue_x_groups<X_GROUPS / 2, X_GROUPS>(ld, r, pair, xb0, xb1);
+      issue_x_groups<X_GROUPS / 2, X_GROUPS, PARTS>(ld, r, pair, xb0, xb1);
     }
   }
   if (s < n) issue_w(ld, r, s, wb);
@@ -536,7 +548,7 @@ __device__ __forceinline__ void issue_few(const Loader& ld, const FewRing& ring,
 }
 // which placement the task's tile has: its routed rows that exist, its output columns that exist
 __device__ __forceinline__ int placement_of(const MokGemmResidue& g, const MokGemmTask& t) {
-  const int cols = (t.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? g.w_gate.rows : g.w_down.rows) - t.col_begin;
+  const int cols = cols_end(t.col_begin, t.flags, t.op == MOK_GEMM_FWD_ROUTED_GATE_UP ? g.w_gate.rows : g.w_down.rows) - t.col_begin;
   return tile_placement(t.row_end - t.row_begin, cols, t.flags);
 }
 
@@ -697,8 +709,8 @@ __device__ __forceinline__ void prefetch(const MokGemmResidue& g, const MokGemmT
   gather_rows(g, v, t, c);
   const Loader ld = make_loader(v, t, c);
   const Rings<DEPTH> r;
-  issue_step(ld, r, -DEPTH, n, 0, 1, 0);
-  issue_step(ld, r, 1 - DEPTH, n, 0, 1, 1);
+  issue_step<true>(ld, r, -DEPTH, n, 0, 1, 0);
+  issue_step<true>(ld, r, 1 - DEPTH, n, 0, 1, 1);
 }
 
 template <int DEPTH>
@@ -964,7 +976,7 @@ __device__ __forceinline__ void mainloop_small(const MokGemmResidue& g, const Mo
 
   // the prologue of the full tile: steps -DEPTH and 1 - DEPTH were issued by `prefetch`
 #pragma unroll
-  for (int u = 2 - DEPTH; u < 0; ++u) issue_step(ld, r, u, n, (u + DEPTH) & ~1, ((u + DEPTH) & ~1) + 1, u + DEPTH);
+  for (int u = 2 - DEPTH; u < 0; ++u) issue_step<true>(ld, r, u, n, (u + DEPTH) & ~1, ((u + DEPTH) & ~1) + 1, u + DEPTH);
   if (upcoming->op != 0) stage(g, *upcoming, counters);
   // (with at least DEPTH slots every step up to here has issued its loads: the count is a constant then, and the wait
   // one instruction instead of a computation and a branch table)
@@ -1015,7 +1027,7 @@ __device__ __forceinline__ void mainloop_small(const MokGemmResidue& g, const Mo
     wait_loads_and_reads_dyn(loads_younger_than_slot<DEPTH>(t_ + 1, t_ - 1, n));
     wg_barrier();
     const bool odd_step = t_ & 1;
-    issue_step(ld, r, t_, n, odd_step ? xnext(xb, XDEPTH - 2) : xnext(xb, XDEPTH - 1), odd_step ? xnext(xb, XDEPTH - 1) : xb, wb);
+    issue_step<true>(ld, r, t_, n, odd_step ? xnext(xb, XDEPTH - 2) : xnext(xb, XDEPTH - 1), odd_step ? xnext(xb, XDEPTH - 1) : xb, wb);
     xb = xnext(xb, 1);
     wb = wb + 1 == DEPTH ? 0 : wb + 1;
     read_operands_small(next, r.x(xb), r.w(wb));
@@ -1328,7 +1340,7 @@ __device__ __forceinline__ void store_down(const MokGemmResidue& g, const MokGem
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const int col = t.col_begin + sp.wr[a] + 8 * q + 4 * (lane >> 5);
-            if (row < t.row_end && col < g.w_down.rows) {
+            if (row < t.row_end && col < cols_end(t.col_begin, t.flags, g.w_down.rows)) {
               uint2 pk;
               pk.x = pack_bf16x2(f[4 * q + 0], f[4 * q + 1]);
               pk.y = pack_bf16x2(f[4 * q + 2], f[4 * q + 3]);
@@ -1363,7 +1375,7 @@ __device__ __forceinline__ void store_down(const MokGemmResidue& g, const MokGem
     constexpr int ROWS = TILE_X / PASSES;  // rows staged per pass
     unsigned char* stage = pipelink_smem + pipelink_mok_gemm_arena();
     const int chunk = lane & 31;                                  // 8 columns = 16 bytes
-    const bool col_ok = t.col_begin + chunk * 8 < g.w_down.rows;  // column extents are multiples of 32
+    const bool col_ok = t.col_begin + chunk * 8 < (small ? cols_end(t.col_begin, t.flags, g.w_down.rows) : g.w_down.rows);  // column extents are multiples of 32
 #pragma unroll
     for (int pass = 0; pass < PASSES; ++pass) {
       if (small) {

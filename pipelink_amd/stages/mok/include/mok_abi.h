@@ -30,6 +30,9 @@ enum {
   MOK_GEMM_FWD_ROUTED_GATE_UP = 3, /* = MOK_GEMM_FWD_ROUTED_GATE of the reference */
   MOK_GEMM_FWD_ROUTED_DOWN = 5
 };
+/* Beside the op in MokFrameworkParams.op: how many 64-column parts the last column tile of each GEMM has (0: the launch runs
+ * whole column tiles whatever its rows) -- gate/up 1 or 2, down 1 to 4. */
+enum { MOK_FWD_LAST_GATE_UP_SHIFT = 12, MOK_FWD_LAST_DOWN_SHIFT = 16, MOK_FWD_LAST_MASK = 0xf };
 /* Beside the op in MokFrameworkParams.op: the grid has room for column tiles cut in parts; whether they are cut the kernel
  * finds from the experts' rows.  Without it none are. */
 enum { MOK_FWD_MAY_CUT = 0x100, MOK_FWD_OP_MASK = 0xff };
@@ -38,7 +41,10 @@ enum { MOK_ACT_FWD_ROUTED = 1 };
 #ifndef MOKGEMMTASK_DEFINED
 #define MOKGEMMTASK_DEFINED
 /* MokGemmTask.flags, MokActTask.flags */
-enum { MOK_TASK_QUARTER = 1 }; /* a quarter of a column tile (32 gate + 32 up columns, or 64 down columns) of at most 32 rows */
+enum {
+  MOK_TASK_QUARTER = 1, /* a quarter of a column tile (32 gate + 32 up columns, or 64 down columns) of at most 32 rows */
+  MOK_TASK_PART = 2     /* 64 output columns (per weight matrix) of a column tile, of any rows */
+};
 
 typedef struct MokGemmTask {
   int32_t op;        /* MOK_GEMM_FWD_ROUTED_GATE_UP or MOK_GEMM_FWD_ROUTED_DOWN */

@@ -82,7 +82,13 @@ constexpr int SMALL_EXTENT = 64;
 // rows: routed rows of the tile that exist; cols: output columns (per weight matrix) from the tile's first that exist
 __device__ __forceinline__ int tile_placement(int rows, int cols, uint32_t flags) {
   return flags & MOK_TASK_QUARTER ? TILE_NARROW
+         : flags & MOK_TASK_PART ? TILE_SMALL_COLS
          : rows <= SMALL_EXTENT ? TILE_SMALL_ROWS : cols <= SMALL_EXTENT ? TILE_SMALL_COLS : TILE_FULL;
+}
+// one past the task's last output column, of `cols` the GEMM has
+__device__ __forceinline__ int cols_end(int col_begin, uint32_t flags, int cols) {
+  const int part = col_begin + SMALL_EXTENT;
+  return flags & MOK_TASK_PART && part < cols ? part : cols;
 }
 struct SmallPlacement {
   int xr0;    // first tile-local routed row of the wave
