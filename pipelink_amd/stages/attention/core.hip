@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include "include/fa_abi.h"
+#include "include/fa_order.hpp"
 
 extern "C" __device__ int pipelink_fa_kv();  // byte offset of the K / V^T buffers in dynamic LDS
 extern "C" __device__ int pipelink_call_mask_key_count(const void* view, int q_first, int q_last);
@@ -76,8 +77,9 @@ __device__ __forceinline__ void issue_block(__amdgpu_buffer_rsrc_t src, uint32_t
   }
 }
 // The transposing read: in a group of 16 lanes, lane i hands in the address of 4 consecutive d of key kbase + i / 4
-// and lane j receives keys kbase .. kbase + 3 at d = dbase + j.
-__device__ __forceinline__ v4s read_v_piece(const unsigned char* at) {
+// and lane j receives keys kbase .. kbase + 3 at d = dbase + j.  (The parameter is restricted for what inlining makes of it, alias
+// scopes on the read: one of which the compiler knows nothing waits for every load into LDS there is, the next block's too.)
+__device__ __forceinline__ v4s read_v_piece(const unsigned char* __restrict__ at) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(const_cast<unsigned char*>(at)));
 }
 // A value of this lane and the one of lane ^ 32, without a trip through the LDS: after the swap the first result
@@ -98,11 +100,7 @@ constexpr int TILE_QUERIES = split ? FA_Q_TILE / 2 : FA_Q_TILE;
 __device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_host_view& view, uint32_t index) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
-  const int heads = p.batch * p.q_heads;
-  const int q_tiles = p.seq / TILE_QUERIES;
-  // Causal tiles cost in proportion to their position: the latest (longest) tiles of every head are
-  // dispatched first, so that the grid does not end on a few long ones.  bh = batch * q_heads + head.
-  const int tile = q_tiles - 1 - (int)(index / heads), bh = index % heads;
+  const auto [tile, bh] = fa_order::tile_of((int)index, p.batch, p.q_heads, p.kv_heads, p.seq / TILE_QUERIES);
   const int b = bh / p.q_heads, h = bh % p.q_heads, kvh = h / (p.q_heads / p.kv_heads);
   const int q0 = tile * TILE_QUERIES, qw = q0 + 32 * (split ? wave & 1 : wave);  // the wave's first query
   const int key0 = split ? 32 * (wave >> 1) : 0;                                 // its first key of every block
@@ -126,6 +124,8 @@ __device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_hos
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.0f;
   float row_max = MASKED, row_sum = 0.0f;
+  // (in a register for good: read where it is used, it is loaded again in every block, behind the block's barrier)
+  const float scale_log2e = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, p.scale_log2e)));
   bool seen = false;  // this lane's query has met a key it may see (decided on unscaled scores: the scale is the caller's)
 
   // the mask package says which stretch of keys the tile's queries may see at all: blocks [first_block, blocks)
@@ -226,7 +226,7 @@ __device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_hos
     // then probabilities may be as large as that (harmless in fp32 sums and bf16 operands, and the final division
     // takes it out again), and the accumulated output and sum need no rescaling -- which they otherwise would
     // in most blocks, because some query of the wave sees a new maximum.
-    const float top = block_max * p.scale_log2e;
+    const float top = block_max * scale_log2e;
     const float new_max = top > row_max + RESCALE_SLACK ? top : row_max;
     const float alpha = __builtin_amdgcn_exp2f(row_max - new_max);
     row_max = new_max;
@@ -239,7 +239,7 @@ __device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_hos
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], p.scale_log2e, -reference));
+        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], scale_log2e, -reference));
         s[t][r] = e;
         block_sum += e;
       }
