@@ -12,22 +12,27 @@ struct Cut {
   int gate_up, down;
 };
 
-// A quarter streams a fourth of a tile's weights, at what one compute unit reaches whatever the others do (about 40 GB/s); it
-// costs a start, the sum of its waves' parts and an end, and each workgroup more a little at the launch's start and end.  So
-// the gain grows with the contraction's slots n and the loss with the launch's tasks after the cut.  us cut / us whole over
-// 2746 random layers (contractions of 1 to 45 slots, 1 to 32 active experts, 13 to 60 us), down tiles cut:
-//   n 4-5    up to 32 tasks 0.96, 33-64 0.99, 65-128 1.03, 193-256 1.13
-//   n 6-7    up to 64 0.95, 65-128 1.00, 193-256 1.04
-//   n 8-9    up to 64 0.90, 65-128 0.97 (one of 11 above 1.01), 129-192 1.00, 257-400 1.09
-//   n 10-13  up to 128 0.91, 129-192 0.98, 257-400 1.06
-//   n 14-19  up to 256 0.88, 257-400 0.95 (up to 1.03)        n 20-45  up to 400 0.79 (0.98 at most)
-// and with n of the gate/up GEMM and both cut, against down tiles only: n 4-5 0.97 / 1.00 / 1.06, n 8-9 0.91 / 0.98, n 10-13 up
-// to 192 0.91, n 14-45 up to 400 0.80: the same line serves both, and the two lines added where only both together pay.  With
-// it 0.902 on average, none above 1.015; the better of the three layouts each time would be 0.891.  (Every launch that fits one
-// turn cut, whatever n: up to 1.4.)  More quarters of a GEMM than run at once take a second turn, whose start costs more than
-// the finer cut gives: one token of 2880 x 2880, top 4 of 32, is 92 gate/up and 48 down tiles: 53.2 us whole, 44.2 with the
-// down tiles cut, 49.4 with both (368 and 192 quarters).
-constexpr int cut_line(int slots) { return 16 * slots - 40; }
+// A quarter takes a fourth of a tile's steps; it costs a start, the sum of its waves' parts and an end, and each workgroup more a
+// little at the launch's start and end.  So the gain grows with the contraction's slots n and the loss with the launch's tasks
+// after the cut.  us cut / us whole of 1360 random layers (contractions of 4 to 45 slots, 1 to 32 active experts, 13 to 60 us),
+// down tiles cut, by the tasks then:
+//   n 4-5    up to 64 tasks 1.04, 65-128 1.05, 129-256 1.11         n 6-7    up to 64 1.00, 65-128 1.01, 129-256 1.09
+//   n 8-9    up to 64 0.99, 65-128 1.01, 129-256 1.08               n 10-13  up to 64 1.00, 65-128 1.02, 129-192 1.04
+//   n 14-19  up to 64 0.98, 65-128 0.99, 129-192 1.01, 193-256 1.05
+//   n 24-31  up to 192 0.96, 193-240 1.00, 241-384 1.02             n 32-39  up to 240 0.94, 241-290 0.97, 290-430 0.99
+//   n 40-45  up to 240 0.91, 241-290 0.94, 291-430 0.97
+// and cut gate/up tiles against the better of the other two, n of their contraction: n 8-9 up to 64 1.00, 65-128 1.03; n 14-19 up
+// to 128 0.98, 129-192 1.02; n 20-45 up to 64 0.90, 65-128 0.93, 129-192 0.98, 193-256 1.01, 257-400 1.07: the same line serves
+// both, and the two lines added where only both together pay.  (It lay twice as high, 16 n - 40, while a whole tile of few rows
+// took 0.4 us a step: with that line 400 further layers take 0.9 % more on average, up to 21 %.)  More quarters of a GEMM than run at once take a
+// second turn, whose start costs more than the finer cut gives.
+constexpr int cut_line(int slots) { return slots < 10 ? 4 * slots + 12 : 7 * slots + 40; }
+// Where whole tiles take two turns of the chip already, quarters of down tiles that end within them fill the second one evenly:
+// 16 experts of 320 x 2432, 36 tokens, 304 + 32 tiles: 32.1 us whole, 29.3 as 304 + 128 tasks.  A third turn loses that: 576 x
+// 2880, 112 tokens, 368 + 48: 38.0 whole, 46.2 as 368 + 192.
+constexpr bool quarters_fill_the_second_turn(int gate_up, int down) {
+  return gate_up + down > CHIP && gate_up + 4 * down <= 2 * CHIP;
+}
 
 // row_tiles: of all experts, none of which has more than NARROW_ROWS rows.  (From the numbers of both GEMMs whatever a launch
 // runs: one launch and two give the same sums.)  The contraction's slots follow from the other GEMM's columns: 64 a slot, 256
@@ -42,7 +47,7 @@ constexpr Cut cut_for(long long rows, int experts, int row_tiles, int gate_up_co
   if (4 * down > CHIP) return c;
   // (the parts of a gate/up tile share cache lines of `hidden`, which only narrow down tiles read at device scope: gate/up tiles
   // are cut only where down tiles are)
-  const bool down_pays = gate_up + 4 * down <= down_line;
+  const bool down_pays = gate_up + 4 * down <= down_line || quarters_fill_the_second_turn(gate_up, down);
   const bool both_pay = 4 * gate_up <= CHIP && 4 * gate_up + 4 * down <= gate_up_line + (down_pays ? 0 : down_line);
   if (down_pays || both_pay) c.down = 2;
   if (both_pay) c.gate_up = 2;

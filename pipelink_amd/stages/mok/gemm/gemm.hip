@@ -553,9 +553,8 @@ __device__ __forceinline__ int placement_of(const MokGemmResidue& g, const MokGe
 }
 
 // ---- narrow tiles: a quarter of a column tile for at most 32 routed rows -----------------------------------------------
-// A launch of a few tokens has fewer column tiles than the chip has compute units, and one compute unit streams weights
-// at about 40 GB/s whatever the others do: the launch takes as long as one tile's stream.  The schedule then cuts each
-// column tile in four (schedule.hpp says when, and what it measured).
+// A launch of a few tokens has fewer column tiles than the chip has compute units, and takes as long as one tile's steps,
+// one after the other.  The schedule then cuts each column tile in four (cut.hpp says when, and what it measured).
 // 64 weight rows would leave waves without a fragment, so the waves split the contraction instead: wave w multiplies every
 // fourth pair of slots, all 64 weight rows x 32 routed rows, from a ring of its own that no other wave touches -- no barrier
 // in the loop -- and the four partial sums meet in wave 0 through LDS.

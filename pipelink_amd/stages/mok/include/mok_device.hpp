@@ -65,8 +65,8 @@ __device__ __forceinline__ int xrow0(int wave, int b) { return wave_x(wave) * 12
 
 // ---- tiles with little to multiply ------------------------------------------------------------------------------
 // A tile that holds at most 64 routed rows (the rows an expert has past its last full tile), or at most 64 output
-// columns per weight matrix (the columns past the last full column tile), is multiplied in another placement: every
-// wave takes 64 routed rows and up to four 32-row weight fragments, in the accumulator's fragments [a][b] with b < 2.
+// columns per weight matrix (the columns past the last full column tile, or a task that is one of a column tile's parts,
+// MOK_TASK_PART), is multiplied in another placement: every wave takes 64 routed rows and up to four 32-row weight fragments, in the accumulator's fragments [a][b] with b < 2.
 //   SMALL_ROWS: all four waves share routed rows 0..63; wave w owns weight fragments a = 0 and a = 2, tile rows
 //               32 w and 128 + 32 w (for the gate/up op: 32 gate columns and the same 32 up columns).
 //   NARROW:     (a task that is a quarter of a column tile, MOK_TASK_QUARTER: at most 32 rows) the waves split the
