@@ -20,6 +20,19 @@ def test_quarters_within_two_turns(tmp_path, gu, dn, experts, parts):
     assert tuple(map(int, out[:2])) == parts
 
 
+# contractions of one to four slots (64 columns and more; what the rule knows is that a column tile's columns are at least begun)
+@pytest.mark.parametrize("gu,dn,counts,parts", [
+    (1, 1, [4, 0, 0, 0], (1, 1)), (1, 1, [2, 1], (1, 1)), (1, 1, [13, 11, 12], (1, 1)),                # 64 x 64, 128 x 128: 11.1 us whole, 12.4 cut
+    (2, 1, [16], (1, 1)), (2, 1, [1, 0, 3, 0], (1, 1)), (2, 1, [1, 1, 1, 2], (1, 1)), (2, 1, [9, 9, 9], (1, 1)),   # 256 x 256
+    (4, 1, [1], (1, 4)),                                                                              # 256 x 512: seven slots of down contraction
+    (2, 2, [1], (4, 4)),                                                                              # 512 x 256: 15.9 us whole, 14.0
+    (2, 2, [1] * 3, (1, 1)),
+])
+def test_the_shortest_contractions_are_not_cut(tmp_path, gu, dn, counts, parts):
+    out = subprocess.run([_compile(tmp_path, SCHEDULE), "0", str(gu), str(dn), *map(str, counts)], check=True, capture_output=True, text=True).stdout.split()
+    assert tuple(map(int, out[:2])) == parts
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,I,counts", [(320, 2432, [3, 1, 32, 9] * 4), (704, 2560, [1, 5] * 8)])
 def test_forward_of_launches_of_two_turns(H, I, counts):
