@@ -57,17 +57,28 @@ constexpr Cut cut_for(long long rows, int experts, int row_tiles, int gate_up_co
   return c;
 }
 
-// Launches of more rows: every column tile is parts of 64 columns (MOK_TASK_PART) if all the parts of each GEMM run at once and
-// an expert has more than 64 rows on average.  A layer of few column tiles leaves most of the chip idle, and a launch takes as
-// long as one tile: its steps, which wait for 16 MFMAs each, and an epilogue of 128 x 128 values a wave.  A part has half the
-// MFMAs and epilogue (gate/up) or a quarter (down), spread over waves of 64 rows.  us whole / parts: 448 x 704, top 2 of 8, 257
-// tokens 33.4 / 27.6, 509 36.0 / 27.9, 2000 38.3 / 32.3; 256 x 256, top 1 of 4, 300 tokens 23.4 / 19.4; 704 x 448, 600 tokens of
-// one expert in four 34.4 / 26.1; 2048 x 512, 400 tokens 45.4 / 40.7; 2880 x 768, 500 tokens 50.1 / 49.9 (long contractions: the
-// whole tile's placed loop makes up for it).  With 16 to 64 rows on average tiles are mostly small ones already, which parts only
-// make more of: 140 tokens of the first layer 19.6 / 22.4, of 640 x 2560 with 50 rows an expert 27.1 / 34.3.
+// Launches of more rows: every column tile is parts of 64 columns (MOK_TASK_PART) where an expert has more than 64 rows on average,
+// all the parts of each GEMM run at once, and these take little time in all.  A layer of few column tiles leaves most of the chip
+// idle, and a launch takes as long as one tile: its steps, which wait for 16 MFMAs each, and an epilogue of 128 x 128 values a wave.
+// A part has half the MFMAs and epilogue (gate/up) or a quarter (down), spread over waves of 64 rows; but a step of it takes a
+// little longer than one of the whole tile's placed loop, the more so the more parts ask for loads.  So the gain is a fixed one, and
+// the loss grows with the two contractions' steps and with the steps of all parts of a GEMM (row tiles x columns x contraction, the
+// same number for either): the line is fitted to us parts - us whole.  us parts / us whole of 836 random layers of 128 to 2880
+// columns, 1 to 32 experts, by what is compared with PART_STEPS:
+//   up to 3000 0.84 (1.02 at most), 6000 0.90 (1.04), 9000 0.94 (1.04), 11000 0.97 (1.06), 14000 0.99 (1.05), above 1.03 (1.09)
+// 448 x 704, top 2 of 8, 257 tokens 33.4 / 27.6, 509 36.0 / 27.9, 2000 38.3 / 32.3; 256 x 256, top 1 of 4, 300 tokens 23.4 / 19.4;
+// 704 x 448, 600 tokens of one expert in four 34.4 / 26.1; 2048 x 512, 400 tokens 45.4 / 40.7; 1664 x 2752, 329 rows of four
+// experts 67.3 / 60.4 (whole / parts); 2880 x 2880, 515 rows of one expert 71.2 / 76.8.  With 64 output columns the down tiles are
+// as narrow already, and whole gate/up tiles take a single step: 41 layers of up to 768 columns of `hidden` 0.97, 50 of more 1.04,
+// up to 1.14 (64 x 1728, 1287 rows of three experts 32.6 / 37.2).
+// With 16 to 64 rows on average tiles are mostly small ones already, which parts only make more of: 140 tokens of the first layer
+// 19.6 / 22.4, of 640 x 2560 with 50 rows an expert 27.1 / 34.3.
 constexpr int PART_COLS = 64;
+constexpr int PART_STEPS = 14000;
 constexpr bool parts_for(long long rows, int experts, int row_tiles, int gate_up_parts, int down_parts) {
-  return rows > 64 * (long long)experts && row_tiles * gate_up_parts <= CHIP && row_tiles * down_parts <= CHIP;
+  return rows > 64 * (long long)experts && row_tiles * gate_up_parts <= CHIP && row_tiles * down_parts <= CHIP &&
+         (down_parts > 1 || gate_up_parts <= 12) &&
+         row_tiles * gate_up_parts * down_parts + 120 * (gate_up_parts + down_parts) <= PART_STEPS;
 }
 }  // namespace mok_framework
 

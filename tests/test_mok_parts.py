@@ -66,6 +66,18 @@ def test_parts_cover_the_columns_once_and_the_grid_has_room_for_them(tmp_path):
     assert int(res.stdout) > 1000
 
 
+# (us whole / parts) where parts are the faster ones, and where they are not: long contractions of several row tiles, 64 output columns
+@pytest.mark.parametrize("H,I,counts,parts", [(448, 704, [128] * 8, True), (2048, 512, [130, 90, 100, 80], True), (576, 320, [300, 33, 0, 70, 191], True),
+                                              (2880, 2880, [515], False), (2880, 2880, [266, 267], False), (2880, 2880, [73] * 4, False),   # 71.2 / 76.8
+                                              (2368, 2304, [853], False), (2880, 2432, [250, 250, 251], False),                            # 63.3 / 68.4
+                                              (64, 1728, [429] * 3, False), (64, 1664, [112] * 8, False), (64, 832, [200] * 4, False),         # 32.6 / 37.2
+                                              (64, 768, [200] * 4, True), (128, 1728, [429] * 3, True), (1664, 2752, [82] * 4, True)])                                       # 67.3 / 60.4
+def test_parts_run_where_they_are_faster(H, I, counts, parts):
+    from mok_route import kinds
+
+    assert ("part" in kinds(H, I, counts)) is parts
+
+
 # rows around a wave's 64, 128 and a tile's 256, experts of few rows and of none among them; columns of one part, an odd number of
 # parts and whole column tiles; contractions from one slot to more than a ring; rows of whole cache lines (one launch) and not
 @pytest.mark.gpu
