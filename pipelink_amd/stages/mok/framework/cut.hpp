@@ -26,10 +26,10 @@ struct Cut {
 // both, and the two lines added where only both together pay.  The line lies above where down tiles alone break even between 10
 // and 19 slots because of the launches that cut both.  Below 5 slots (three of a narrow tile's four waves have little or nothing to
 // multiply) nothing is cut for that contraction: 64 x 64, 4 rows, 11.1 us whole, 12.4 cut; 256 x 128, 3 rows, 12.9 / 15.0; 520
-// layers, 320 of them of contractions up to 12 slots, take 1.4 % less on average than with a line of 4 n + 12 from one slot on.
-// From 5 to 9 slots small launches of one or two experts gain by cutting both: 512 x 256, one row, 15.9 /
-// 14.0.  More quarters of a GEMM than run at once take a second turn, whose start costs more than the finer cut gives.
-constexpr int cut_line(int slots) { return slots < 5 ? 0 : slots < 10 ? 4 * slots + 4 : 7 * slots + 40; }
+// layers, 320 of them of contractions up to 12 slots, take 1.3 % less on average than with a line of 4 n + 12 from one slot on,
+// 17 % at best and 7 % more at worst (one row of 256 x 384).  From 5 to 9 slots small launches of one or two experts gain by
+// cutting both: 512 x 256, one row, 15.9 / 14.0.  More quarters of a GEMM than run at once take a second turn, whose start costs more than the finer cut gives.
+constexpr int cut_line(int slots) { return slots < 5 ? 0 : slots < 10 ? 4 * slots + 12 : 7 * slots + 40; }
 // Where whole tiles take two turns of the chip already, quarters of down tiles that end within them fill the second one evenly:
 // 16 experts of 320 x 2432, 36 tokens, 304 + 32 tiles: 32.1 us whole, 29.3 as 304 + 128 tasks.  A third turn loses that: 576 x
 // 2880, 112 tokens, 368 + 48: 38.0 whole, 46.2 as 368 + 192.
