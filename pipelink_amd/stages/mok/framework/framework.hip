@@ -163,7 +163,9 @@ __device__ __forceinline__ void run_tiles(const void* params, const MokFramework
     MokGemmTask task = sched.decode(q, i, cursor);
     // the first tile has no mainloop in front of it to look ahead from
     pipelink_call_gemm_stage(&view, &task, &counters);
-    __syncthreads();  // waits for the staged loads, then the barrier
+    // what was staged has landed for every wave (the barrier itself waits for no global -> LDS load)
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __syncthreads();
     bool early = false;  // the prefetch of the tile at the loop's head has been issued
     mok::GemmCarry carry;
     // The tile after this one: the workgroup's second turn.  From there on tiles are handed out by the list's queue (a

@@ -87,13 +87,11 @@ int main(int argc, char** argv) {
 """
 
 
-@pytest.fixture(scope="module")
-def trace(tmp_path_factory):
+def _worker(d, hip):
     if CLANG is None:
         pytest.skip("needs clang")
-    d = tmp_path_factory.mktemp("worker")
     (d / "hip").mkdir()
-    (d / "hip" / "hip_runtime.h").write_text(HIP)
+    (d / "hip" / "hip_runtime.h").write_text(hip)
     (d / "worker.cpp").write_text(PROGRAM)
     subprocess.run([CLANG, "-std=c++17", "-O1", "-w", "-x", "c++", f"-I{d}", f"-I{STAGES}",
                     f"-I{os.path.join(ROOT, 'pipelink_amd', 'pipec', 'include')}", str(d / "worker.cpp"), "-o", str(d / "worker")], check=True)
@@ -101,6 +99,11 @@ def trace(tmp_path_factory):
     def run(*args):
         return subprocess.run([str(d / "worker"), *map(str, args)], check=True, capture_output=True, text=True).stdout.splitlines()
     return run
+
+
+@pytest.fixture(scope="module")
+def trace(tmp_path_factory):
+    return _worker(tmp_path_factory.mktemp("worker"), HIP)
 
 
 # full tiles and small ones, narrow parts of column tiles (8 rows, few tiles); one tile a workgroup and several; down tiles
@@ -124,3 +127,14 @@ def test_a_barrier_lies_between_staging_a_task_and_reading_it_and_back(trace, ro
         elif event != "wait":
             assert not ({"read", "write"} - {event}) & since, (n, events[max(0, n - 8):n + 1])
             since.add(event)
+
+
+def test_a_wave_waits_for_its_own_staged_loads_before_the_first_tile(tmp_path):
+    """What a workgroup's first task stages (no mainloop ends behind it) is waited for in the source itself: the barrier waits for
+    no global -> LDS load, whatever the compiler puts in front of it."""
+    run = _worker(tmp_path, HIP.replace("s_waitcnt(x) ((void)0)", 's_waitcnt(x) ((x) == 0x0F70 ? (void)puts("landed") : (void)0)'))
+    events = run(300, 23, 12, 24, 0)[:-1]
+    starts = [n for n, e in enumerate(events) if e == "workgroup"]
+    staged = [events.index("write", n) for n in starts]
+    assert len(staged) == 24
+    assert all(events[n + 1:n + 3] == ["landed", "barrier"] for n in staged)
