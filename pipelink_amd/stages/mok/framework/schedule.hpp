@@ -133,8 +133,10 @@ struct Schedule {
   // The down tile list q runs in the place of `item` (launches of both GEMMs): the rest of the expert in whose middle the list
   // begins comes last.  That expert's gate/up tiles are divided alike, some of them the end of the list before, which run last
   // of all gate/up tiles: its down tiles, first in this list, held workgroups for up to a tile's time.  us in the old order /
-  // this: 14 tokens of 2880 x 2880, top 4 of 32, 152.4 / 138.9; 10 142.0 / 135.8; 20 and 27 157.9 / 159.1; 1003 212.7 / 210.8;
-  // 4000 429 / 421; 8192 801 / 794.  (Launches of parts are one turn of the chip: one token 34.6 / 35.8.)
+  // this: 14 tokens of 2880 x 2880, top 4 of 32, 28 experts with rows, 153.6 / 141.0; 10 145.8 / 141.3; 20, 29 experts, 156.6 / 143.0;
+  // 2000 264.1 / 261.6; 4000 419.8 / 415.2; 8192 752 / 745.  With 31 of the 32 experts, 20 to 33 tokens, it costs 162.0 / 163.0; 130
+  // random layers 0.2 % on average.  (Launches of quarters are one turn of the chip: one token 34.6 / 35.8.  Parts are rotated:
+  // 447 random layers 0.6 % longer by it.)
   MOK_SCHED_FN int rotated(int q, int d, int item) const {
     const int first = share(q, d), end = share(q + 1, d);
     const int e = MOK_SCHED_COUNT(g.num_experts, [&](int x) { return tab.tile_begin[x] * down_cols <= first; }) - 1;  // of item `first`
@@ -145,7 +147,8 @@ struct Schedule {
   }
 
   // item i of list q -> task.  `cursor` is the expert of the item this workgroup decoded last: a workgroup's items
-  // come in growing order as long as it stays in one GEMM, so the search usually ends where it starts.
+  // come in growing order as long as it stays in one GEMM (down tiles: up to where a rotated list wraps), so the search usually
+  // ends where it starts.
   MOK_SCHED_FN MokGemmTask decode(int q, int i, int& cursor) const {
     const int gu = gate_up_items(), d = down_items();
     const int mine = share(q + 1, gu) - share(q, gu);
