@@ -100,21 +100,20 @@ constexpr int TILE_QUERIES = split ? FA_Q_TILE / 2 : FA_Q_TILE;
 __device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_host_view& view, uint32_t index) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, l32 = lane & 31;
-  const auto [tile, bh] = fa_order::tile_of((int)index, p.batch, p.q_heads, p.kv_heads, p.seq / TILE_QUERIES);
-  const int b = bh / p.q_heads, h = bh % p.q_heads, kvh = h / (p.q_heads / p.kv_heads);
+  const auto [tile, bh, group] = fa_order::tile_of(index, p.batch, p.q_heads, p.kv_heads, p.seq / TILE_QUERIES);
   const int q0 = tile * TILE_QUERIES, qw = q0 + 32 * (split ? wave & 1 : wave);  // the wave's first query
   const int key0 = split ? 32 * (wave >> 1) : 0;                                 // its first key of every block
   const uint32_t head_bytes = (uint32_t)p.seq * FA_D * 2;
   const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.k) + ((int64_t)b * p.kv_heads + kvh) * p.seq * FA_D, 0, (int)head_bytes, 0x00020000);
+      const_cast<uint16_t*>(p.k) + (int64_t)group * p.seq * FA_D, 0, (int)head_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(p.v) + ((int64_t)b * p.kv_heads + kvh) * p.seq * FA_D, 0, (int)head_bytes, 0x00020000);
+      const_cast<uint16_t*>(p.v) + (int64_t)group * p.seq * FA_D, 0, (int)head_bytes, 0x00020000);
   unsigned char* buf = pipelink_smem + pipelink_fa_kv();
 
   // this lane's query row as the B operand of S^T = K . Q^T: 16 bytes per 16-element step of d
   v8bf qf[8];
   {
-    const uint16_t* qrow = p.q + (((int64_t)b * p.q_heads + h) * p.seq + qw + l32) * FA_D;
+    const uint16_t* qrow = p.q + ((int64_t)bh * p.seq + qw + l32) * FA_D;
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) qf[kk] = __builtin_bit_cast(v8bf, *reinterpret_cast<const v4i*>(qrow + 16 * kk + 8 * half));
   }
@@ -316,6 +315,7 @@ __device__ __forceinline__ void attend(const FaCoreParams& p, const pipelink_hos
   }
   // ---- O[b][query][h][d] = O^T / row_sum, bf16 ------------------------------------------------------------
   const float inv = row_sum > 0.0f ? __builtin_amdgcn_rcpf(row_sum) : 0.0f;
+  const int b = (uint32_t)bh / (uint32_t)p.q_heads, h = bh - b * p.q_heads;
   uint16_t* orow = p.o + ((int64_t)b * p.seq + qw + l32) * ((int64_t)p.q_heads * FA_D) + (int64_t)h * FA_D;
 #pragma unroll
   for (int db = 0; db < 4; ++db)
