@@ -150,6 +150,37 @@ def test_window_mask_matches_the_oracle_on_every_head(window):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("window", [2, 33, 34, 66, 80, 97, 161, 450])
+def test_windows_a_little_past_whole_blocks_on_whole_and_half_tiles(window):
+    """Windows of 2 to 33 keys more than a multiple of 64: in a tile's blocks of keys there are waves of which no query sees a key,
+    which leave the block without reading it.  Every wave must still have handed in its part of the next one.  Bars: bf16 probabilities
+    and result."""
+    import json
+
+    from pipelink_amd.host.attention import open_session
+
+    paths = fa_build.images()
+    q, k, v = oa.inputs(1, 8, 4, 896, seed=window)
+    ref = oa.attention(q, k, v, None, window=window)
+    for image in ("window_linked", "window_half_linked"):
+        link = json.loads((paths[image].parent / "link.json").read_text())   # (as an object: run as it is, at any size)
+        sess = open_session(link, _bits(q), _bits(k), _bits(v), window=window, image=paths[image])
+        try:
+            for _ in range(2):
+                sess.write("o", np.full((1, 896, 1024), 0x7FC0, dtype=np.uint16))
+                sess.launch()
+                sess.synchronize()
+                o = _from_bits(sess.read("o"))
+                for (b, h), want in ref.items():
+                    got = o[b, :, h * 128:(h + 1) * 128]
+                    assert torch.isfinite(got).all()
+                    assert (got - want).abs().max().item() <= 1e-2 * want.abs().max().item(), (image, b, h)
+                    assert ((got - want).norm() / want.norm()).item() <= 1e-2, (image, b, h)
+        finally:
+            sess.close()
+
+
+@pytest.mark.gpu
 def test_window_mask_with_a_small_softmax_scale():
     """A caller's scale far below 1 / sqrt(128): queries whose first streamed block holds no key they may see must
     still give that block zero weight (whether a query has seen a key is decided on unscaled scores)."""
