@@ -117,3 +117,75 @@ def test_wait_counts_equal_the_loads_behind_the_slot_in_issue_order(tmp_path):
     assert res.returncode == 0, res.stdout
     assert "depth 4:" in res.stdout and "depth 2:" in res.stdout and "few rows:" in res.stdout
     assert ", 0 wrong" in res.stdout.splitlines()[0]
+
+
+FEW_LOOP = r"""
+#define MOK_COUNT_FN constexpr inline
+#include "load_counts.hpp"
+#include <cstdio>
+#include <vector>
+using namespace mok_gemm_owner::counts;
+// The loop of tiles of few rows as it is written: the first slots' loads, a wait; then a step waits for all but so many of the wave's
+// loads, issues those of the slot a ring ahead into the place it has just read (behind the last slot with an operand without
+// extent), and reads the next slot.  Scale loads go in front of an even slot's, the routed rows' of every eighth.
+int main() {
+  int bad = 0;
+  auto wrong = [&](const char* what, int n, int t) { if (bad++ < 10) printf("%s: n %d step %d\n", what, n, t); };
+  for (int n = 1; n <= 64; ++n) {
+    struct Issued { int slot; bool scale; };
+    std::vector<Issued> order;
+    std::vector<int> place(FEW_DEPTH, -1);        // what the ring's places hold
+    size_t landed = 0;                            // loads a wait has seen in: all but the youngest it lets go
+    auto issue = [&](int s, int at) {
+      if (s < n) {
+        if ((s & 7) == 0) order.push_back({s, true});
+        if ((s & 1) == 0) order.push_back({s, true});
+      }
+      for (int i = 0; i < FEW_LOADS; ++i) order.push_back({s, false});
+      place[at] = s;
+    };
+    auto wait = [&](size_t left) { if (order.size() > left && order.size() - left > landed) landed = order.size() - left; };
+    auto in_flight = [&](int slot) { for (size_t i = landed; i < order.size(); ++i) if (order[i].slot == slot) return true; return false; };
+    auto behind = [&](int slot) {                 // tile loads younger than the slot's
+      int count = 0;
+      for (size_t i = 0; i < order.size(); ++i) count = order[i].slot == slot ? 0 : count + !order[i].scale;
+      return count;
+    };
+    for (int s = 0; s < FEW_DEPTH && s < n; ++s) issue(s, s);
+    const int first = n < FEW_DEPTH ? 0 : (FEW_DEPTH - 1) * FEW_LOADS;
+    wait(first);
+    if (in_flight(0) || (first && behind(0) != first)) wrong("prologue", n, -1);
+    // places of the present and the next slot, as the loop advances them
+    int here = 0, ahead = 1;
+    for (int t = 0; t < (n & ~1); ++t) {
+      wait((FEW_DEPTH - 2) * FEW_LOADS);
+      if (t + 1 < n) {
+        if (place[here] != t || place[ahead] != t + 1) wrong("the places", n, t);
+        if (in_flight(t + 1)) wrong("a slot that has not landed", n, t);
+        if (n >= FEW_DEPTH && behind(t + 1) != (FEW_DEPTH - 2) * FEW_LOADS) wrong("waits for more than the slot", n, t);
+      }
+      issue(t + FEW_DEPTH, here);
+      here = ahead;
+      ahead = ahead + 1 == FEW_DEPTH ? 0 : ahead + 1;
+    }
+  }
+  printf("few rows, as written: %d wrong\n", bad);
+  return bad != 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_the_constant_waits_of_the_few_rows_loop(tmp_path):
+    (tmp_path / "few.cpp").write_text(FEW_LOOP)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", f"-I{GEMM}", str(tmp_path / "few.cpp"), "-o", str(tmp_path / "few")], check=True)
+    res = subprocess.run([str(tmp_path / "few")], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
+    # the harness restates these; the kernel's are the ones that count
+    with open(os.path.join(GEMM, "gemm.hip")) as f:
+        loop = f.read()
+    loop = loop[loop.index("void mainloop_few_rows"):]
+    loop = loop[:loop.index("\n}\n")]
+    for line in ("if (n < FEW_DEPTH) wait_loads_and_reads<0>();", "else wait_loads_and_reads<(FEW_DEPTH - 1) * FEW_LOADS>();",
+                 "wait_loads_and_reads<(FEW_DEPTH - 2) * FEW_LOADS>();", "int s = FEW_DEPTH;", "for (; j + 1 < n; j += 2) {"):
+        assert loop.count(line) == 1
