@@ -52,3 +52,22 @@ def test_no_barrier_is_reached_with_a_load_into_lds_in_flight(image):
     text = text[text.index("<pipelink_kernel>:"):]
     assert len(re.findall(r"buffer_load_dwordx4[^\n]* lds", text)) >= 16
     assert _unwaited_barriers(text) == []
+
+
+@pytest.mark.parametrize("image", ["linked", "window_linked", "half_linked", "window_half_linked", "one_unit"])
+def test_reads_of_v_wait_for_no_load(image):
+    """The next block's keys and values fly while this one's are read: the compiler puts no wait for them in front of the transposing
+    reads (it does where it knows nothing of what these may alias)."""
+    text = subprocess.run([str(LLVM_BIN / "llvm-objdump"), "-d", str(fa_build.images()[image])], capture_output=True, text=True, check=True).stdout
+    reads, flying, waited = 0, False, False   # loads into LDS issued behind the last barrier; a wait for loads behind those
+    for line in text[text.index("<pipelink_kernel>:"):].splitlines():
+        if re.match(r"\s+s_barrier", line):
+            flying = waited = False
+        elif re.match(r"\s+buffer_load_dwordx4.* lds", line):
+            flying, waited = True, False
+        elif re.match(r"\s+s_waitcnt.*vmcnt", line):
+            waited = True
+        elif re.match(r"\s+ds_read_b64_tr_b16", line):
+            reads += 1
+            assert not (flying and waited), line
+    assert reads >= 32
