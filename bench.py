@@ -60,7 +60,7 @@ def executed_flops(counts):
     share over the whole contraction unless the share starts past the expert's last row or past the last output
     column (then it only loads); shares that are partly past the end are multiplied in full.  A tile of at most 64
     rows or at most 64 columns (per matrix) is in the small placement: four waves x 64 rows x the 32-row weight
-    fragments they hold (few rows: 2 per wave; few columns: 2 per wave and matrix)."""
+    fragments they hold (few rows: 2 per wave, and of at most 32 rows one fragment of those; few columns: 2 per wave and matrix)."""
     total = 0.0
     for c in counts:
         for first in range(0, int(c), TILE):
@@ -68,8 +68,8 @@ def executed_flops(counts):
             row_waves = 1 if rows <= TILE // 2 else 2
             for cols, k, step, matrices in ((I, H, TILE // 2, 2), (H, I, TILE, 1)):  # gate/up (two matrices), down
                 for col_begin in range(0, cols, step):
-                    if rows <= 64:      # few rows: every wave 64 rows x 2 fragments of 32 weight rows
-                        total += 4 * 64 * 64 * 2.0 * k
+                    if rows <= 64:      # few rows: every wave 64 (or 32) rows x 2 fragments of 32 weight rows
+                        total += 4 * (32 if rows <= 32 else 64) * 64 * 2.0 * k
                     elif cols - col_begin <= 64:  # few columns: every wave 64 rows x 64 columns of each matrix
                         total += 4 * 64 * 64 * matrices * 2.0 * k
                     else:
