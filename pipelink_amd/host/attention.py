@@ -22,13 +22,21 @@ def _half_tiles_pay(heads: int, s: int, window: int | None) -> bool:
     of 128.  Half tiles shorten a tile's chain of key blocks, which is all a launch takes while compute units are left over;
     they cost a start and a merge per workgroup, which short chains do not earn back, and loads twice once every compute unit
     has two workgroups.  us half / us whole over 3700 random shapes (1 to 384 tiles, S 128 to 4096, causal and windows of 20
-    keys up; a launch against itself: 0.95 .. 1.05), by the longest chain L of a whole tile in blocks, the average A and the load F = tiles * A / (256 L):
+    keys up; a launch against itself: 0.95 .. 1.05), by the longest chain L of a whole tile in blocks, the average A and the load F = tiles * A / (256 L),
+    with whole and half tiles that waited for the next block's loads in front of their V reads:
       up to 128 tiles    0.69 .. 0.98 whatever the chains
       129 to 256 tiles   L 2: 1.2, L 4: 0.97 to 1.04, L 6: 0.97 (up to 1.16), L 8: 0.93 (up to 1.08); from L 10 on and F up to 0.78:
                          0.79 .. 0.98, two shapes of 460 above 1 (1.01 and 1.03, L 10); beyond: up to 1.11
       257 to 384 tiles   from L 12 on and F up to 0.78: 0.81 .. 0.98; beyond: up to 1.26; L 10: 0.9 to 1.13, L 7 and
                          less: 1.03 to 1.37
-      512 tiles          1.07 (S 2048), 1.16 (S 512)"""
+      512 tiles          1.07 (S 2048), 1.16 (S 512)
+    Without that wait half tiles are the shorter ones a little further; 260 shapes of 1 to 512 tiles:
+      up to 128 tiles    0.67 .. 0.98
+      129 to 256 tiles   L 3 and less: 0.92 to 1.13, L 4 and 5: 0.91 to 1.07, L 6 to 9: 0.76 to 0.92; from L 10 on 0.70 .. 0.87
+      257 to 384 tiles   from L 12 on 0.76 .. 0.92, L 8 to 11: 0.93 to 1.16, less 1.06 to 1.24
+      385 to 512 tiles   from L 20 on 0.79 .. 0.99, L 12 to 19: 0.98 to 1.06, less 1.11 to 1.20
+    The line is the first table's still: 1.6 % above the better of the two on average, 1.32 at worst (1920 keys, a window of 443,
+    135 tiles)."""
     tiles = heads * (s // Q_TILE)
     if tiles <= COMPUTE_UNITS // 2 or tiles > HALF_TILES_UP_TO:
         return tiles <= COMPUTE_UNITS // 2

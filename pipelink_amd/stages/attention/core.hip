@@ -19,9 +19,9 @@
 // A tile is a chain of key blocks; a grid that leaves most SIMDs with one wave or none takes as long as the longest chain,
 // with nothing beside it.  With half tiles waves 0 and 1 have 32 queries each and the first 32 keys of every block, waves 2
 // and 3 the same queries and the other 32 keys: twice the workgroups, each block half as long for a wave.  The two halves
-// of a query's sum meet through LDS at the end.  us, whole / half tiles: B 1, 32 heads, S 1152, window 700 (288 tiles) 26.3 /
-// 21.2; S 512 causal (128 tiles) 14.6 / 11.8; 8 heads, S 4096 (256 tiles) 81.8 / 62.4; 32 heads, S 2048 (512 tiles) 57.6 /
-// 61.4; the stated B 4, S 4096 (4096 tiles) 583 / 695: with two waves on every SIMD a key block costs its loads twice.
+// of a query's sum meet through LDS at the end.  us, whole / half tiles: B 1, 32 heads, S 1152, window 700 (288 tiles) 25.9 /
+// 20.6; S 512 causal (128 tiles) 14.5 / 11.8; 8 heads, S 4096 (256 tiles) 82.1 / 60.9; 32 heads, S 2048 (512 tiles) 54.1 /
+// 51.8, S 512 of 128 heads (512 tiles) 19.9 / 24.5; B 4, S 4096 (4096 tiles) 550 / 655: with two waves on every SIMD a key block costs its loads twice.
 //
 // Two LDS buffers per operand: block i + 1 is in flight while block i is multiplied; one barrier per block.
 #include <pipelink/stage.hpp>

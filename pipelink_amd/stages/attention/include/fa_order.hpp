@@ -15,10 +15,10 @@ struct Tile {
 // Causal tiles cost in proportion to their position: the latest (longest) tiles of every head come first, so that the grid does
 // not end on a few long ones.  Workgroups are dealt to the XCDs in turn, each with an L2 of its own: the query heads that share a
 // KV head are kept on one XCD (on 8 / sets of them where the KV heads of the batch are no multiple of 8), where its L2 reads their
-// keys and values once.  Dealt head by head, a group of four heads was on four XCDs.  us before / after: B 4, 32 / 8 heads, S 4096
-// 546 / 541, with a window of 1024 321 / 289; S 1024 49.1 / 46.2; S 512 18.8 / 17.6; B 3, 32 / 4 heads, S 2048 111 / 108; B 4, 16 / 16
-// heads, S 2048, where no heads share, 78.0 / 77.9.  (Group after group, so that an XCD streams one at a time, loses the order of
-// lengths: the last 78 / 104, B 3, 8 / 2 heads, S 4096 103 / 131.)
+// keys and values once.  Dealt head by head, a group of four heads was on four XCDs.  us head by head / this: B 4, 32 / 8 heads, S
+// 4096 574 / 550, with a window of 1024 320 / 299; S 1024 58.4 / 54.9; S 512 20.5 / 19.9; B 3, 32 / 4 heads, S 2048 130 / 124; B 4, 16 /
+// 16 heads, S 2048, where no heads share and the orders are the same, 91 / 92.  (Group after group, so that an XCD streams one at a
+// time, loses the order of lengths: the last 78 / 104, B 3, 8 / 2 heads, S 4096 103 / 131.)
 // (The sets are a power of two, and one set is the order head by head: three divisions and shifts.  With a division by each
 // of the set counts the smallest launches took 0.2 us more, S 128 of 32 / 8 heads 6.6 / 6.8.)
 FA_ORDER_FN Tile tile_of(unsigned index, unsigned batch, unsigned q_heads, unsigned kv_heads, unsigned q_tiles) {

@@ -58,8 +58,8 @@ static_assert(TILE_X == mok::TILE_X && TILE_W == mok::TILE_W, "the schedule's ti
 
 // Asks a queue for its next number, without waiting for the answer.  (An addition of one lane is made one of a wave by the
 // compiler, which has the answer spread over the lanes at once: 1 to 2 us in front of the next tile's first loads.  A wrapping
-// increment it leaves alone.)  us with the addition / this, and the two accesses of LDS that waited for everything: one token of
-// 2880 x 2880, top 4 of 32, 36.3 / 34.8; 27 160.1 / 158.2; 128 167.0 / 164.7; 448 x 704, 60 tokens 19.7 / 18.9.  Full tiles keep
+// increment it leaves alone.)  us with the addition / this, and the two accesses of LDS that waited for everything, back to back on
+// one state: one token of 2880 x 2880, top 4 of 32, 36.3 / 34.8; 27 160.1 / 158.2; 128 167.0 / 164.7; 448 x 704, 60 tokens 19.7 / 18.9.  Full tiles keep
 // the addition: there the increment's register is the one that makes the next mainloop wait (2000 tokens 277.0 / 279.5).
 __device__ __forceinline__ uint32_t take_one(uint32_t* queue) {
 #ifdef __HIP_DEVICE_COMPILE__

@@ -1055,7 +1055,7 @@ __device__ __forceinline__ void mainloop_small(const MokGemmResidue& g, const Mo
 // A step has 256 clocks of MFMAs; what bounds it while the memory is not busy is the other instructions one wave issues, about
 // five clocks each.  With the ring position a product, the waits a switch on a computed count and every fragment's address its
 // own (110 instructions and eight branches a step) a step took 0.41 us, whatever its loads were of; with 50 instructions and no
-// branch 0.22.  us before / after: one token of 2880 x 2880, top 4 of 32, 41.7 / 36.3; two 54.0 / 43.0; three 60.3 / 54.0; 128,
+// branch 0.22.  us before / after, back to back on one state: one token of 2880 x 2880, top 4 of 32, 41.7 / 36.3; two 54.0 / 43.0; three 60.3 / 54.0; 128,
 // where all compute units stream at once, 169.0 / 166.8.
 template <int B>  // routed-row fragments
 __device__ __forceinline__ void mainloop_few_rows(const MokGemmResidue& g, const MokGemmTask& t, AccFrag& acc, const GemmCarry& carry,
@@ -1514,8 +1514,8 @@ extern "C" __device__ void mok_gemm_fwd_small(const void* view, const MokGemmTas
         break;
       }
       if (placement == mok::TILE_SMALL_ROWS) {  // (the deep ring needs the arena of depth 4; mok_gemm_prefetch decides alike)
-        // (32 rows, one fragment of them: half the MFMAs and three quarters of the LDS reads.  us with two fragments / this: one
-        // token of 2880 x 2880, top 4 of 32, 34.7 / 32.5; two 42.3 / 39.8; 128 164.8 / 164.1; 448 x 704, 60 tokens 18.9 / 18.6)
+        // (32 rows, one fragment of them: half the MFMAs and three quarters of the LDS reads.  us with two fragments / this, back
+        // to back on one state: one token of 2880 x 2880, top 4 of 32, 34.7 / 32.5; two 42.3 / 39.8; 128 164.8 / 164.1; 448 x 704, 60 tokens 18.9 / 18.6)
         if (task->row_end - task->row_begin <= 32) mok_gemm_owner::mainloop_few_rows<1>(g, *task, *acc, *carry, upcoming, *counters);
         else mok_gemm_owner::mainloop_few_rows<2>(g, *task, *acc, *carry, upcoming, *counters);
         break;
