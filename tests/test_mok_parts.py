@@ -82,8 +82,13 @@ def test_parts_run_where_they_are_faster(H, I, counts, parts):
 # parts and whole column tiles; contractions from one slot to more than a ring; rows of whole cache lines (one launch) and not
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,I,counts", [(64, 64, [65]), (128, 192, [127, 0, 129]), (448, 704, [128, 64, 200, 65]), (320, 128, [256, 257, 1]),
-                                        (256, 640, [511, 3]), (576, 320, [300, 33, 0, 70, 191]), (1088, 448, [100, 90])])
+                                        (256, 640, [511, 3]), (576, 320, [300, 33, 0, 70, 191]), (1088, 448, [100, 90]),
+                                        # contractions of 26, 36, 43 and 45 slots, and next to where parts end
+                                        (1664, 2752, [82] * 4), (2304, 448, [130, 0, 90, 70]), (192, 2880, [257, 66]), (2880, 192, [300, 1]), (64, 768, [200] * 4)])
 def test_forward_in_parts_matches_the_oracle_and_whole_tiles(H, I, counts):
+    from mok_route import kinds
+
+    assert kinds(H, I, counts) == {"part"} and "part" not in kinds(H, I, counts, parts=False)
     from oracle import moe_ffn
     from pipelink_amd.host import mok_inputs
     from pipelink_amd.host.mok import MoKSession, code_pitch
